@@ -21,12 +21,15 @@
 //    reduce_partials sums in a fixed order (deterministic).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 typedef __bf16 bf16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 namespace {
 
@@ -163,6 +166,296 @@ __global__ void __launch_bounds__(256) k_no_conv_fwd(NoConvArgs a) {
       if (a.y32) a.y32[o] = v;
       if (a.y) a.y[o] = (bf16)v;
     }
+  }
+}
+
+// ---------------------------------------------------------------- 3x3x3 conv
+// conv_fwd for 27 taps: the same sums in the same order as k_no_conv_fwd
+// (taps outer, channels inner, so the results are the same bits), with the
+// operands' traffic cut to what the LDS can deliver beside the matrix cores.
+//
+// A wave owns 32 R consecutive voxels and all Cout channels. The three taps
+// of one (dz, dy) read the same run of voxel rows, shifted by the dilation:
+// the wave copies that run (32 R + 2 dil rows) into LDS of its own once and
+// reads it three times, so x is fetched 9 times instead of 27, and no
+// barrier is needed for it; the next run travels to registers while this
+// one is computed. A voxel whose neighbour lies outside the grid reads a row
+// of zeros instead. The weights of a tap are staged for the whole workgroup,
+// one tap ahead, with one barrier per tap in its middle: with three buffers
+// no wave waits for another at a tap's edge (where only two fit, a second
+// barrier guards the buffer that is written). The operands of each step are
+// read from LDS during the step before, also across taps.
+//
+// Workgroups are persistent (as many as the chip holds) and flow from one
+// tile of voxels into the next: its first run and weights are fetched during
+// the last taps of the tile before, and the output stores drain beside its
+// first ones. XCD w mod 8 takes a contiguous eighth of the tiles, so that
+// the neighbouring rows which its workgroups share sit in one L2.
+constexpr int kConvMaxDil = 8;  // the staged runs are sized for dilations up to this
+constexpr int kConvLds = 160 * 1024;
+constexpr int kCus = 256;
+
+template <int KS, int NT, int R>
+struct ConvShape {
+  static constexpr int kCin = KS * 16, kCout = NT * 32;
+  static constexpr int kLd = kCin + 8;      // LDS row length: 16 bytes of padding spread the rows over the banks
+  static constexpr int kPieces = KS * 2;    // 16-byte pieces per row
+  static constexpr int kRun = ((32 * R + 2 * kConvMaxDil) * kPieces + 63) / 64;  // pieces per lane of a staged run
+  static constexpr int kRows = (kRun * 64 + kPieces - 1) / kPieces;             // LDS rows of a wave's run
+  static constexpr int kW = (kCout * kPieces + 255) / 256;                       // weight pieces per thread
+  static constexpr int kBufs = (kWaves * kRows + 3 * kCout + 1) * kLd * 2 <= kConvLds ? 3 : 2;
+  static constexpr int kLds = (kWaves * kRows + kBufs * kCout + 1) * kLd * 2;    // bytes
+};
+
+// Exchanges the upper half-wave of a with the lower half-wave of b.
+__device__ __forceinline__ void half_swap(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  bf16x2 p;
+  p[0] = (bf16)lo;
+  p[1] = (bf16)hi;
+  return __builtin_bit_cast(uint32_t, p);
+}
+
+template <int KS, int NT, int R>
+__global__ void __launch_bounds__(256, 1) k_no_conv27(NoConvArgs a, int tiles) {
+  using S = ConvShape<KS, NT, R>;
+  constexpr int Ld = S::kLd, kBufs = S::kBufs;
+  __shared__ __align__(16) bf16 lds[S::kLds / 2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 31, kg = lane >> 5;
+  bf16* const sx = lds + wave * S::kRows * Ld;
+  bf16* const sw = lds + kWaves * S::kRows * Ld;
+  bf16* const zero = sw + kBufs * S::kCout * Ld;
+  const int V = a.Z * a.Y * a.X;
+  const int M = a.B * V;
+  const uint32_t bytes = (uint32_t)M * (S::kCin * 2);
+  // this workgroup's tiles: tile0, tile0 + step, ... below tile_end
+  int tile0 = blockIdx.x, step = gridDim.x, tile_end = tiles;
+  if (gridDim.x % 8u == 0u) {
+    const int q = blockIdx.x % 8u;
+    tile0 = (int)((long)tiles * q / 8) + blockIdx.x / 8u;
+    tile_end = (int)((long)tiles * (q + 1) / 8);
+    step = gridDim.x / 8u;
+  }
+  if (tile0 >= tile_end) return;
+  if (threadIdx.x < Ld / 8) {
+    bf16x8 z;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z[e] = (bf16)0.0f;
+    *reinterpret_cast<bf16x8*>(zero + threadIdx.x * 8) = z;
+  }
+  // coordinates of the lane's voxel in each of the wave's R voxel tiles
+  int vx[R], vy[R], vz[R];
+  auto locate = [&](int m0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int m = m0 + r * 32 + col;
+      int q = m % V;
+      vz[r] = m < M ? q / (a.Y * a.X) : -(1 << 20);  // past the end: every neighbour is outside
+      q %= a.Y * a.X;
+      vy[r] = q / a.X;
+      vx[r] = q % a.X;
+    }
+  };
+  bf16x8 px[S::kRun], pw[S::kW];
+  const char* const xb = reinterpret_cast<const char*>(a.x);
+  // the run of (dz, dy): rows m0 + (dz Y + dy) X - dil onwards, contiguous in
+  // memory; pieces outside the tensor are read from its start and never used
+  auto fetch_x = [&](int m0, int g, int i0, int i1) {
+    const int off = ((g / 3 - 1) * a.Y + (g % 3 - 1)) * a.dil * a.X - a.dil;
+    const int start = (m0 + off) * (S::kCin * 2) + lane * 16;
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      const uint32_t o = (uint32_t)(start + i * 1024);
+      px[i] = *reinterpret_cast<const bf16x8*>(xb + (o < bytes ? o : 0u));
+    }
+  };
+  auto store_x = [&]() {
+#pragma unroll
+    for (int i = 0; i < S::kRun; ++i) {
+      const int q = i * 64 + lane;
+      *reinterpret_cast<bf16x8*>(sx + (q / S::kPieces) * Ld + (q % S::kPieces) * 8) = px[i];
+    }
+  };
+  // piece i of this thread; past the last one threads repeat earlier pieces
+  auto w_piece = [&](int i) {
+    constexpr int n = S::kCout * S::kPieces;
+    const int q = i * 256 + threadIdx.x;
+    return n < 256 ? q % n : (q < n ? q : q - 256);
+  };
+  auto fetch_w = [&](int t) {
+    const bf16* src = a.w + (long)t * (S::kCout * S::kCin);
+#pragma unroll
+    for (int i = 0; i < S::kW; ++i) pw[i] = *reinterpret_cast<const bf16x8*>(src + w_piece(i) * 8);
+  };
+  auto store_w = [&](int buf) {
+    bf16* dst = sw + buf * S::kCout * Ld;
+#pragma unroll
+    for (int i = 0; i < S::kW; ++i) {
+      const int q = w_piece(i);
+      *reinterpret_cast<bf16x8*>(dst + (q / S::kPieces) * Ld + (q % S::kPieces) * 8) = pw[i];
+    }
+  };
+  bf16x8 xf[2][R], wf[2][NT];  // operands of this step and the next
+  const bf16* xr[R];
+  auto aim = [&](int g, int s) {  // the lane's voxels at tap (g, s): their rows in the run, or the zeros
+    const int dz = (g / 3 - 1) * a.dil, dy = (g % 3 - 1) * a.dil;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int zz = vz[r] + dz, yy = vy[r] + dy, xx = vx[r] + (s - 1) * a.dil;
+      const bool in = (unsigned)zz < (unsigned)a.Z && (unsigned)yy < (unsigned)a.Y && (unsigned)xx < (unsigned)a.X;
+      xr[r] = (in ? sx + (r * 32 + col + s * a.dil) * Ld : zero) + kg * 8;
+    }
+  };
+  auto load_step = [&](int k, int buf) {
+    const bf16* wr = sw + buf * S::kCout * Ld + col * Ld + kg * 8;
+#pragma unroll
+    for (int r = 0; r < R; ++r) xf[k & 1][r] = *reinterpret_cast<const bf16x8*>(xr[r] + k * 16);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wf[k & 1][j] = *reinterpret_cast<const bf16x8*>(wr + j * 32 * Ld + k * 16);
+  };
+  f32x16 acc[R][NT];
+  int m0 = (tile0 * kWaves + wave) * (32 * R);
+  fetch_x(m0, 0, 0, S::kRun);
+  fetch_w(0);
+  store_x();
+  store_w(0);
+  fetch_w(1);
+  __syncthreads();
+  locate(m0);
+  aim(0, 0);
+  load_step(0, 0);
+  int wbuf = 0;  // two buffers: the one that holds this tap's weights
+  for (int tile = tile0; tile < tile_end; tile += step) {  // uniform over the workgroup
+    const int m_next = tile + step < tile_end ? m0 + step * (kWaves * 32 * R) : m0;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[r][j][i] = 0.0f;
+    for (int g = 0; g < 9; ++g) {
+      const int gn = g < 8 ? g + 1 : 0, mn = g < 8 ? m0 : m_next;
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        const int t = 3 * g + s;
+        const int cur = kBufs == 3 ? s : wbuf, nxt = kBufs == 3 ? (s + 1) % 3 : wbuf ^ 1;
+        // weights of tap t + 1. Three buffers: theirs was last read in tap
+        // t - 2, and every wave is past that one since tap t - 1's barrier
+        if (kBufs == 2) __syncthreads();
+        store_w(nxt);
+        fetch_w(t < 25 ? t + 2 : t - 25);
+        fetch_x(mn, gn, s * S::kRun / 3, (s + 1) * S::kRun / 3);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+          if (k + 1 < KS) {
+            load_step(k + 1, cur);
+          } else {
+            // the next tap's first operands; after the third tap the next run
+            // takes this one's place (LDS operations of a wave stay in order:
+            // only the compiler needs telling that other lanes read it)
+            if (s == 2) {
+              asm volatile("" ::: "memory");
+              store_x();
+              asm volatile("" ::: "memory");
+              if (g == 8) locate(m_next);
+            }
+            aim(s < 2 ? g : gn, (s + 1) % 3);
+            load_step(0, nxt);
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+              acc[r][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k & 1][j], xf[k & 1][r], acc[r][j], 0, 0, 0);
+          // one LDS read between two matrix instructions
+#pragma unroll
+          for (int i = 0; i < R * NT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if (k == KS / 2 - 1) __syncthreads();
+        }
+        wbuf ^= 1;
+      }
+    }
+    // Epilogue. A lane holds voxel col of each tile and, per group q of four
+    // values, channels j * 32 + 8 q + 4 kg + (0..3); the half-waves exchange
+    // groups so that a lane moves eight consecutive channels (16 bytes):
+    // those of group 2 p for kg = 0, of group 2 p + 1 for kg = 1.
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int m = m0 + r * 32 + col;
+      const long row = (long)(m < M ? m : 0) * S::kCout + 8 * kg;
+      uint4 res[NT][2];
+      if (a.res) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            res[j][p] = *reinterpret_cast<const uint4*>(a.res + row + j * 32 + 16 * p);
+      }
+      if (a.bias)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[r][j][i] += a.bias[j * 32 + 8 * (i / 4) + 4 * kg + i % 4];
+      if (a.relu)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[r][j][i] = acc[r][j][i] > 0.0f ? acc[r][j][i] : 0.0f;
+      auto store_bf16 = [&](bf16* dst) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const f32x16& v = acc[r][j];
+            uint4 o = make_uint4(pack_bf16(v[8 * p], v[8 * p + 1]), pack_bf16(v[8 * p + 2], v[8 * p + 3]),
+                                 pack_bf16(v[8 * p + 4], v[8 * p + 5]), pack_bf16(v[8 * p + 6], v[8 * p + 7]));
+            half_swap(o.x, o.z);
+            half_swap(o.y, o.w);
+            if (m < M) *reinterpret_cast<uint4*>(dst + row + j * 32 + 16 * p) = o;
+          }
+      };
+      if (a.h) store_bf16(a.h);
+      if (a.res) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            uint4 o = res[j][p];
+            half_swap(o.x, o.z);
+            half_swap(o.y, o.w);
+            const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              acc[r][j][8 * p + 2 * e] += __uint_as_float(w[e] << 16);
+              acc[r][j][8 * p + 2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
+            }
+          }
+      }
+      if (a.y32 && m < M) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[r][j][4 * q + e];
+            *reinterpret_cast<f32x4*>(a.y32 + (long)m * S::kCout + j * 32 + 8 * q + 4 * kg) = v;
+          }
+      }
+      if (a.y) store_bf16(a.y);
+    }
+    m0 = m_next;
   }
 }
 
@@ -440,6 +733,59 @@ static inline unsigned nb(long n, int t) { return (unsigned)((n + t - 1) / t); }
 #define NO_EMPTY(n) \
   if ((n) <= 0) return 0
 
+namespace {
+
+template <int KS, int NT, int R>
+bool conv27_launch(const NoConvArgs& a, long M, hipStream_t st) {
+  // persistent workgroups: one resident set
+  static const int per_cu = [] {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_no_conv27<KS, NT, R>, 256, 0);
+    return e == hipSuccess && n > 0 ? n : 1;
+  }();
+  const unsigned tiles = nb(M, 32 * R * kWaves);
+  const unsigned grid = std::min(tiles, (unsigned)(kCus * per_cu));
+  hipLaunchKernelGGL((k_no_conv27<KS, NT, R>), dim3(grid), dim3(256), 0, st, a, (int)tiles);
+  return true;
+}
+
+template <int KS, int NT>
+bool conv27_r(const NoConvArgs& a, long M, hipStream_t st) {
+  // Two voxel tiles per wave; one where that leaves half the CUs without a
+  // workgroup (M <= 32768: 1008 voxels of 128 -> 128 channels 35 us against
+  // 56). Three or four per wave need fewer LDS reads per matrix instruction,
+  // but their registers cost more than that gains (96 -> 96 channels, 524288
+  // voxels: 304 us with two, 326 with three, 505 with four, which spills).
+  if (M <= kCus / 2 * 64 * kWaves) return conv27_launch<KS, NT, 1>(a, M, st);
+  return conv27_launch<KS, NT, 2>(a, M, st);
+}
+
+template <int KS>
+bool conv27_n(const NoConvArgs& a, long M, hipStream_t st) {
+  switch (a.Cout / 32) {
+    case 1: return conv27_r<KS, 1>(a, M, st);
+    case 2: return conv27_r<KS, 2>(a, M, st);
+    case 3: return conv27_r<KS, 3>(a, M, st);
+    default: return conv27_r<KS, 4>(a, M, st);
+  }
+}
+
+// The staged kernel for the shapes that it covers; false: not covered.
+bool conv27(const NoConvArgs& a, long M, hipStream_t st) {
+  // byte offsets into x, from a run's start before the first voxel to past the last workgroup's voxels, fit an int
+  const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
+  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * a.Cin * 2 >= (1L << 31)) return false;
+  switch (a.Cin) {
+    case 32: return conv27_n<2>(a, M, st);
+    case 64: return conv27_n<4>(a, M, st);
+    case 96: return conv27_n<6>(a, M, st);
+    case 128: return conv27_n<8>(a, M, st);
+    default: return false;
+  }
+}
+
+}  // namespace
+
 extern "C" {
 
 int dsmc_no_conv_fwd(const void* x, const void* w, const float* bias, const void* res, void* y, float* y32,
@@ -451,6 +797,7 @@ int dsmc_no_conv_fwd(const void* x, const void* w, const float* bias, const void
                B, Z, Y, X, Cin, Cout, taps, dil, relu};
   long M = (long)B * Z * Y * X;
   NO_EMPTY(M);
+  if (conv27(a, M, (hipStream_t)stream)) return hipGetLastError() == hipSuccess ? 0 : -3;
   const size_t lds = 2ull * Cout * (Cin + 8) * sizeof(bf16);  // two taps of weights
   hipLaunchKernelGGL(k_no_conv_fwd, dim3(nb(M, 32 * kWaves)), dim3(256), lds, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
