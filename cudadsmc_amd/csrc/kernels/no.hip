@@ -581,12 +581,234 @@ __global__ void __launch_bounds__(256) k_no_conv_bwd_w(NoBwdWArgs a) {
   }
 }
 
-// out[i] (+)= sum over chunks of part[c][i], fixed order.
-__global__ void k_no_reduce_partials(const float* part, long n, int chunks, float* out, int accumulate) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// ------------------------------------------------- 3x3x3 weight gradient
+// conv_bwd_w for 27 taps: dw[t] = dy^T x(shifted by tap t), K = voxels, so
+// both operands need the voxel index innermost while memory has the channel
+// innermost. Rows are staged in LDS as they come (16-byte copies) and read
+// with the transposing LDS load: of 16 lanes, lane 4 r + q names the four
+// channels 4 q of row r, and lane c receives channel c of rows 0..3.
+//
+// A workgroup takes four consecutive taps, one per wave, and a range of
+// voxels: a wave keeps its tap's whole Cout x Cin product in registers, so
+// dy is read once per voxel for the four taps, and the runs of x rows of the
+// (at most two) (dz, dy) that they belong to serve the taps that share them.
+// A row whose neighbour lies outside the grid is read as zeros: per block of
+// voxels each wave makes a bit mask of its tap's inside voxels. Blocks flow
+// through three LDS buffers: while one is multiplied, the next is stored and
+// the one after that is on its way to registers, with one barrier per block.
+//
+// LDS traffic bounds it: (TM + TN) KB read per TM TN MFMAs of 32 cycles and
+// wave (85 B per cycle and CU for 96 x 96 channels) and about 36 B written.
+// With blocks of 32 voxels two workgroups share a CU and cover each other's
+// waits; with 64 there is one. The sums and their order are those of
+// k_no_conv_bwd_w (16 voxels per MFMA, in order within a chunk), so the
+// results are the same bits. 96 x 96 channels, 524288 voxels: 1212 -> 310 us
+// (750 TFLOP/s with the reduction); longer chunks that filled the chip evenly
+// were 5% faster, but lengthen the chains of additions.
+template <int TM, int TN, bool PAIR>
+struct BwdShape {
+  static constexpr int kCo = TM * 32, kCi = TN * 32;
+  // row lengths that put four consecutive rows' 64-byte pieces in different banks (16 or 48 words modulo 64)
+  static constexpr int ld(int c) { return c == 64 ? 96 : c == 128 ? 160 : c; }
+  static constexpr int kLdY = ld(kCo), kLdX = ld(kCi);
+  static constexpr int buf(int kb) { return kb * kLdY + 2 * (kb + 2 * kConvMaxDil) * kLdX; }
+  static constexpr bool kPairs = TM * TN <= 9;  // registers for two waves per SIMD
+  static constexpr int kB = !PAIR && (3 * buf(64) + kLdX) * 2 <= kConvLds ? 64 : 32;  // voxels per block
+  static constexpr int kRunX = kB + 2 * kConvMaxDil;                          // rows of a run of x
+  static constexpr int kBuf = buf(kB);
+  static constexpr int kPY = kCo / 8, kPX = kCi / 8;                          // 16-byte pieces per row
+  static constexpr int kNY = (kB * kPY + 255) / 256, kNX = (2 * kRunX * kPX + 255) / 256;  // pieces per thread
+  static constexpr int kLds = (3 * kBuf + kLdX) * 2;
+};
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) bf16 lds_bf16;
+
+// rows r..r+3 of the lane's 16-lane group, transposed (see above)
+__device__ __forceinline__ s16x4 lds_tr(const lds_bf16* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+}
+
+template <int TM, int TN, bool PAIR>
+__global__ void __launch_bounds__(256, PAIR ? 2 : 1) k_no_conv27_bwd_w(NoBwdWArgs a) {
+  using S = BwdShape<TM, TN, PAIR>;
+  constexpr int kB = S::kB;
+  __shared__ __align__(16) bf16 lds[S::kLds / 2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = lane >> 5;
+  const int M = a.B * a.Z * a.Y * a.X;
+  // XCD b mod 8 takes a contiguous share of the (chunk, tap group) list, tap
+  // groups fastest: the groups of a chunk share its rows in one L2
+  const unsigned T = gridDim.x, q8 = blockIdx.x % 8u;
+  const unsigned item = q8 * (T / 8u) + min(q8, T % 8u) + blockIdx.x / 8u;
+  const int chunk = item / 7u, t0 = (item % 7u) * 4;
+  const int t = t0 + wave;  // this wave's tap (27: none, the wave only stages)
+  const int b0 = chunk * (a.chunk / kB), b1 = min(b0 + a.chunk / kB, (M + kB - 1) / kB);  // the chunk's blocks
+  lds_bf16* const base = (lds_bf16*)lds;
+  lds_bf16* const zero = base + 3 * S::kBuf;
+  if (threadIdx.x < S::kLdX) lds[3 * S::kBuf + threadIdx.x] = (bf16)0.0f;
+
+  // staging: pieces of dy and of the two runs of x, at fixed places per thread
+  const int gA = t0 / 3, gB = min((t0 + 3) / 3, 8);
+  const int offA = ((gA / 3 - 1) * a.Y + (gA % 3 - 1)) * a.dil * a.X - a.dil;
+  const int offB = ((gB / 3 - 1) * a.Y + (gB % 3 - 1)) * a.dil * a.X - a.dil;
+  const uint32_t ybytes = (uint32_t)M * (S::kCo * 2), xbytes = (uint32_t)M * (S::kCi * 2);
+  const char* const yb = reinterpret_cast<const char*>(a.dy);
+  const char* const xb = reinterpret_cast<const char*>(a.x);
+  bf16x8 py[S::kNY], px[S::kNX];
+  auto piece = [&](int i, int n) {  // piece i of this thread; past the last one threads repeat earlier pieces
+    const int q = i * 256 + threadIdx.x;
+    return n < 256 ? q % n : (q < n ? q : q - 256);
+  };
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < S::kNY; ++i) {
+      const uint32_t o = (uint32_t)(b * kB) * (S::kCo * 2) + piece(i, kB * S::kPY) * 16;
+      py[i] = *reinterpret_cast<const bf16x8*>(yb + (o < ybytes ? o : 0u));
+    }
+#pragma unroll
+    for (int i = 0; i < S::kNX; ++i) {
+      constexpr int n = S::kRunX * S::kPX;
+      const int q = piece(i, 2 * n);
+      const uint32_t o = (uint32_t)((b * kB + (q < n ? offA : offB)) * (S::kCi * 2) + (q < n ? q : q - n) * 16);
+      px[i] = *reinterpret_cast<const bf16x8*>(xb + (o < xbytes ? o : 0u));
+    }
+  };
+  auto store = [&](int b, lds_bf16* buf) {
+#pragma unroll
+    for (int i = 0; i < S::kNY; ++i) {
+      const int q = piece(i, kB * S::kPY), row = q / S::kPY;
+      bf16x8 v = py[i];
+      if (b * kB + row >= M)  // rows past the end meet rows of zeros, but may not be infinite
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (bf16)0.0f;
+      *reinterpret_cast<__attribute__((address_space(3))) bf16x8*>(buf + row * S::kLdY + (q % S::kPY) * 8) = v;
+    }
+#pragma unroll
+    for (int i = 0; i < S::kNX; ++i) {
+      const int q = piece(i, 2 * S::kRunX * S::kPX);
+      *reinterpret_cast<__attribute__((address_space(3))) bf16x8*>(buf + kB * S::kLdY + (q / S::kPX) * S::kLdX +
+                                                                    (q % S::kPX) * 8) = px[i];
+    }
+  };
+  // the lane's voxel of the block (kB = 32: lanes 32.. repeat), advanced by kB voxels per block
+  int dz, dyo, dx;
+  tap_offset(min(t, 26), 27, a.dil, dz, dyo, dx);
+  int m = b0 * kB + (lane & (kB - 1));
+  int vx = m % a.X, vy = m / a.X % a.Y, vz = m / (a.X * a.Y) % a.Z;
+  const int ax = kB % a.X, ay = kB / a.X % a.Y, az = kB / (a.X * a.Y) % a.Z;
+  uint64_t inside = 0;  // bit v: voxel v of the block has its neighbour inside the grid
+  auto look = [&]() {
+    const int zz = vz + dz, yy = vy + dyo, xx = vx + dx;
+    inside = __ballot(m < M && (unsigned)zz < (unsigned)a.Z && (unsigned)yy < (unsigned)a.Y &&
+                      (unsigned)xx < (unsigned)a.X);
+    m += kB;
+    vx += ax;
+    if (vx >= a.X) vx -= a.X, ++vy;
+    vy += ay;
+    if (vy >= a.Y) vy -= a.Y, ++vz;
+    vz += az;
+    if (vz >= a.Z) vz -= a.Z;
+  };
+  // the lane's part of a transposing read: row (kg * 8 + (lane % 16) / 4) of
+  // the step's 16, channels 16 ((lane / 16) % 2) + 4 (lane % 4)
+  const int rrow = kg * 8 + (lane & 15) / 4, rcol = (lane & 16) + (lane & 3) * 4;
+  const int xrow = ((t / 3 == gA ? 0 : S::kRunX) + (t % 3) * a.dil);  // the tap's first row in the staged runs
+  bf16x8 fy[2][TM], fx[2][TN];
+  auto load_step = [&](int k, const lds_bf16* buf) {
+    const lds_bf16* y = buf + (k * 16 + rrow) * S::kLdY + rcol;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const s16x4 lo = lds_tr(y + j * 32), hi = lds_tr(y + 4 * S::kLdY + j * 32);
+      fy[k & 1][j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    const lds_bf16* x = buf + kB * S::kLdY + (xrow + k * 16 + rrow) * S::kLdX;
+    const uint32_t bits = (uint32_t)(inside >> (k * 16)) >> rrow;
+    const lds_bf16* x0 = ((bits & 1u) ? x : zero) + rcol;
+    const lds_bf16* x1 = ((bits & 16u) ? x + 4 * S::kLdX : zero) + rcol;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const s16x4 lo = lds_tr(x0 + j * 32), hi = lds_tr(x1 + j * 32);
+      fx[k & 1][j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+  };
+  lds_bf16 *cur = base, *nxt = base + S::kBuf, *far = base + 2 * S::kBuf;
+  fetch(b0);
+  store(b0, cur);
+  fetch(b0 + 1 < b1 ? b0 + 1 : b0);
+  __syncthreads();
+  look();
+  load_step(0, cur);
+  constexpr int kSteps = kB / 16;
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  for (int b = b0; b < b1; ++b) {  // uniform over the workgroup
+    // block b + 1 goes to the buffer last read for block b - 2, which every
+    // wave is past since block b - 1's barrier
+    store(b + 1 < b1 ? b + 1 : b, nxt);
+    fetch(b + 2 < b1 ? b + 2 : b);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kSteps; ++k) {
+      if (k + 1 < kSteps) {
+        load_step(k + 1, cur);
+      } else {
+        look();
+        load_step(0, nxt);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fy[k & 1][i], fx[k & 1][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < TM * TN; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (k == kSteps / 2 - 1) __syncthreads();
+    }
+    lds_bf16* const p = cur;
+    cur = nxt;
+    nxt = far;
+    far = p;
+  }
+  if (t >= 27) return;
+  float* const out = a.part + ((long)chunk * 27 + t) * (S::kCo * S::kCi) + 4 * kg * S::kCi + (lane & 31);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) out[(i * 32 + 8 * (e / 4) + e % 4) * S::kCi + j * 32] = acc[i][j][e];
+}
+
+// out[i] (+)= sum over chunks of part[c][i], in the chunks' order: one value
+// per thread, the loads of kRedLoads chunks in flight.
+constexpr int kRedLoads = 16;
+
+__global__ void __launch_bounds__(256) k_no_reduce_partials(const float* part, long n, int chunks, float* out,
+                                                            int accumulate) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   float s = 0.0f;
-  for (int c = 0; c < chunks; ++c) s += part[(long)c * n + i];
+  int c = 0;
+  for (; c + kRedLoads <= chunks; c += kRedLoads) {
+    float v[kRedLoads];
+#pragma unroll
+    for (int k = 0; k < kRedLoads; ++k) v[k] = part[(c + k) * n + i];
+#pragma unroll
+    for (int k = 0; k < kRedLoads; ++k) s += v[k];
+  }
+  for (; c < chunks; ++c) s += part[c * n + i];
   out[i] = accumulate ? out[i] + s : s;
 }
 
@@ -784,6 +1006,42 @@ bool conv27(const NoConvArgs& a, long M, hipStream_t st) {
   }
 }
 
+// Items are (chunk, tap group); two workgroups per CU where there are items
+// for both and the registers allow it.
+template <int TM, int TN>
+void conv27_bwd_w_launch(const NoBwdWArgs& a, int chunks, hipStream_t st) {
+  if constexpr (BwdShape<TM, TN, true>::kPairs) {
+    if (chunks * 7 > kCus) {
+      hipLaunchKernelGGL((k_no_conv27_bwd_w<TM, TN, true>), dim3(chunks * 7), dim3(256), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_no_conv27_bwd_w<TM, TN, false>), dim3(chunks * 7), dim3(256), 0, st, a);
+}
+
+template <int TM>
+void conv27_bwd_w_n(const NoBwdWArgs& a, int chunks, hipStream_t st) {
+  switch (a.Cin / 32) {
+    case 1: return conv27_bwd_w_launch<TM, 1>(a, chunks, st);
+    case 2: return conv27_bwd_w_launch<TM, 2>(a, chunks, st);
+    case 3: return conv27_bwd_w_launch<TM, 3>(a, chunks, st);
+    default: return conv27_bwd_w_launch<TM, 4>(a, chunks, st);
+  }
+}
+
+// The staged weight gradient where it applies; false: not covered.
+bool conv27_bwd_w(const NoBwdWArgs& a, long M, int chunks, hipStream_t st) {
+  const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
+  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * std::max(a.Cin, a.Cout) * 2 >= (1L << 31))
+    return false;
+  switch (a.Cout / 32) {
+    case 1: conv27_bwd_w_n<1>(a, chunks, st); return true;
+    case 2: conv27_bwd_w_n<2>(a, chunks, st); return true;
+    case 3: conv27_bwd_w_n<3>(a, chunks, st); return true;
+    default: conv27_bwd_w_n<4>(a, chunks, st); return true;
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -822,8 +1080,10 @@ int dsmc_no_conv_bwd_w(const void* x, const void* dy, float* dw, float* part, lo
   long n = (long)taps * Cout * Cin;
   if ((long)chunks * n > part_floats) return -5;
   NoBwdWArgs a{(const bf16*)x, (const bf16*)dy, part, B, Z, Y, X, Cin, Cout, taps, dil, chunk};
-  const size_t lds = (size_t)(Cout + Cin) * kLdk * sizeof(bf16);
-  hipLaunchKernelGGL(k_no_conv_bwd_w, dim3(chunks, taps), dim3(256), lds, (hipStream_t)stream, a);
+  if (!conv27_bwd_w(a, M, chunks, (hipStream_t)stream)) {
+    const size_t lds = (size_t)(Cout + Cin) * kLdk * sizeof(bf16);
+    hipLaunchKernelGGL(k_no_conv_bwd_w, dim3(chunks, taps), dim3(256), lds, (hipStream_t)stream, a);
+  }
   hipLaunchKernelGGL(k_no_reduce_partials, dim3(nb(n, 256)), dim3(256), 0, (hipStream_t)stream, part, n, chunks,
                      dw, accumulate);
   return hipGetLastError() == hipSuccess ? 0 : -3;

@@ -50,3 +50,28 @@ def test_staged_convolution(B, shape, cin, cout, dil):
     assert np.max(np.abs(g32 - yw)) <= acc + 2.0 ** -23 * np.max(np.abs(yw))
     assert np.all(np.abs(gh - hw) <= 2.0 ** -8 * np.abs(hw) + acc)
     assert np.all(np.abs(gy - yw) <= 2.0 ** -8 * np.abs(yw) + 2 * acc)
+
+
+@pytest.mark.parametrize("B,shape,cin,cout,dil,chunk", [
+    (1, (1, 1, 1), 32, 32, 1, 64), (1, (2, 3, 37), 64, 128, 8, 64), (2, (5, 7, 11), 128, 96, 2, 128),
+    (1, (4, 1, 17), 128, 128, 0, 64), (3, (3, 5, 9), 96, 32, 4, 4096), (1, (9, 3, 19), 32, 64, 9, 64),
+    # many voxels in a partial, and enough of them for two workgroups per CU
+    (1, (40, 50, 51), 32, 96, 3, 65536), (1, (40, 50, 51), 64, 32, 8, 1024), (2, (60, 50, 51), 32, 32, 1, 2048)])
+def test_staged_weight_gradient(B, shape, cin, cout, dil, chunk):
+    from cudadsmc_amd import neural
+
+    print(f"conv27 weight gradient B={B} shape={shape} cin={cin} cout={cout} dil={dil} chunk={chunk}", flush=True)
+    rng = np.random.default_rng(cin + cout + dil)
+    M = B * int(np.prod(shape))
+    x = no_ref.bf16_round(rng.standard_normal((B,) + shape + (cin,)).astype(np.float32))
+    dy = no_ref.bf16_round(rng.standard_normal((B,) + shape + (cout,)).astype(np.float32))
+    n = 27 * cout * cin
+    part = torch.full(((M + chunk - 1) // chunk * n,), float("nan"), device="cuda")  # no partial may be read unwritten
+    dw = torch.full((27, cout, cin), 7.0, device="cuda")
+    want = no_ref.conv_grad_w(x, dy, 27, dil)
+    for times, accumulate in ((1, False), (2, True)):
+        neural.conv_bwd_w(bf(x).reshape(M, cin), bf(dy).reshape(M, cout), dw, part, B, shape, cin, cout, 27, dil,
+                          chunk=chunk, accumulate=accumulate)
+        got = dw.cpu().numpy()
+        # FP32 accumulation, as in the tests of the general kernel: 2e-5 of the largest value
+        assert np.max(np.abs(got - times * want)) <= 2e-5 * np.max(np.abs(times * want))
