@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 typedef __bf16 bf16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -191,6 +192,9 @@ __global__ void __launch_bounds__(256) k_no_conv_fwd(NoConvArgs a) {
 // the last taps of the tile before, and the output stores drain beside its
 // first ones. XCD w mod 8 takes a contiguous eighth of the tiles, so that
 // the neighbouring rows which its workgroups share sit in one L2.
+//
+// 96 -> 96 channels, 524288 voxels: 594 -> 298 us (440 -> 876 TFLOP/s; a
+// large library product reaches 1220 here).
 constexpr int kConvMaxDil = 8;  // the staged runs are sized for dilations up to this
 constexpr int kConvLds = 160 * 1024;
 constexpr int kCus = 256;
@@ -219,6 +223,75 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   p[0] = (bf16)lo;
   p[1] = (bf16)hi;
   return __builtin_bit_cast(uint32_t, p);
+}
+
+// Bias, ReLU, residual and stores of 32 voxels. A lane holds voxel m and, per
+// group q of four values of tile j, channels j * 32 + 8 q + 4 kg + (0..3);
+// the half-waves exchange groups so that a lane moves eight consecutive
+// channels (16 bytes): those of group 2 p for kg = 0, of 2 p + 1 for kg = 1.
+template <int NT>
+__device__ __forceinline__ void conv_store(const NoConvArgs& a, int m, int M, int kg, f32x16 (&acc)[NT]) {
+  constexpr int kCout = NT * 32;
+  const long row = (long)(m < M ? m : 0) * kCout + 8 * kg;
+  uint4 res[NT][2];
+  if (a.res) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) res[j][p] = *reinterpret_cast<const uint4*>(a.res + row + j * 32 + 16 * p);
+  }
+  if (a.bias)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[j][i] += a.bias[j * 32 + 8 * (i / 4) + 4 * kg + i % 4];
+  if (a.relu)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[j][i] = acc[j][i] > 0.0f ? acc[j][i] : 0.0f;
+  auto store_bf16 = [&](bf16* dst) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const f32x16& v = acc[j];
+        uint4 o = make_uint4(pack_bf16(v[8 * p], v[8 * p + 1]), pack_bf16(v[8 * p + 2], v[8 * p + 3]),
+                             pack_bf16(v[8 * p + 4], v[8 * p + 5]), pack_bf16(v[8 * p + 6], v[8 * p + 7]));
+        half_swap(o.x, o.z);
+        half_swap(o.y, o.w);
+        if (m < M) *reinterpret_cast<uint4*>(dst + row + j * 32 + 16 * p) = o;
+      }
+  };
+  if (a.h) store_bf16(a.h);
+  if (a.res) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        uint4 o = res[j][p];
+        half_swap(o.x, o.z);
+        half_swap(o.y, o.w);
+        const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc[j][8 * p + 2 * e] += __uint_as_float(w[e] << 16);
+          acc[j][8 * p + 2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
+        }
+      }
+  }
+  if (a.y32 && m < M) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[j][4 * q + e];
+        *reinterpret_cast<f32x4*>(a.y32 + (long)m * kCout + j * 32 + 8 * q + 4 * kg) = v;
+      }
+  }
+  if (a.y) store_bf16(a.y);
 }
 
 template <int KS, int NT, int R>
@@ -386,76 +459,49 @@ __global__ void __launch_bounds__(256, 1) k_no_conv27(NoConvArgs a, int tiles) {
         wbuf ^= 1;
       }
     }
-    // Epilogue. A lane holds voxel col of each tile and, per group q of four
-    // values, channels j * 32 + 8 q + 4 kg + (0..3); the half-waves exchange
-    // groups so that a lane moves eight consecutive channels (16 bytes):
-    // those of group 2 p for kg = 0, of group 2 p + 1 for kg = 1.
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int m = m0 + r * 32 + col;
-      const long row = (long)(m < M ? m : 0) * S::kCout + 8 * kg;
-      uint4 res[NT][2];
-      if (a.res) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int p = 0; p < 2; ++p)
-            res[j][p] = *reinterpret_cast<const uint4*>(a.res + row + j * 32 + 16 * p);
-      }
-      if (a.bias)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[r][j][i] += a.bias[j * 32 + 8 * (i / 4) + 4 * kg + i % 4];
-      if (a.relu)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[r][j][i] = acc[r][j][i] > 0.0f ? acc[r][j][i] : 0.0f;
-      auto store_bf16 = [&](bf16* dst) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const f32x16& v = acc[r][j];
-            uint4 o = make_uint4(pack_bf16(v[8 * p], v[8 * p + 1]), pack_bf16(v[8 * p + 2], v[8 * p + 3]),
-                                 pack_bf16(v[8 * p + 4], v[8 * p + 5]), pack_bf16(v[8 * p + 6], v[8 * p + 7]));
-            half_swap(o.x, o.z);
-            half_swap(o.y, o.w);
-            if (m < M) *reinterpret_cast<uint4*>(dst + row + j * 32 + 16 * p) = o;
-          }
-      };
-      if (a.h) store_bf16(a.h);
-      if (a.res) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            uint4 o = res[j][p];
-            half_swap(o.x, o.z);
-            half_swap(o.y, o.w);
-            const uint32_t w[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              acc[r][j][8 * p + 2 * e] += __uint_as_float(w[e] << 16);
-              acc[r][j][8 * p + 2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
-            }
-          }
-      }
-      if (a.y32 && m < M) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            f32x4 v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[r][j][4 * q + e];
-            *reinterpret_cast<f32x4*>(a.y32 + (long)m * S::kCout + j * 32 + 8 * q + 4 * kg) = v;
-          }
-      }
-      if (a.y) store_bf16(a.y);
-    }
+    for (int r = 0; r < R; ++r) conv_store<NT>(a, m0 + r * 32 + col, M, kg, acc[r]);
     m0 = m_next;
+  }
+}
+
+// conv_fwd for one tap: reading x and writing y bound it. A wave keeps the
+// weights in registers and walks over tiles of 32 voxels, the next tile's
+// rows on their way while this one is multiplied. Same sums as k_no_conv_fwd.
+// 524288 voxels: 96 -> 32 channels 50 -> 22 us, 32 -> 96 75 -> 26 us.
+template <int KS, int NT>
+__global__ void __launch_bounds__(256) k_no_conv1(NoConvArgs a, int tiles) {
+  constexpr int kCin = KS * 16;
+  const int lane = threadIdx.x & 63;
+  const int col = lane & 31, kg = lane >> 5;
+  const int M = a.B * a.Z * a.Y * a.X;
+  const int waves = gridDim.x * kWaves;
+  int tile = blockIdx.x * kWaves + (threadIdx.x >> 6);
+  if (tile >= tiles) return;
+  bf16x8 wf[KS][NT], xf[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      wf[k][j] = *reinterpret_cast<const bf16x8*>(a.w + (j * 32 + col) * kCin + k * 16 + kg * 8);
+  auto fetch = [&](int t) {
+    const int m = min(t * 32 + col, M - 1);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) xf[k] = *reinterpret_cast<const bf16x8*>(a.x + (long)m * kCin + k * 16 + kg * 8);
+  };
+  fetch(tile);
+  for (; tile < tiles; tile += waves) {
+    f32x16 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[j][i] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k][j], xf[k], acc[j], 0, 0, 0);
+    fetch(min(tile + waves, tiles - 1));
+    conv_store<NT>(a, tile * 32 + col, M, kg, acc);
   }
 }
 
@@ -812,31 +858,78 @@ __global__ void __launch_bounds__(256) k_no_reduce_partials(const float* part, l
   out[i] = accumulate ? out[i] + s : s;
 }
 
-// db[co] partial sums: workgroup b sums voxels [b * kBiasChunk, (b + 1) *
-// kBiasChunk) of every channel into part[b][co]; each thread takes channel
-// co = 32 j + (t mod 32) and every eighth voxel (coalesced 64-byte rows),
-// and the eight voxel lanes are added in a fixed order.
+// db[co] partial sums: part[b][co] sums voxels [b * kBiasChunk, (b + 1) *
+// kBiasChunk). A thread takes eight channels (16 bytes) and every eighth
+// voxel, and the eight voxel lanes are added in a fixed order; a workgroup of
+// 256 threads takes 256 / Cout chunks. FUSE: dz = dy * (h > 0) is formed and
+// stored on the way, and its sums taken. 524288 x 96: 69 -> 20 us for the sums
+// alone; with the ReLU 54 us in place of 136 + 69.
 constexpr int kBiasChunk = 512;
 
-__global__ void __launch_bounds__(256) k_no_bias_grad(const bf16* dy, long M, int Cout, float* part) {
-  __shared__ float red[8][kMaxC];
-  const int t = threadIdx.x, cl = t & 31, vl = t >> 5;
-  const long m0 = (long)blockIdx.x * kBiasChunk;
-  for (int j = 0; j < Cout / 32; ++j) {
-    const int co = j * 32 + cl;
-    float s = 0.0f;
-#pragma unroll 8
-    for (int i = vl; i < kBiasChunk; i += 8) {
-      const long m = m0 + i;
-      if (m < M) s += bf2f(dy[m * Cout + co]);
+template <bool FUSE, bool VEC>
+__global__ void __launch_bounds__(256) k_no_bias_grad(const bf16* dy, const bf16* h, bf16* dz, long M, int Cout,
+                                                      float* part) {
+  __shared__ float red[8][256];
+  const int t = threadIdx.x, pieces = Cout / 8;
+  const int sub = t / Cout, vl = t % Cout / pieces, pc = t % pieces;  // chunk of the workgroup, voxel lane, channels 8 pc..
+  const int per = 256 / Cout;
+  const long chunk = (long)blockIdx.x * per + sub;
+  const long m0 = chunk * kBiasChunk;
+  if (sub < per) {
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.0f;
+    auto load = [](const bf16* p) {
+      bf16x8 v;
+      if (VEC) {
+        v = *reinterpret_cast<const bf16x8*>(p);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[e];
+      }
+      return v;
+    };
+    auto batch = [&](int i, auto whole) {  // voxels i, i + 8, ... i + 56; whole: all of them exist
+      bf16x8 v[8], act[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {  // past the end: the last voxel's values, not used
+        const long m = m0 + i + 8 * k;
+        const long at = (whole() ? m : min(m, M - 1)) * Cout + pc * 8;
+        v[k] = load(dy + at);
+        if (FUSE) act[k] = load(h + at);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const long m = m0 + i + 8 * k;
+        if (!whole() && m >= M) break;
+        if (FUSE) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[k][e] = bf2f(act[k][e]) > 0.0f ? v[k][e] : (bf16)0.0f;
+          bf16* const o = dz + m * Cout + pc * 8;
+          if (VEC) {
+            *reinterpret_cast<bf16x8*>(o) = v[k];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = v[k][e];
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += bf2f(v[k][e]);
+      }
+    };
+    if (m0 + kBiasChunk <= M) {
+      for (int i = vl; i < kBiasChunk; i += 64) batch(i, std::true_type{});
+    } else {
+      for (int i = vl; i < kBiasChunk && m0 + i < M; i += 64) batch(i, std::false_type{});
     }
-    red[vl][co] = s;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[vl][sub * Cout + pc * 8 + e] = s[e];
   }
   __syncthreads();
-  if (t < Cout) {
+  if (sub < per && m0 < M) {
     float s = 0.0f;
     for (int v = 0; v < 8; ++v) s += red[v][t];
-    part[(long)blockIdx.x * Cout + t] = s;
+    part[chunk * Cout + t % Cout] = s;
   }
 }
 
@@ -857,11 +950,22 @@ __global__ void __launch_bounds__(256) k_no_reduce_rows(const float* part, int n
   if (t == 0) out[i] = accumulate ? out[i] + red[0] : red[0];
 }
 
-// dz = dy * (h > 0)  (ReLU backward through the stored activation)
+// dz = dy * (h > 0)  (ReLU backward through the stored activation), eight
+// values per thread (16 bytes) where the arrays are 16-byte aligned (50M
+// values: 136 -> 48 us; one value per thread keeps too few bytes in flight)
+template <int W>
 __global__ void k_no_relu_bwd(const bf16* dy, const bf16* h, bf16* dz, long n) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * W;
   if (i >= n) return;
-  dz[i] = bf2f(h[i]) > 0.0f ? dy[i] : (bf16)0.0f;
+  if (W == 8 && i + W <= n) {
+    bf16x8 g = *reinterpret_cast<const bf16x8*>(dy + i);
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(h + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = bf2f(a[e]) > 0.0f ? g[e] : (bf16)0.0f;
+    *reinterpret_cast<bf16x8*>(dz + i) = g;
+    return;
+  }
+  for (long q = i; q < n && q < i + W; ++q) dz[q] = bf2f(h[q]) > 0.0f ? dy[q] : (bf16)0.0f;
 }
 
 // c = a + b
@@ -874,30 +978,37 @@ __global__ void k_no_add(const bf16* a, const bf16* b, bf16* c, long n) {
 // Masked mean-squared error of pred [M][C] (FP32, only the first Cf channels
 // are fields) against target [M][Cf]; dpred = 2 (pred - target) mask / count,
 // written as BF16 [M][C] (zero in the padding channels); per-block loss sums.
-__global__ void k_no_mse(const float* pred, const float* target, const float* mask, long M, int C, int Cf,
-                         float inv_count, bf16* dpred, float* loss_part) {
-  __shared__ float red[256];
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// A wave takes the 256 elements of a block, four per lane; only the field
+// channels of pred are read. 524288 x 32: 49 -> 26 us (64-bit divisions per
+// element before).
+__global__ void __launch_bounds__(256) k_no_mse(const float* pred, const float* target, const float* mask, long M,
+                                                int C, int Cf, float inv_count, bf16* dpred, float* loss_part) {
+  const long n = M * C;
+  const long block = (long)blockIdx.x * 4 + threadIdx.x / 64;
+  const long i0 = block * 256 + (threadIdx.x & 63) * 4;
+  if (block * 256 >= n) return;
   float l = 0.0f;
-  if (i < M * C) {
-    long m = i / C;
-    int c = (int)(i - m * C);
+  long m = i0 < (1L << 32) ? (long)((uint32_t)i0 / (uint32_t)C) : i0 / C;
+  int c = (int)(i0 - m * C);
+  bf16x4 out;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
     float g = 0.0f;
-    if (c < Cf) {
-      float w = mask ? mask[m] : 1.0f;
-      float d = (pred[i] - target[m * Cf + c]) * w;
-      l = d * d * inv_count;
+    if (i0 + k < n && c < Cf) {
+      const float w = mask ? mask[m] : 1.0f;
+      const float d = (pred[i0 + k] - target[m * Cf + c]) * w;
+      l += d * d * inv_count;
       g = 2.0f * d * inv_count;
     }
-    dpred[i] = (bf16)g;
+    out[k] = (bf16)g;
+    if (++c == C) c = 0, ++m;
   }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
+  if (i0 + 4 <= n && (reinterpret_cast<uintptr_t>(dpred) & 7u) == 0u)
+    *reinterpret_cast<bf16x4*>(dpred + i0) = out;
+  else
+    for (int k = 0; k < 4 && i0 + k < n; ++k) dpred[i0 + k] = out[k];
+  for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off);
+  if ((threadIdx.x & 63) == 0) loss_part[block] = l;
 }
 
 // Adam on FP32 master weights, BF16 copy refreshed.
@@ -952,6 +1063,7 @@ __global__ void k_no_inputs(const float* p, const float* sphere, const float* bo
 
 // ------------------------------------------------------------------ C ABI
 static inline unsigned nb(long n, int t) { return (unsigned)((n + t - 1) / t); }
+static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0u; }
 #define NO_EMPTY(n) \
   if ((n) <= 0) return 0
 
@@ -992,11 +1104,42 @@ bool conv27_n(const NoConvArgs& a, long M, hipStream_t st) {
   }
 }
 
+template <int KS>
+bool conv1_n(const NoConvArgs& a, long M, hipStream_t st) {
+  const unsigned tiles = nb(M, 32);
+  const dim3 grid(std::min(nb(tiles, kWaves), 4u * kCus));  // four workgroups per CU
+  switch (a.Cout / 32) {
+    case 1: hipLaunchKernelGGL((k_no_conv1<KS, 1>), grid, dim3(256), 0, st, a, (int)tiles); break;
+    case 2: hipLaunchKernelGGL((k_no_conv1<KS, 2>), grid, dim3(256), 0, st, a, (int)tiles); break;
+    case 3: hipLaunchKernelGGL((k_no_conv1<KS, 3>), grid, dim3(256), 0, st, a, (int)tiles); break;
+    default: hipLaunchKernelGGL((k_no_conv1<KS, 4>), grid, dim3(256), 0, st, a, (int)tiles); break;
+  }
+  return true;
+}
+
+// The staged kernels move 16 bytes at a time; arrays that start elsewhere
+// (views at odd offsets) go to the general ones.
+bool conv_aligned(const NoConvArgs& a) {
+  return aligned16(a.x) && aligned16(a.w) && aligned16(a.res) && aligned16(a.y) && aligned16(a.y32) && aligned16(a.h);
+}
+
+bool conv1(const NoConvArgs& a, long M, hipStream_t st) {
+  if (a.taps != 1 || M >= (1L << 31) - 64 || !conv_aligned(a)) return false;
+  switch (a.Cin) {
+    case 32: return conv1_n<2>(a, M, st);
+    case 64: return conv1_n<4>(a, M, st);
+    case 96: return conv1_n<6>(a, M, st);
+    case 128: return conv1_n<8>(a, M, st);
+    default: return false;
+  }
+}
+
 // The staged kernel for the shapes that it covers; false: not covered.
 bool conv27(const NoConvArgs& a, long M, hipStream_t st) {
   // byte offsets into x, from a run's start before the first voxel to past the last workgroup's voxels, fit an int
   const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
-  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * a.Cin * 2 >= (1L << 31)) return false;
+  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * a.Cin * 2 >= (1L << 31) || !conv_aligned(a))
+    return false;
   switch (a.Cin) {
     case 32: return conv27_n<2>(a, M, st);
     case 64: return conv27_n<4>(a, M, st);
@@ -1032,7 +1175,8 @@ void conv27_bwd_w_n(const NoBwdWArgs& a, int chunks, hipStream_t st) {
 // The staged weight gradient where it applies; false: not covered.
 bool conv27_bwd_w(const NoBwdWArgs& a, long M, int chunks, hipStream_t st) {
   const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
-  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * std::max(a.Cin, a.Cout) * 2 >= (1L << 31))
+  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * std::max(a.Cin, a.Cout) * 2 >= (1L << 31) ||
+      !aligned16(a.x) || !aligned16(a.dy))
     return false;
   switch (a.Cout / 32) {
     case 1: conv27_bwd_w_n<1>(a, chunks, st); return true;
@@ -1040,6 +1184,24 @@ bool conv27_bwd_w(const NoBwdWArgs& a, long M, int chunks, hipStream_t st) {
     case 3: conv27_bwd_w_n<3>(a, chunks, st); return true;
     default: conv27_bwd_w_n<4>(a, chunks, st); return true;
   }
+}
+
+template <bool FUSE>
+int bias_grad(const void* dy, const void* h, void* dz, long M, int Cout, float* db, float* part, long part_floats,
+              int accumulate, hipStream_t st) {
+  NO_EMPTY(M);
+  if (Cout % 32 || Cout > kMaxC) return -1;
+  const int chunks = (int)nb(M, kBiasChunk);
+  if ((long)chunks * Cout > part_floats) return -5;
+  const dim3 grid(nb(chunks, 256 / Cout));
+  if (aligned16(dy) && aligned16(h) && aligned16(dz))
+    hipLaunchKernelGGL((k_no_bias_grad<FUSE, true>), grid, dim3(256), 0, st, (const bf16*)dy, (const bf16*)h, (bf16*)dz,
+                       M, Cout, part);
+  else
+    hipLaunchKernelGGL((k_no_bias_grad<FUSE, false>), grid, dim3(256), 0, st, (const bf16*)dy, (const bf16*)h,
+                       (bf16*)dz, M, Cout, part);
+  hipLaunchKernelGGL(k_no_reduce_rows, dim3(Cout), dim3(256), 0, st, part, Cout, chunks, db, accumulate);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 }  // namespace
@@ -1055,7 +1217,7 @@ int dsmc_no_conv_fwd(const void* x, const void* w, const float* bias, const void
                B, Z, Y, X, Cin, Cout, taps, dil, relu};
   long M = (long)B * Z * Y * X;
   NO_EMPTY(M);
-  if (conv27(a, M, (hipStream_t)stream)) return hipGetLastError() == hipSuccess ? 0 : -3;
+  if (conv27(a, M, (hipStream_t)stream) || conv1(a, M, (hipStream_t)stream)) return hipGetLastError() == hipSuccess ? 0 : -3;
   const size_t lds = 2ull * Cout * (Cin + 8) * sizeof(bf16);  // two taps of weights
   hipLaunchKernelGGL(k_no_conv_fwd, dim3(nb(M, 32 * kWaves)), dim3(256), lds, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
@@ -1091,21 +1253,22 @@ int dsmc_no_conv_bwd_w(const void* x, const void* dy, float* dw, float* part, lo
 
 int dsmc_no_bias_grad(const void* dy, long M, int Cout, float* db, float* part, long part_floats, int accumulate,
                       void* stream) {
-  NO_EMPTY(M);
-  if (Cout % 32 || Cout > kMaxC) return -1;
-  int chunks = (int)nb(M, kBiasChunk);
-  if ((long)chunks * Cout > part_floats) return -5;
-  hipLaunchKernelGGL(k_no_bias_grad, dim3(chunks), dim3(256), 0, (hipStream_t)stream, (const bf16*)dy, M, Cout,
-                     part);
-  hipLaunchKernelGGL(k_no_reduce_rows, dim3(Cout), dim3(256), 0, (hipStream_t)stream, part, Cout, chunks, db,
-                     accumulate);
-  return hipGetLastError() == hipSuccess ? 0 : -3;
+  return bias_grad<false>(dy, nullptr, nullptr, M, Cout, db, part, part_floats, accumulate, (hipStream_t)stream);
+}
+
+int dsmc_no_relu_bias_bwd(const void* dy, const void* h, void* dz, long M, int Cout, float* db, float* part,
+                          long part_floats, int accumulate, void* stream) {
+  return bias_grad<true>(dy, h, dz, M, Cout, db, part, part_floats, accumulate, (hipStream_t)stream);
 }
 
 int dsmc_no_relu_bwd(const void* dy, const void* h, void* dz, long n, void* stream) {
   NO_EMPTY(n);
-  hipLaunchKernelGGL(k_no_relu_bwd, dim3(nb(n, 256)), dim3(256), 0, (hipStream_t)stream, (const bf16*)dy,
-                     (const bf16*)h, (bf16*)dz, n);
+  if (aligned16(dy) && aligned16(h) && aligned16(dz))
+    hipLaunchKernelGGL(k_no_relu_bwd<8>, dim3(nb(n, 256 * 8)), dim3(256), 0, (hipStream_t)stream, (const bf16*)dy,
+                       (const bf16*)h, (bf16*)dz, n);
+  else
+    hipLaunchKernelGGL(k_no_relu_bwd<1>, dim3(nb(n, 256)), dim3(256), 0, (hipStream_t)stream, (const bf16*)dy,
+                       (const bf16*)h, (bf16*)dz, n);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -1119,7 +1282,7 @@ int dsmc_no_add(const void* a, const void* b, void* c, long n, void* stream) {
 int dsmc_no_mse(const float* pred, const float* target, const float* mask, long M, int C, int Cf, float inv_count,
                 void* dpred, float* loss_part, void* stream) {
   NO_EMPTY(M * C);
-  hipLaunchKernelGGL(k_no_mse, dim3(nb(M * C, 256)), dim3(256), 0, (hipStream_t)stream, pred, target, mask, M, C,
+  hipLaunchKernelGGL(k_no_mse, dim3(nb(M * C, 1024)), dim3(256), 0, (hipStream_t)stream, pred, target, mask, M, C,
                      Cf, inv_count, (bf16*)dpred, loss_part);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

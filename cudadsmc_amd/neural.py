@@ -52,6 +52,7 @@ def _bind() -> C.CDLL:
         "dsmc_no_conv_bwd_w": [P, P, P, P, Lg, I, I, I, I, I, I, I, I, I, I, P],
         "dsmc_no_bias_grad": [P, Lg, I, P, P, Lg, I, P],
         "dsmc_no_relu_bwd": [P, P, P, Lg, P],
+        "dsmc_no_relu_bias_bwd": [P, P, P, Lg, I, P, P, Lg, I, P],
         "dsmc_no_add": [P, P, P, Lg, P],
         "dsmc_no_mse": [P, P, P, Lg, I, I, F, P, P, P],
         "dsmc_no_adam": [P, P, P, P, P, Lg, F, F, F, F, F, F, F, P],
@@ -100,6 +101,12 @@ def conv_bwd_w(x, dy, dw, part, B, shape, cin, cout, taps, dil, chunk=4096, accu
 def bias_grad(dy, M, cout, db, part, accumulate=False):
     _chk(_bind().dsmc_no_bias_grad(_p(dy), M, cout, _p(db), _p(part), part.numel(), int(accumulate), _stream()),
          "bias_grad")
+
+
+def relu_bias_bwd(dy, h, dz, M, cout, db, part, accumulate=False):
+    """relu_bwd and bias_grad of its result in one pass."""
+    _chk(_bind().dsmc_no_relu_bias_bwd(_p(dy), _p(h), _p(dz), M, cout, _p(db), _p(part), part.numel(),
+                                       int(accumulate), _stream()), "relu_bias_bwd")
 
 
 def relu_bwd(dy, h, dz):
@@ -228,15 +235,13 @@ class FieldOperator:
         cur = 0
         conv_fwd(self.dpred, self.flip["wh"], None, B, self.shape, C_OUT, W, 1, 1, y=self.dx[cur])
         for i in range(L, 0, -1):
-            relu_bwd(self.dx[cur][:M], self.hs[i][:M], self.dz[:M])
+            relu_bias_bwd(self.dx[cur], self.hs[i], self.dz, M, W, g[f"b{i}"], self.bpart)
             conv_bwd_w(self.xs[i - 1], self.dz, g[f"w{i}"], self.part, B, self.shape, W, W, 27, self.dil[i - 1])
-            bias_grad(self.dz, M, W, g[f"b{i}"], self.bpart)
             conv_fwd(self.dz, self.flip[f"w{i}"], None, B, self.shape, W, W, 27, self.dil[i - 1],
                      res=self.dx[cur], y=self.dx[1 - cur])
             cur = 1 - cur
-        relu_bwd(self.dx[cur][:M], self.hs[0][:M], self.dz[:M])
+        relu_bias_bwd(self.dx[cur], self.hs[0], self.dz, M, W, g["b0"], self.bpart)
         conv_bwd_w(a0, self.dz, g["w0"], self.part, B, self.shape, C_IN, W, 27, 1)
-        bias_grad(self.dz, M, W, g["b0"], self.bpart)
 
     def loss_and_grad(self, target, mask, B: int) -> "object":
         """Masked MSE of self.pred against target (FP32 [M][5]); fills dpred.

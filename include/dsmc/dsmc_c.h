@@ -386,6 +386,10 @@ int dsmc_no_conv_bwd_w(const void* x, const void* dy, float* dw, float* part, lo
 /* db[co] (+)= sum over voxels of dy[m][co]. */
 int dsmc_no_bias_grad(const void* dy, long M, int Cout, float* db, float* part, long part_floats, int accumulate,
                       void* stream);
+/* dsmc_no_relu_bwd and dsmc_no_bias_grad of its result in one pass: dz = dy
+ * where h > 0, else 0 ([M][Cout]), and db[co] (+)= sum over voxels of dz[m][co]. */
+int dsmc_no_relu_bias_bwd(const void* dy, const void* h, void* dz, long M, int Cout, float* db, float* part,
+                          long part_floats, int accumulate, void* stream);
 /* dz = dy where h > 0, else 0. */
 int dsmc_no_relu_bwd(const void* dy, const void* h, void* dz, long n, void* stream);
 /* c = a + b (BF16). */

@@ -75,3 +75,38 @@ def test_staged_weight_gradient(B, shape, cin, cout, dil, chunk):
         got = dw.cpu().numpy()
         # FP32 accumulation, as in the tests of the general kernel: 2e-5 of the largest value
         assert np.max(np.abs(got - times * want)) <= 2e-5 * np.max(np.abs(times * want))
+
+
+@pytest.mark.parametrize("M,cout,skew", [(1, 32, 0), (513, 128, 0), (1000, 96, 1), (4097, 64, 0), (70001, 96, 0)])
+def test_relu_and_bias_gradient_in_one_pass(M, cout, skew):
+    """Against the two separate kernels (the same values and sums) and the
+    float64 sums; skew: arrays that are not 16-byte aligned."""
+    from cudadsmc_amd import neural
+
+    rng = np.random.default_rng(M)
+    dy, h = (bf(rng.standard_normal(M * cout + skew))[skew:] for _ in range(2))
+    dz, dz2 = (torch.full((M * cout + skew,), 5.0, dtype=torch.bfloat16, device="cuda")[skew:] for _ in range(2))
+    part = torch.full(((M + 511) // 512 * cout,), float("nan"), device="cuda")
+    db, db2 = torch.zeros(cout, device="cuda"), torch.zeros(cout, device="cuda")
+    neural.relu_bias_bwd(dy, h, dz, M, cout, db, part)
+    neural.relu_bwd(dy, h, dz2)
+    neural.bias_grad(dz2, M, cout, db2, part)
+    want = torch.where(h > 0, dy, torch.zeros_like(dy))
+    assert torch.equal(dz, want) and torch.equal(dz2, want) and torch.equal(db, db2)
+    exact = want.double().reshape(M, cout).sum(0)
+    # FP32 sums of M BF16 values in chains of at most 64 and their partials
+    assert float((db.double() - exact).abs().max()) <= 1e-6 * float(want.double().abs().reshape(M, cout).sum(0).max())
+
+
+@pytest.mark.parametrize("M,cin,cout", [(1, 32, 32), (33, 96, 32), (127, 32, 96), (5000, 64, 128), (140001, 128, 64)])
+def test_pointwise_convolution(M, cin, cout):
+    from cudadsmc_amd import neural
+
+    rng = np.random.default_rng(M + cin)
+    x, w = bf(rng.standard_normal((M, cin))), bf(rng.standard_normal((1, cout, cin)) / np.sqrt(cin))
+    y32 = torch.full((M * cout + 64,), 3.0, device="cuda")
+    neural.conv_fwd(x, w, None, 1, (1, 1, M), cin, cout, 1, 1, y32=y32)
+    want = x.double() @ w[0].double().T
+    # FP32 accumulation of at most 128 products
+    assert float((y32[:M * cout].reshape(M, cout).double() - want).abs().max()) <= 2e-5 * float(want.abs().max())
+    assert bool((y32[M * cout:] == 3.0).all())
