@@ -13,7 +13,7 @@
 //   ntc                       : float2[ncells]      {(sigma c_r)max, remainder}
 //   samples                   : double[5][ncells]   {N, sum vx, sum vy, sum vz, sum |v|^2}
 //   RNG                       : uint32[20][n_streams] (19-word window + spare)
-// A step is scan(count) -> scatter -> cells(tile kernel) [-> inject].
+// A step is scan(count) -> scatter -> cells(tile kernel) [-> walls and inject].
 #pragma once
 #include <stdint.h>
 
@@ -146,8 +146,12 @@ struct InstDesc {
   unsigned long long* defer_bits;  // PHYSICS with a body: bit s set = slot s deferred [cap / 64 + 2]
   uint32_t* defer_list; // PHYSICS with a body: deferred slots of this step, compacted [cap]
   uint32_t n_wall_wg;   // PHYSICS with a body: workgroups of the wall pass
-  long long* wall_part;  // PHYSICS with a body: [n_wall_wg][4] each wall-pass workgroup's fixed-point sums
-                        // of the step (folded into wall_acc by one workgroup after the pass)
+  uint32_t wall_direct; // the wall pass reads the bitmask itself (small instances; else the list)
+  uint32_t n_inj_wg;    // workgroups of the freestream injection
+  uint32_t n_scatter_wg;  // workgroups of the scatter
+  uint32_t n_wall_part; // slots of wall_part (at least n_wall_wg)
+  long long* wall_part;  // PHYSICS with a body: [n_wall_part][4] each wall-pass workgroup's fixed-point sums
+                        // of the step (folded into wall_acc and cleared by the next step's scan or a host read)
   double wall_scale[2]; // fixed-point scale of a velocity change (2^36 / v_ref) and of a change of |v|^2
                         // (2^33 / v_ref^2)
   double wall_unit[2];  // value of one fixed-point unit: m v_ref / 2^36 (momentum), m v_ref^2 / 2^34 (energy)

@@ -22,11 +22,26 @@ void keys_count(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st);
 int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* cursor, bool clear_in, uint32_t* scratch,
          uint32_t* total_out, hipStream_t st);
 // Step kernels take an array of n_inst descriptors (grid.y = instance).
-void scatter(const InstDesc* d, uint32_t par, uint32_t grid, hipStream_t st, uint32_t n_inst = 1);
-// Scan of the step: which = 0 cell counts, 1 injection face counts; max_n =
-// largest count array of the batch; scratch: n_inst * (kScanMaxTiles + 1).
-void step_scan(const InstDesc* d, uint32_t n_inst, uint32_t which, uint32_t max_n, uint32_t* scratch,
-               hipStream_t st);
+//
+// Scan of the step: cell offsets and the inflow numbers of the freestream
+// faces. One launch for instances of up to kScanSmall cells, else two. With
+// 65536 cells (16 blocks of 4096) a block reads at most 240 KB of counts
+// again to find its offset, which takes less than the second launch; beyond
+// that the reading grows with the square of the cells.
+constexpr uint32_t kScanSmall = 65536;
+struct StepScan {
+  uint32_t n_cell = 0, n_face = 0;  // blocks of 4096 cells and faces (largest instance)
+  bool small = false;
+  uint32_t words() const { return n_cell + n_face; }  // scratch per instance (uint32)
+};
+StepScan step_scan_plan(uint32_t max_cells, uint32_t max_faces);
+void step_scan(const InstDesc* d, const StepScan& p, uint32_t* ts, hipStream_t st, uint32_t n_inst = 1);
+// Scatter, clearing of the counts, and the face offsets. blocks: the sum of
+// scatter_blocks over the instances; map: {instance, its block} of each block
+// (null for one instance).
+uint32_t scatter_blocks(const InstDesc& I);
+void scatter(const InstDesc* d, uint32_t par, uint32_t blocks, const uint2* map, const StepScan& p, const uint32_t* ts,
+             hipStream_t st);
 // Stable sort operator: cell offsets (n_cells + 1) and the permutation of a
 // stable sort by key (keys >= n_cells dropped, listed last). work:
 // op_sort_work_words(n, n_cells) uint32. No allocation, no memset.
@@ -35,17 +50,21 @@ int op_sort(const uint32_t* keys, uint32_t n, uint32_t n_cells, uint32_t* perm, 
             uint32_t* work, hipStream_t st);
 void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t n_vwg, hipStream_t st,
           uint32_t n_inst = 1);
-// PHYSICS wall pass over the tiles the tile kernel queued (opar = the
-// buffer the tile kernel wrote); `grid` workgroups per instance.
-void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t grid, hipStream_t st, uint32_t n_inst = 1);
+// PHYSICS: the wall pass over the particles the tile kernel deferred (opar =
+// the buffer it wrote) and the inflow; blocks and map as for the scatter.
+// Before it, instances that are not wall_direct compact the deferred
+// particles (`grid` workgroups per instance).
+uint32_t wall_blocks(const InstDesc& I);
+void defer_list(const InstDesc* d, uint32_t grid, hipStream_t st, uint32_t n_inst = 1);
+void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, const uint2* map, hipStream_t st);
+// Folds the wall sums of the last step into wall_acc (before a host read).
+void wall_sum(const InstDesc* d, hipStream_t st);
 void load_reference(const InstDesc* d, uint32_t par, uint32_t ppc, uint32_t n_threads, float sux, float suy,
                     float suz, float temp, hipStream_t st);
 void move_zero(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st);
 void load_count(const InstDesc* d, uint32_t n_streams, const float* fn, hipStream_t st);
 void load_generate(const InstDesc* d, uint32_t par, uint32_t n_streams, const float* fu, const float* fv,
                    const float* fw, const float* fT, hipStream_t st);
-void inject_count(const InstDesc* d, uint32_t n_threads, hipStream_t st, uint32_t n_inst = 1);
-void inject_generate(const InstDesc* d, uint32_t opar, uint32_t n_threads, hipStream_t st, uint32_t n_inst = 1);
 void sample_cells(const InstDesc* d, uint32_t par, uint32_t mode, uint32_t ncells, hipStream_t st);
 void validate(const InstDesc* d, uint32_t par, uint32_t n, uint32_t* bad, hipStream_t st);
 

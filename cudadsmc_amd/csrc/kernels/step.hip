@@ -1,6 +1,6 @@
 // HIP kernels of the DSMC step for gfx950 (CDNA4, wave64).
 //
-// Step = scan(count) -> scatter -> tile [-> inject], replacing the
+// Step = scan(count) -> scatter -> tile [-> walls and inject], replacing the
 // reference's CalculateCellIDs -> thrust::sort_by_key -> cudaMemset ->
 // FindCellBoundaries -> ComputeBird -> IntegrateAndProcessCollisions ->
 // SampleCellStatistics sequence (include/gpu_dsmc.inl:221-274).
@@ -97,6 +97,15 @@ __device__ __forceinline__ void count_keys(gptr<uint32_t> cnt, uint32_t key) {
 }
 
 }  // namespace
+
+// Work of a block in a launch whose instances need different numbers of
+// blocks: {instance, its block}, read from the batch's map (a solver on its
+// own has no map). A grid of the largest instance's size for each would be
+// mostly blocks that exit (an ensemble of 10k to 500k particles: 213k blocks
+// of the scatter, 100 of 150 us).
+__device__ __forceinline__ uint2 block_of(const uint2* map) {
+  return map ? gload(gmem(map) + blockIdx.x) : make_uint2(0u, blockIdx.x);
+}
 
 // ======================================================================= RNG
 // InitMersenneTwistersDev (dsmc_kernel.cu:548-562): seed every stream.
@@ -263,110 +272,160 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(uint32_t* in, uint3
   if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = *total;
 }
 
-// Step scans over a batch of instances (grid.y = instance). which = 0: the
-// cell counts (count -> cell_start, count cleared, total in ctr[1]);
-// which = 1: the injection face counts, in place (total in face_count[n]).
-// scratch: kScanMaxTiles + 1 words per instance.
-__device__ __forceinline__ void bscan_args(const InstDesc& I, uint32_t which, uint32_t*& in, uint32_t& n) {
-  in = which ? I.face_count : I.count;
-  n = which ? I.n_face_cells : I.ncells;
-}
+// Scan of the step over a batch of instances (grid.y = instance): the cell
+// counts become cell_start and the scatter's cursors, and the freestream
+// faces' inflow of the step is counted beside it (offsets: k_scatter). The
+// counts stay: the scatter clears them. Two forms:
+//
+//  * k_scan_small (instances of at most kScanSmall cells): one launch. Each
+//    block of 4096 cells sums the counts before it by itself, so no block
+//    waits for another; the last one reads 15 blocks of 16 KB from L2.
+//  * k_scan_reduce + k_scan_apply_step: block sums first, then each block adds
+//    up the sums before it (at most 4096 words).
+//
+// Blocks: [0, n_cell) cell tiles, [n_cell, n_cell + n_face) face tiles, and
+// in the launch that ends the scan one block that folds the wall sums of the
+// step before. ts: the batch's tile sums, `stride` words per instance, cells
+// first. ctr[4] still holds the step before (the scatter advances it).
+constexpr uint32_t kScanSmall = dsmc_launch::kScanSmall;
 
-__global__ void __launch_bounds__(kScanThreads) k_bscan_reduce(const InstDesc* __restrict__ D, uint32_t which,
-                                                              uint32_t* scratch) {
-  const InstDesc& I = D[blockIdx.y];
-  uint32_t* in;
-  uint32_t n;
-  bscan_args(I, which, in, n);
-  if (blockIdx.x * kScanTile >= n) return;
-  __shared__ uint32_t red[kScanThreads / 64];
-  uint32_t base = blockIdx.x * kScanTile;
-  uint32_t sum = 0;
-  if (base + kScanTile <= n && (reinterpret_cast<uintptr_t>(in) & 15u) == 0u) {
-    // a whole tile of a 16-byte aligned array: vector loads, consecutive lanes on consecutive vectors
-    const gptr<const uint4> src = gmem<const uint4>(reinterpret_cast<const uint4*>(in + base));
-#pragma unroll
-    for (uint32_t k = 0; k < kScanItems / 4u; ++k) {
-      const uint4 q = gload(src + k * kScanThreads + threadIdx.x);
-      sum += (q.x + q.y) + (q.z + q.w);
-    }
-  } else {
-#pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) {
-      uint32_t i = base + k * kScanThreads + threadIdx.x;
-      if (i < n) sum += in[i];
-    }
+// Block-wide exclusive scan of v and sum of w over NW waves; sh: 2 NW words.
+template <uint32_t NW>
+__device__ __forceinline__ uint32_t block_scan_sum(uint32_t v, uint32_t w, uint32_t& total, uint32_t& wsum,
+                                                   uint32_t* sh) {
+  const uint32_t lane = lane_id(), wid = threadIdx.x / 64u;
+  uint32_t x = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(x, off);
+    if (lane >= (uint32_t)off) x += y;
   }
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off);
-  if (lane_id() == 0) red[threadIdx.x / 64] = sum;
+  for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+  if (lane == 63) {
+    sh[wid] = x;
+    sh[NW + wid] = w;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (uint32_t w = 0; w < kScanThreads / 64; ++w) t += red[w];
-    scratch[blockIdx.y * (dsmc_launch::kScanMaxTiles + 1) + blockIdx.x] = t;
+  uint32_t before = 0u;
+  total = wsum = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < NW; ++k) {
+    before += k < wid ? sh[k] : 0u;
+    total += sh[k];
+    wsum += sh[NW + k];
+  }
+  return before + x - v;
+}
+
+__device__ __forceinline__ uint32_t face_of(const InstDesc& I, uint32_t g) {
+  uint32_t f = 0;
+  while (f < 5 && g >= I.face_off[f + 1]) ++f;
+  return f;
+}
+
+// Injection draws Philox4x32-10 under key (seed, kInjectKey1), so no stream
+// state moves and every particle is independent: the count of face cell g
+// draws counter (g, step, 0, 0); particle j of g draws (g, step, 1 + j, b)
+// for its b-th rejection block (two tries per block) and (g, step, 1 + j,
+// 2^31 + k) for its other variates.
+constexpr uint32_t kInjectKey1 = 0xBB67AE85u;
+
+__device__ __forceinline__ uint32_t inject_number(const InstDesc& I, uint32_t g, uint32_t stepno) {
+  const dsmc_rng::U32x4 c = {{g, stepno, 0u, 0u}};
+  const dsmc_rng::U32x4 r = dsmc_rng::philox4x32_10(c, I.wall_key[0], kInjectKey1);
+  return dm_f2u_sat(I.inj_lambda[face_of(I, g)] + dsmc_rng::px_unit(r.v[0]));
+}
+
+// Inflow numbers of face tile f (kScanTile faces) and their sum; NT threads.
+template <uint32_t NT>
+__device__ __forceinline__ void count_faces(const InstDesc& I, uint32_t f, uint32_t* ts, uint32_t* sh) {
+  const uint32_t stepno = I.ctr[4] + 1u;
+  uint32_t sum = 0u;
+  for (uint32_t k = threadIdx.x; k < kScanTile; k += NT) {
+    const uint32_t g = f * kScanTile + k;
+    if (g >= I.n_face_cells) break;
+    const uint32_t c = inject_number(I, g, stepno);
+    I.face_count[g] = c;
+    sum += c;
+  }
+  uint32_t total, wsum;
+  block_scan_sum<NT / 64>(0u, sum, total, wsum, sh);
+  if (threadIdx.x == 0) ts[f] = wsum;
+}
+
+// The wall pass's per-workgroup sums of one step into the running totals:
+// exact 64-bit integer sums (any order gives the same value), converted once
+// per step, and cleared, so that a fold without a step between adds nothing.
+// NT threads; red: 4 words per wave.
+template <uint32_t NT>
+__device__ __forceinline__ void fold_walls(const InstDesc& I, long long* red) {
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / 64u;
+  const gptr<long long> part = gmem(I.wall_part);
+  long long v[4] = {0, 0, 0, 0};
+  for (uint32_t w = tid; w < I.n_wall_part; w += NT)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] += part[w * 4u + k];
+      part[w * 4u + k] = 0;
+    }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    long long x = v[k];
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
+    if (lane == 0) red[wid * 4 + k] = x;
+  }
+  __syncthreads();
+  if (tid < 4) {
+    long long t = 0;
+    for (uint32_t q = 0; q < NT / 64; ++q) t += red[q * 4 + tid];
+    gmem(I.wall_acc)[tid] += (double)t * I.wall_unit[tid < 3 ? 0 : 1];
   }
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_bscan_tiles(const InstDesc* __restrict__ D, uint32_t which,
-                                                             uint32_t* scratch) {
-  const InstDesc& I = D[blockIdx.y];
-  uint32_t* in;
-  uint32_t n;
-  bscan_args(I, which, in, n);
-  if (n == 0) return;
-  uint32_t* ts = scratch + blockIdx.y * (dsmc_launch::kScanMaxTiles + 1);
-  const uint32_t n_tiles = (n + kScanTile - 1) / kScanTile;
-  __shared__ uint32_t sh[kScanThreads / 64 + 1];
-  uint32_t v[kScanItems];
-  uint32_t local = 0;
+// What the block with the last cells leaves for the step.
+__device__ __forceinline__ void scan_done(const InstDesc& I, uint32_t total) {
+  I.cell_start[I.ncells] = total;
+  I.ctr[1] = total;
+  I.ctr[5] = 0u;  // deferred particles of the step
+  for (uint32_t q = 0; q < 8u; ++q) I.ctr[kTileQueueCtr + q] = 0u;  // the tile kernel's queues
+}
+
+// Offsets and cursors of N consecutive cells from base: v their counts, off
+// the first one's offset. Whole groups move as 16-byte vectors (the engine's
+// arrays are 256-byte aligned). Instances without tile-local ranking start
+// their cursors at the offsets.
+template <uint32_t N>
+__device__ __forceinline__ void store_offsets(const InstDesc& I, uint32_t base, const uint32_t (&v)[N], uint32_t off) {
+  const uint32_t n = I.ncells;
+  if (base + N <= n) {
+    uint4 l[N / 4u];
 #pragma unroll
-  for (uint32_t k = 0; k < kScanItems; ++k) {
-    uint32_t i = threadIdx.x * kScanItems + k;
-    v[k] = i < n_tiles ? ts[i] : 0u;
-    local += v[k];
+    for (uint32_t k = 0; k < N / 4u; ++k)
+      l[k] = I.tile_dyn ? gload(gmem<const uint4>(reinterpret_cast<const uint4*>(I.local_cnt + base)) + k)
+                        : make_uint4(0u, 0u, 0u, 0u);
+    const gptr<uint4> dst = gmem(reinterpret_cast<uint4*>(I.cell_start + base));
+    const gptr<uint4> cur = gmem(reinterpret_cast<uint4*>(I.cursor + base));
+#pragma unroll
+    for (uint32_t k = 0; k < N / 4u; ++k) {
+      const uint32_t o0 = off, o1 = o0 + v[4 * k], o2 = o1 + v[4 * k + 1], o3 = o2 + v[4 * k + 2];
+      off = o3 + v[4 * k + 3];
+      gstore(dst + k, make_uint4(o0, o1, o2, o3));
+      gstore(cur + k, make_uint4(o0 + l[k].x, o1 + l[k].y, o2 + l[k].z, o3 + l[k].w));
+    }
+    return;
   }
-  uint32_t total;
-  uint32_t off = block_exclusive_scan(local, &total, sh);
-#pragma unroll
-  for (uint32_t k = 0; k < kScanItems; ++k) {
-    uint32_t i = threadIdx.x * kScanItems + k;
-    if (i < n_tiles) ts[i] = off;
+  for (uint32_t k = 0; k < N && base + k < n; ++k) {
+    I.cell_start[base + k] = off;
+    I.cursor[base + k] = off + (I.tile_dyn ? I.local_cnt[base + k] : 0u);
     off += v[k];
   }
-  if (threadIdx.x == 0) {
-    ts[dsmc_launch::kScanMaxTiles] = total;
-    if (which == 0) {
-      I.ctr[1] = total;
-      I.ctr[4] += 1u;  // step number (counter of the wall draws)
-      I.ctr[5] = 0u;   // deferred particles of the step
-      for (uint32_t q = 0; q < 8u; ++q) I.ctr[kTileQueueCtr + q] = 0u;  // the tile kernel's queues
-    }
-  }
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_bscan_apply(const InstDesc* __restrict__ D, uint32_t which,
-                                                             const uint32_t* scratch) {
-  const InstDesc& I = D[blockIdx.y];
-  uint32_t* in;
-  uint32_t n;
-  bscan_args(I, which, in, n);
-  if (blockIdx.x * kScanTile >= n) return;
-  const uint32_t* ts = scratch + blockIdx.y * (dsmc_launch::kScanMaxTiles + 1);
-  uint32_t* out = which ? I.face_count : I.cell_start;
-  __shared__ uint32_t sh[kScanThreads / 64 + 1];
-  // each thread scans kScanItems consecutive entries; a thread whose entries
-  // all lie below n moves them as 16-byte vectors when the arrays are 16-byte
-  // aligned (the engine's are 256-byte aligned; base is a multiple of 16)
-  uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-  const bool whole = base + kScanItems <= n &&
-                     ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out) |
-                       (which ? 0u : (reinterpret_cast<uintptr_t>(I.cursor) | reinterpret_cast<uintptr_t>(I.local_cnt)))) &
-                      15u) == 0u;
-  uint32_t v[kScanItems];
-  if (whole) {
-    const gptr<const uint4> src = gmem<const uint4>(reinterpret_cast<const uint4*>(in + base));
+template <uint32_t N>
+__device__ __forceinline__ void load_counts(const InstDesc& I, uint32_t base, uint32_t (&v)[N]) {
+  if (base + N <= I.ncells) {
+    const gptr<const uint4> src = gmem<const uint4>(reinterpret_cast<const uint4*>(I.count + base));
 #pragma unroll
-    for (uint32_t k = 0; k < kScanItems / 4u; ++k) {
+    for (uint32_t k = 0; k < N / 4u; ++k) {
       const uint4 q = gload(src + k);
       v[4 * k] = q.x;
       v[4 * k + 1] = q.y;
@@ -375,49 +434,120 @@ __global__ void __launch_bounds__(kScanThreads) k_bscan_apply(const InstDesc* __
     }
   } else {
 #pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) v[k] = base + k < n ? in[base + k] : 0u;
+    for (uint32_t k = 0; k < N; ++k) v[k] = base + k < I.ncells ? I.count[base + k] : 0u;
   }
-  // the cells' counts of particles that stayed in their tile (cursor =
-  // offset + count), loaded before the scan's barriers
-  uint4 l[kScanItems / 4u];
-#pragma unroll
-  for (uint32_t k = 0; k < kScanItems / 4u; ++k)
-    l[k] = (which == 0 && whole) ? gload(gmem<const uint4>(reinterpret_cast<const uint4*>(I.local_cnt + base)) + k)
-                                 : make_uint4(0u, 0u, 0u, 0u);
-  uint32_t local = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < kScanItems; ++k) local += v[k];
-  uint32_t tot;
-  uint32_t off = block_exclusive_scan(local, &tot, sh) + ts[blockIdx.x];
-  if (whole) {
-    const gptr<uint4> dst = gmem(reinterpret_cast<uint4*>(out + base));
-    const gptr<uint4> clr = gmem(reinterpret_cast<uint4*>(in + base));
+}
+
+constexpr uint32_t kSmallThreads = 1024;
+
+__global__ void __launch_bounds__(kSmallThreads) k_scan_small(const InstDesc* __restrict__ D, uint32_t n_cell,
+                                                              uint32_t n_face, uint32_t* ts, uint32_t stride) {
+  const InstDesc& I = D[blockIdx.y];
+  __shared__ __align__(8) uint32_t sh[4 * 2 * kSmallThreads / 64];
+  const uint32_t b = blockIdx.x, tid = threadIdx.x;
+  if (b >= n_cell + n_face) {
+    if (I.defer_bits) fold_walls<kSmallThreads>(I, reinterpret_cast<long long*>(sh));
+    return;
+  }
+  if (b >= n_cell) {
+    if ((b - n_cell) * kScanTile < I.n_face_cells)
+      count_faces<kSmallThreads>(I, b - n_cell, ts + blockIdx.y * stride + n_cell, sh);
+    return;
+  }
+  const uint32_t n = I.ncells;
+  if (b * kScanTile >= n) return;
+  // the counts of the tiles before this one, all of whose cells exist
+  const gptr<const uint4> src = gmem<const uint4>(reinterpret_cast<const uint4*>(I.count));
+  uint32_t pre = 0u;
+#pragma unroll 5
+  for (uint32_t k = 0; k < b; ++k) {
+    const uint4 q = gload(src + k * kSmallThreads + tid);
+    pre += (q.x + q.y) + (q.z + q.w);
+  }
+  const uint32_t base = b * kScanTile + tid * 4u;
+  uint32_t v[4];
+  load_counts<4>(I, base, v);
+  uint32_t total, before;
+  const uint32_t off = block_scan_sum<kSmallThreads / 64>((v[0] + v[1]) + (v[2] + v[3]), pre, total, before, sh);
+  store_offsets<4>(I, base, v, before + off);
+  if ((b + 1u) * kScanTile >= n && tid == 0) scan_done(I, before + total);
+}
+
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce_step(const InstDesc* __restrict__ D, uint32_t n_cell,
+                                                                  uint32_t* ts, uint32_t stride) {
+  const InstDesc& I = D[blockIdx.y];
+  __shared__ uint32_t sh[2 * kScanThreads / 64];
+  const uint32_t b = blockIdx.x;
+  uint32_t* const t = ts + blockIdx.y * stride;
+  if (b >= n_cell) {
+    if ((b - n_cell) * kScanTile < I.n_face_cells) count_faces<kScanThreads>(I, b - n_cell, t + n_cell, sh);
+    return;
+  }
+  const uint32_t n = I.ncells, base = b * kScanTile;
+  if (base >= n) return;
+  uint32_t sum = 0u;
+  if (base + kScanTile <= n) {  // consecutive lanes on consecutive vectors
+    const gptr<const uint4> src = gmem<const uint4>(reinterpret_cast<const uint4*>(I.count + base));
 #pragma unroll
     for (uint32_t k = 0; k < kScanItems / 4u; ++k) {
-      const uint32_t o0 = off, o1 = o0 + v[4 * k], o2 = o1 + v[4 * k + 1], o3 = o2 + v[4 * k + 2];
-      off = o3 + v[4 * k + 3];
-      gstore(dst + k, make_uint4(o0, o1, o2, o3));
-      if (which == 0) {
-        gstore(clr + k, make_uint4(0u, 0u, 0u, 0u));
-        gstore(gmem(reinterpret_cast<uint4*>(I.cursor + base)) + k,
-               make_uint4(o0 + l[k].x, o1 + l[k].y, o2 + l[k].z, o3 + l[k].w));
-      }
+      const uint4 q = gload(src + k * kScanThreads + threadIdx.x);
+      sum += (q.x + q.y) + (q.z + q.w);
     }
   } else {
-#pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) {
-      uint32_t i = base + k;
-      if (i < n) {
-        out[i] = off;
-        if (which == 0) {
-          in[i] = 0u;
-          I.cursor[i] = off + I.local_cnt[i];
-        }
-      }
-      off += v[k];
-    }
+    for (uint32_t i = base + threadIdx.x; i < n; i += kScanThreads) sum += I.count[i];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = ts[dsmc_launch::kScanMaxTiles];
+  uint32_t total, wsum;
+  block_scan_sum<kScanThreads / 64>(0u, sum, total, wsum, sh);
+  if (threadIdx.x == 0) t[b] = wsum;
+}
+
+__global__ void __launch_bounds__(kScanThreads) k_scan_apply_step(const InstDesc* __restrict__ D, uint32_t n_cell,
+                                                                 const uint32_t* ts, uint32_t stride) {
+  const InstDesc& I = D[blockIdx.y];
+  __shared__ __align__(8) uint32_t sh[4 * 2 * kScanThreads / 64];
+  const uint32_t b = blockIdx.x;
+  if (b >= n_cell) {
+    if (I.defer_bits) fold_walls<kScanThreads>(I, reinterpret_cast<long long*>(sh));
+    return;
+  }
+  if (b * kScanTile >= I.ncells) return;
+  const gptr<const uint32_t> t = gmem<const uint32_t>(ts + blockIdx.y * stride);
+  uint32_t pre = 0u;
+  for (uint32_t k = threadIdx.x; k < b; k += kScanThreads) pre += t[k];
+  // each thread scans kScanItems consecutive cells
+  const uint32_t base = b * kScanTile + threadIdx.x * kScanItems;
+  uint32_t v[kScanItems];
+  load_counts<kScanItems>(I, base, v);
+  uint32_t local = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < kScanItems; ++k) local += v[k];
+  uint32_t total, before;
+  const uint32_t off = block_scan_sum<kScanThreads / 64>(local, pre, total, before, sh);
+  store_offsets<kScanItems>(I, base, v, before + off);
+  if ((b + 1u) * kScanTile >= I.ncells && threadIdx.x == 0) scan_done(I, before + total);
+}
+
+// Face tile f: inflow numbers to offsets, in place (total in face_count[n]).
+__device__ __forceinline__ void offset_faces(const InstDesc& I, uint32_t f, const uint32_t* ts, uint32_t* sh) {
+  const uint32_t n = I.n_face_cells;
+  if (f * kScanTile >= n) return;
+  uint32_t pre = 0u;
+  for (uint32_t k = threadIdx.x; k < f; k += kScanThreads) pre += ts[k];
+  const uint32_t base = f * kScanTile + threadIdx.x * kScanItems;
+  uint32_t v[kScanItems], local = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    v[k] = base + k < n ? I.face_count[base + k] : 0u;
+    local += v[k];
+  }
+  uint32_t total, before;
+  uint32_t off = block_scan_sum<kScanThreads / 64>(local, pre, total, before, sh) + before;
+#pragma unroll
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    if (base + k < n) I.face_count[base + k] = off;
+    off += v[k];
+  }
+  if ((f + 1u) * kScanTile >= n && threadIdx.x == 0) I.face_count[n] = before + total;
 }
 
 // =================================================================== scatter
@@ -439,11 +569,29 @@ __global__ void __launch_bounds__(kScanThreads) k_bscan_apply(const InstDesc* __
 constexpr uint32_t kScatterRounds = 4;
 constexpr uint32_t kScatterSpan = 1024;  // cells per workgroup pass (a multiple of every tile size)
 
-__global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip, uint32_t par) {
-  const InstDesc& I = Ip[blockIdx.y];
+//
+// Beside that the launch clears the counts for the next step (the scan has
+// read them), advances the step number and, in the blocks after the instance's n_scatter_wg,
+// turns the face tiles' inflow numbers into offsets.
+__global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip, uint32_t par, const uint2* map,
+                                                 const uint32_t* face_ts, uint32_t stride) {
+  const uint2 blk = block_of(map);
+  const InstDesc& I = Ip[blk.x];
+  const uint32_t bx = blk.y, grid = I.n_scatter_wg;
   __shared__ uint32_t s_cnt[kScatterSpan];
   __shared__ uint32_t s_tp[kScatterSpan / 32u + 1u];
   const uint32_t tid = threadIdx.x;
+  if (bx >= grid) {
+    offset_faces(I, bx - grid, face_ts + blk.x * stride, s_cnt);
+    return;
+  }
+  if (bx == 0 && tid == 0) I.ctr[4] += 1u;  // step number (counter of the draws)
+  {
+    const gptr<uint4> cnt4 = gmem(reinterpret_cast<uint4*>(I.count));
+    const uint32_t n4 = I.ncells / 4u;
+    for (uint32_t i = bx * 256u + tid; i < n4; i += grid * 256u) gstore(cnt4 + i, make_uint4(0u, 0u, 0u, 0u));
+    if (bx == 0 && tid < I.ncells % 4u) I.count[4u * n4 + tid] = 0u;
+  }
   const uint32_t n = I.ctr[0];
   const gptr<const uint32_t> keys = gmem<const uint32_t>(I.key[par]);
   const gptr<const uint32_t> start = gmem<const uint32_t>(I.cell_start);
@@ -456,7 +604,7 @@ __global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip
   const uint32_t S = I.tile_dyn ? min(tp0[I.ntiles], n) : 0u;
   // tiles per pass: up to kScatterSpan cells, fewer when the instance has
   // too few tiles to give every workgroup a pass
-  const uint32_t K = max(1u, min(kScatterSpan / tile_cells, I.ntiles / gridDim.x));
+  const uint32_t K = max(1u, min(kScatterSpan / tile_cells, I.ntiles / grid));
   // Slots of the pass's tiles [t0, t0 + K) (runs starting at s_tp[]), in
   // rounds of 256 slots from q0 (below q1). Each lane keeps the tile of its
   // last slot in t (its slots only grow). A particle that stayed in its
@@ -521,7 +669,7 @@ __global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip
     }
   };
   const uint32_t passes = S ? (I.ntiles + K - 1u) / K : 0u;
-  for (uint32_t g = blockIdx.x; g < passes; g += gridDim.x) {  // uniform over the workgroup
+  for (uint32_t g = bx; g < passes; g += grid) {  // uniform over the workgroup
     const uint32_t t0 = g * K;
     const uint32_t c0 = t0 * I.tile_cells;
     for (uint32_t c = tid; c < K * tile_cells; c += 256u) s_cnt[c] = c0 + c < I.ncells ? start[c0 + c] : 0u;
@@ -535,7 +683,7 @@ __global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip
     for (uint32_t q0 = p0; q0 < p1; q0 += 256u * kScatterRounds) place_tiled(q0, p1, c0, K, t, kk);
     __syncthreads();  // s_cnt and s_tp are set again for the next pass
   }
-  for (uint32_t q0 = S + blockIdx.x * 256u * kScatterRounds; q0 < n; q0 += gridDim.x * 256u * kScatterRounds)
+  for (uint32_t q0 = S + bx * 256u * kScatterRounds; q0 < n; q0 += grid * 256u * kScatterRounds)
     place_rest(q0, n);
 }
 
@@ -1166,7 +1314,7 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __rest
                             per_xcd, e, &s_pop, s_start[b ^ 1u],
                              s_nearc[b ^ 1u], pf, s_raw, s_perm, s_owner, s_vx, s_vy, s_vz, stepno, ntl, cacc);
     __syncthreads();
-    if (tid < nc) gmem(I.local_cnt)[c0 + tid] = s_ntc_off[tid];
+    if (I.tile_dyn && tid < nc) gmem(I.local_cnt)[c0 + tid] = s_ntc_off[tid];
     tile = tile_n;
   }
 
@@ -1197,14 +1345,14 @@ template __global__ void k_tile<kModePhysics>(const InstDesc*, uint32_t, uint32_
 // after collisions, before the move; one bit per slot in defer_bits) fly
 // with walls and faces here, in two launches.
 //
-// k_defer_list compacts the marked slots: each wave takes chunks of 64
+// k_defer_list (large instances) compacts the marked slots: each wave takes chunks of 64
 // bitmask words (4096 slots) and finds their set bits with one coalesced
 // load; the workgroup reserves room for its waves' chunks in defer_list with
 // one atomic; each word's slots are written as one contiguous run (lane l
 // tests bit l) and the words cleared.
 __global__ void __launch_bounds__(kTileThreads) k_defer_list(const InstDesc* __restrict__ Ip) {
   const InstDesc& I = Ip[blockIdx.y];
-  if (!I.defer_bits || blockIdx.x >= I.n_wall_wg) return;
+  if (!I.defer_bits || I.wall_direct || blockIdx.x >= I.n_wall_wg) return;
   __shared__ uint32_t s_tot[kTileThreads / 64u + 1u];
   const uint32_t lane = lane_id(), wave = threadIdx.x / 64u;
   const uint32_t nwords = (I.ctr[1] + 63u) / 64u;  // deferred slots lie below the sorted count
@@ -1256,20 +1404,132 @@ __global__ void __launch_bounds__(kTileThreads) k_defer_list(const InstDesc* __r
   }
 }
 
-// k_walls moves the listed particles, one per thread (a grid-stride loop
-// over the list); the 64 lanes of a wavefront fly their particles together,
-// testing the triangle entries of all their cells as one pool. The pass holds no RNG state (Philox draws keyed by slot
-// and step). Wall forces and heat are summed in 64-bit fixed point, so the
-// order in which particles are listed and run does not change the sums;
-// each workgroup stores its sums in its own slot of wall_part, and
-// k_wall_sum adds them to wall_acc.
+// ================================================================= injection
+// Freestream inflow through open faces (PHYSICS): face cell g of face f
+// injects floor(lambda_f + R) particles with the flux-weighted half-range
+// Maxwellian normal velocity (acceptance-rejection on the speed-ratio
+// density z exp(-(z - s)^2), Bird 1994 sec. 12.1) and Gaussian tangential
+// components, placed on the face and advanced a random fraction of dt.
+//
+// One thread per injected particle t (workgroup ib of nib, grid-stride): its
+// face cell is the last g with face_count[g] <= t (face_count holds the
+// exclusive offsets), it is particle t - face_count[g] of that cell, and it
+// goes to slot sorted count + t.
+__device__ __forceinline__ void inject_generate(const InstDesc& I, uint32_t opar, uint32_t ib, uint32_t nib) {
+  const uint32_t F = I.n_face_cells;
+  if (F == 0) return;
+  const uint32_t t0 = ib * kTileThreads + threadIdx.x;
+  const uint32_t base = I.ctr[1];
+  const uint32_t tot = I.face_count[F];
+  if (t0 == 0) {
+    uint32_t end = base + tot;
+    if (end > I.cap || end < base) {  // capacity exceeded: drop the excess, flag it
+      end = I.cap;
+      atomicOr(&I.ctr[3], kStatusCapacity);
+    }
+    I.ctr[0] = end;
+    I.ctr[2] += end - base;
+  }
+  const uint32_t stepno = I.ctr[4];
+  const uint32_t k0 = I.wall_key[0];
+  const gptr<const uint32_t> fc = gmem<const uint32_t>(I.face_count);
+  const float twopi = 6.28318530717958647692f;
+  const float vm = I.vm_inf;
+  const float sd = vm * 0.70710678118654752f;  // sqrt(kT/m)
+  for (uint32_t t = t0; t < tot; t += nib * kTileThreads) {
+    const uint32_t idx = base + t;
+    if (idx >= I.cap || idx < base) break;  // later t only go further
+    uint32_t lo = 0u, hi = F;  // fc[lo] <= t < fc[hi]
+    while (hi - lo > 1u) {
+      const uint32_t mid = lo + (hi - lo) / 2u;
+      if (fc[mid] <= t) lo = mid;
+      else hi = mid;
+    }
+    const uint32_t g = lo, j = t - fc[g];
+    const uint32_t f = face_of(I, g);
+    const uint32_t local = g - I.face_off[f];
+    const uint32_t axis = f >> 1;           // normal axis
+    const uint32_t ta = axis == 0 ? 1u : 0u;  // first tangential axis
+    const uint32_t tb = axis == 2 ? 1u : 2u;  // second tangential axis
+    const uint32_t na = I.dim[ta];
+    const uint32_t ia = local % na, ib = local / na;
+    const float sign = (f & 1u) ? -1.0f : 1.0f;  // inward normal direction
+    const float un = sign * I.U[axis];           // inward stream component
+    const float sr = un / vm;                    // speed ratio of the inflow
+    float zlo = sr - 5.0f;
+    zlo = zlo > 0.0f ? zlo : 0.0f;
+    float zhi = sr + 5.0f;
+    zhi = zhi > 1.0e-3f ? zhi : 1.0e-3f;
+    float zs = 0.5f * (sr + sqrtf(sr * sr + 2.0f));  // mode of z exp(-(z-s)^2)
+    zs = zs < zlo ? zlo : (zs > zhi ? zhi : zs);
+    const float gmax = zs * dm_expf(-(zs - sr) * (zs - sr));
+    float z = zlo;
+    bool ok = false;
+    for (uint32_t b = 0; b < 500u && !ok; ++b) {
+      const dsmc_rng::U32x4 c = {{g, stepno, 1u + j, b}};
+      const dsmc_rng::U32x4 r = dsmc_rng::philox4x32_10(c, k0, kInjectKey1);
+      for (int h = 0; h < 2 && !ok; ++h) {
+        z = zlo + (zhi - zlo) * dsmc_rng::px_unit(r.v[2 * h]);
+        const float gz = z * dm_expf(-(z - sr) * (z - sr));
+        ok = gz > gmax * dsmc_rng::px_unit(r.v[2 * h + 1]);
+      }
+    }
+    const dsmc_rng::U32x4 ca = {{g, stepno, 1u + j, 0x80000000u}};
+    const dsmc_rng::U32x4 ra = dsmc_rng::philox4x32_10(ca, k0, kInjectKey1);
+    const dsmc_rng::U32x4 cb = {{g, stepno, 1u + j, 0x80000001u}};
+    const dsmc_rng::U32x4 rb = dsmc_rng::philox4x32_10(cb, k0, kInjectKey1);
+    const float vn = z * vm;
+    const float a1 = sqrtf(-2.0f * dm_logf(dsmc_rng::px_unit(ra.v[0])));
+    float s1, c1;
+    dm_sincosf(twopi * dsmc_rng::px_unit(ra.v[1]), &s1, &c1);
+    float p[3], v[3];
+    v[axis] = sign * vn;
+    v[ta] = I.U[ta] + sd * a1 * c1;
+    v[tb] = I.U[tb] + sd * a1 * s1;
+    p[axis] = (f & 1u) ? I.gmax[axis] : I.gmin[axis];
+    p[ta] = I.gmin[ta] + ((float)ia + dsmc_rng::px_unit(ra.v[2])) * I.cell[ta];
+    p[tb] = I.gmin[tb] + ((float)ib + dsmc_rng::px_unit(ra.v[3])) * I.cell[tb];
+    const float fr = dsmc_rng::px_unit(rb.v[0]) * I.dt;
+    float x = p[0] + v[0] * fr, y = p[1] + v[1] * fr, zz = p[2] + v[2] * fr;
+    x = x < I.gmin[0] ? I.gmin[0] : (x > I.gmax[0] ? I.gmax[0] : x);
+    y = y < I.gmin[1] ? I.gmin[1] : (y > I.gmax[1] ? I.gmax[1] : y);
+    zz = zz < I.gmin[2] ? I.gmin[2] : (zz > I.gmax[2] ? I.gmax[2] : zz);
+    I.px[opar][idx] = x; I.py[opar][idx] = y; I.pz[opar][idx] = zz;
+    I.vx[opar][idx] = v[0]; I.vy[opar][idx] = v[1]; I.vz[opar][idx] = v[2];
+    const uint32_t key = cell_key_phys(I, x, y, zz);
+    I.key[opar][idx] = key;
+    gatomic_add(gmem(I.count) + key, 1u);
+  }
+}
+
+// k_walls moves the deferred particles, one per thread; the 64 lanes of a
+// wavefront fly their particles together, testing the triangle entries of all
+// their cells as one pool. They come from the compacted list (a grid-stride
+// loop over it), or, where one small instance has the GPU to itself
+// (wall_direct), from the bitmask: each wave takes whole words, 64 slots, and
+// moves the marked lanes - the compaction's launch and round trip take longer
+// than the idle lanes (100k particles: list, walls and sum 6 + 22 + 4 us, 15
+// direct; 64 such instances together: 53 us against 154).
+// The pass holds no RNG state (Philox draws keyed by slot and step). Wall
+// forces and heat are summed in 64-bit fixed point, so the order in which
+// particles are taken does not change the sums; each workgroup stores its
+// sums in its own slot of wall_part, which the next step's scan (or the host,
+// before it reads the totals) folds into wall_acc.
+//
+// The workgroups after the instance's n_wall_wg inject the inflow beside
+// that: both only add to the cell counts, injection writes the slots after
+// the sorted ones and the wall pass deferred slots below them.
 __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __restrict__ Ip, uint32_t opar,
-                                                       uint32_t flags) {
-  const InstDesc& I = Ip[blockIdx.y];
-  if (!I.defer_bits || blockIdx.x >= I.n_wall_wg) return;
+                                                       uint32_t flags, const uint2* map) {
+  const uint2 blk = block_of(map);
+  const InstDesc& I = Ip[blk.x];
+  const uint32_t bx = blk.y, n_wg = I.defer_bits ? I.n_wall_wg : 0u;
+  if (bx >= n_wg) {
+    inject_generate(I, opar, bx - n_wg, I.n_inj_wg);
+    return;
+  }
   __shared__ long long s_red[kTileThreads / 64][4];
   __shared__ unsigned long long s_hit[kTileThreads / 64][64];
-  const uint32_t cnt = I.ctr[5];
   const uint32_t stepno = I.ctr[4];
   const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / 64;
   const gptr<float> px = gmem(I.px[opar]);
@@ -1279,19 +1539,14 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __res
   const gptr<float> vy = gmem(I.vy[opar]);
   const gptr<float> vz = gmem(I.vz[opar]);
   const gptr<uint32_t> key = gmem(I.key[opar]);
-  const gptr<const uint32_t> list = gmem<const uint32_t>(I.defer_list);
   WallAcc acc = {0, 0, 0, 0};
   const WaveHitLds hl = {s_hit[wid]};
-  // uniform trip count over the workgroup: the wall flights run the
-  // wavefront's lanes together, and the counting is wave-aggregated
-  // (neighbouring list entries mostly land in the same cell)
-  for (uint32_t b = blockIdx.x * kTileThreads; b < cnt; b += I.n_wall_wg * kTileThreads) {
-    const uint32_t i = b + tid;
-    const bool act = i < cnt;
-    uint32_t slot = 0;
+  // called by whole wavefronts: the wall flights run their lanes together,
+  // and the counting is wave-aggregated (neighbouring slots mostly land in
+  // the same cell)
+  auto fly = [&](bool act, uint32_t slot) {
     float x = 0.0f, y = 0.0f, z = 0.0f, ux = 0.0f, uy = 0.0f, uz = 0.0f;
     if (act) {
-      slot = list[i];
       x = px[slot], y = py[slot], z = pz[slot];
       ux = vx[slot], uy = vy[slot], uz = vz[slot];
     }
@@ -1308,6 +1563,23 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __res
       if (flags & kFlagHits) gmem(I.hits)[slot] = hits;
     }
     count_keys(gmem(I.count), k);
+  };
+  if (I.wall_direct) {
+    const gptr<unsigned long long> bits = gmem(I.defer_bits);
+    const uint32_t nwords = (I.ctr[1] + 63u) / 64u;  // deferred slots lie below the sorted count
+    for (uint32_t w = bx * (kTileThreads / 64u) + wid; w < nwords; w += n_wg * (kTileThreads / 64u)) {
+      const unsigned long long word = bits[w];
+      if (word == 0ull) continue;  // uniform over the wave
+      fly((word >> lane) & 1ull, w * 64u + lane);
+      if (lane == 0) bits[w] = 0ull;
+    }
+  } else {
+    const gptr<const uint32_t> list = gmem<const uint32_t>(I.defer_list);
+    const uint32_t cnt = I.ctr[5];
+    for (uint32_t b = bx * kTileThreads; b < cnt; b += n_wg * kTileThreads) {
+      const bool act = b + tid < cnt;
+      fly(act, act ? list[b + tid] : 0u);
+    }
   }
   long long v[4] = {acc.fx, acc.fy, acc.fz, acc.heat};
 #pragma unroll
@@ -1320,35 +1592,15 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __res
   if (tid < 4) {  // the workgroup's own slot: plain stores, no contention
     long long t = 0;
     for (uint32_t q = 0; q < kTileThreads / 64; ++q) t += s_red[q][tid];
-    gmem(I.wall_part)[blockIdx.x * 4u + tid] = t;
+    gmem(I.wall_part)[bx * 4u + tid] = t;
   }
 }
 
-// One workgroup per instance folds the wall pass's per-workgroup sums into
-// the running totals: exact 64-bit integer sums (any order gives the same
-// value), converted once per step.
+// Folds the wall sums that no step has folded yet, for a host read of the
+// totals.
 __global__ void __launch_bounds__(kTileThreads) k_wall_sum(const InstDesc* __restrict__ Ip) {
-  const InstDesc& I = Ip[blockIdx.y];
-  if (!I.defer_bits) return;
-  __shared__ long long s_red[kTileThreads / 64][4];
-  const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / 64;
-  const gptr<const long long> part = gmem<const long long>(I.wall_part);
-  long long v[4] = {0, 0, 0, 0};
-  for (uint32_t w = tid; w < I.n_wall_wg; w += kTileThreads)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] += part[w * 4u + k];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    long long x = v[k];
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
-    if (lane == 0) s_red[wid][k] = x;
-  }
-  __syncthreads();
-  if (tid < 4) {
-    long long t = 0;
-    for (uint32_t q = 0; q < kTileThreads / 64; ++q) t += s_red[q][tid];
-    gmem(I.wall_acc)[tid] += (double)t * I.wall_unit[tid < 3 ? 0 : 1];
-  }
+  __shared__ long long s_red[kTileThreads / 64 * 4];
+  fold_walls<kTileThreads>(*Ip, s_red);
 }
 
 // =================================================================== loading
@@ -1507,127 +1759,6 @@ __global__ void k_load_generate(const InstDesc* __restrict__ Ip, uint32_t par, c
   mt_store(I, s, rng);
 }
 
-// ================================================================= injection
-// Freestream inflow through open faces (PHYSICS): face cell g of face f
-// injects floor(lambda_f + R) particles with the flux-weighted half-range
-// Maxwellian normal velocity (acceptance-rejection on the speed-ratio
-// density z exp(-(z - s)^2), Bird 1994 sec. 12.1) and Gaussian tangential
-// components, placed on the face and advanced a random fraction of dt.
-__device__ __forceinline__ uint32_t face_of(const InstDesc& I, uint32_t g) {
-  uint32_t f = 0;
-  while (f < 5 && g >= I.face_off[f + 1]) ++f;
-  return f;
-}
-
-// Injection draws Philox4x32-10 under key (seed, kInjectKey1), so no stream
-// state moves and every particle is independent: the count of face cell g
-// draws counter (g, step, 0, 0); particle j of g draws (g, step, 1 + j, b)
-// for its b-th rejection block (two tries per block) and (g, step, 1 + j,
-// 2^31 + k) for its other variates.
-constexpr uint32_t kInjectKey1 = 0xBB67AE85u;
-
-__global__ void k_inject_count(const InstDesc* __restrict__ Ip) {
-  const InstDesc& I = Ip[blockIdx.y];
-  const uint32_t stepno = I.ctr[4];
-  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < I.n_face_cells; g += gridDim.x * blockDim.x) {
-    const dsmc_rng::U32x4 c = {{g, stepno, 0u, 0u}};
-    const dsmc_rng::U32x4 r = dsmc_rng::philox4x32_10(c, I.wall_key[0], kInjectKey1);
-    I.face_count[g] = dm_f2u_sat(I.inj_lambda[face_of(I, g)] + dsmc_rng::px_unit(r.v[0]));
-  }
-}
-
-// One thread per injected particle t (grid-stride): its face cell is the
-// last g with face_count[g] <= t (face_count holds the exclusive offsets),
-// it is particle t - face_count[g] of that cell, and it goes to slot
-// sorted count + t.
-__global__ void k_inject_generate(const InstDesc* __restrict__ Ip, uint32_t opar) {
-  const InstDesc& I = Ip[blockIdx.y];
-  const uint32_t F = I.n_face_cells;
-  if (F == 0) return;
-  const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t base = I.ctr[1];
-  const uint32_t tot = I.face_count[F];
-  if (t0 == 0) {
-    uint32_t end = base + tot;
-    if (end > I.cap || end < base) {  // capacity exceeded: drop the excess, flag it
-      end = I.cap;
-      atomicOr(&I.ctr[3], kStatusCapacity);
-    }
-    I.ctr[0] = end;
-    I.ctr[2] += end - base;
-  }
-  const uint32_t stepno = I.ctr[4];
-  const uint32_t k0 = I.wall_key[0];
-  const gptr<const uint32_t> fc = gmem<const uint32_t>(I.face_count);
-  const float twopi = 6.28318530717958647692f;
-  const float vm = I.vm_inf;
-  const float sd = vm * 0.70710678118654752f;  // sqrt(kT/m)
-  for (uint32_t t = t0; t < tot; t += gridDim.x * blockDim.x) {
-    const uint32_t idx = base + t;
-    if (idx >= I.cap || idx < base) break;  // later t only go further
-    uint32_t lo = 0u, hi = F;  // fc[lo] <= t < fc[hi]
-    while (hi - lo > 1u) {
-      const uint32_t mid = lo + (hi - lo) / 2u;
-      if (fc[mid] <= t) lo = mid;
-      else hi = mid;
-    }
-    const uint32_t g = lo, j = t - fc[g];
-    const uint32_t f = face_of(I, g);
-    const uint32_t local = g - I.face_off[f];
-    const uint32_t axis = f >> 1;           // normal axis
-    const uint32_t ta = axis == 0 ? 1u : 0u;  // first tangential axis
-    const uint32_t tb = axis == 2 ? 1u : 2u;  // second tangential axis
-    const uint32_t na = I.dim[ta];
-    const uint32_t ia = local % na, ib = local / na;
-    const float sign = (f & 1u) ? -1.0f : 1.0f;  // inward normal direction
-    const float un = sign * I.U[axis];           // inward stream component
-    const float sr = un / vm;                    // speed ratio of the inflow
-    float zlo = sr - 5.0f;
-    zlo = zlo > 0.0f ? zlo : 0.0f;
-    float zhi = sr + 5.0f;
-    zhi = zhi > 1.0e-3f ? zhi : 1.0e-3f;
-    float zs = 0.5f * (sr + sqrtf(sr * sr + 2.0f));  // mode of z exp(-(z-s)^2)
-    zs = zs < zlo ? zlo : (zs > zhi ? zhi : zs);
-    const float gmax = zs * dm_expf(-(zs - sr) * (zs - sr));
-    float z = zlo;
-    bool ok = false;
-    for (uint32_t b = 0; b < 500u && !ok; ++b) {
-      const dsmc_rng::U32x4 c = {{g, stepno, 1u + j, b}};
-      const dsmc_rng::U32x4 r = dsmc_rng::philox4x32_10(c, k0, kInjectKey1);
-      for (int h = 0; h < 2 && !ok; ++h) {
-        z = zlo + (zhi - zlo) * dsmc_rng::px_unit(r.v[2 * h]);
-        const float gz = z * dm_expf(-(z - sr) * (z - sr));
-        ok = gz > gmax * dsmc_rng::px_unit(r.v[2 * h + 1]);
-      }
-    }
-    const dsmc_rng::U32x4 ca = {{g, stepno, 1u + j, 0x80000000u}};
-    const dsmc_rng::U32x4 ra = dsmc_rng::philox4x32_10(ca, k0, kInjectKey1);
-    const dsmc_rng::U32x4 cb = {{g, stepno, 1u + j, 0x80000001u}};
-    const dsmc_rng::U32x4 rb = dsmc_rng::philox4x32_10(cb, k0, kInjectKey1);
-    const float vn = z * vm;
-    const float a1 = sqrtf(-2.0f * dm_logf(dsmc_rng::px_unit(ra.v[0])));
-    float s1, c1;
-    dm_sincosf(twopi * dsmc_rng::px_unit(ra.v[1]), &s1, &c1);
-    float p[3], v[3];
-    v[axis] = sign * vn;
-    v[ta] = I.U[ta] + sd * a1 * c1;
-    v[tb] = I.U[tb] + sd * a1 * s1;
-    p[axis] = (f & 1u) ? I.gmax[axis] : I.gmin[axis];
-    p[ta] = I.gmin[ta] + ((float)ia + dsmc_rng::px_unit(ra.v[2])) * I.cell[ta];
-    p[tb] = I.gmin[tb] + ((float)ib + dsmc_rng::px_unit(ra.v[3])) * I.cell[tb];
-    const float fr = dsmc_rng::px_unit(rb.v[0]) * I.dt;
-    float x = p[0] + v[0] * fr, y = p[1] + v[1] * fr, zz = p[2] + v[2] * fr;
-    x = x < I.gmin[0] ? I.gmin[0] : (x > I.gmax[0] ? I.gmax[0] : x);
-    y = y < I.gmin[1] ? I.gmin[1] : (y > I.gmax[1] ? I.gmax[1] : y);
-    zz = zz < I.gmin[2] ? I.gmin[2] : (zz > I.gmax[2] ? I.gmax[2] : zz);
-    I.px[opar][idx] = x; I.py[opar][idx] = y; I.pz[opar][idx] = zz;
-    I.vx[opar][idx] = v[0]; I.vy[opar][idx] = v[1]; I.vz[opar][idx] = v[2];
-    const uint32_t key = cell_key_phys(I, x, y, zz);
-    I.key[opar][idx] = key;
-    gatomic_add(gmem(I.count) + key, 1u);
-  }
-}
-
 // ================================================================== utility
 // Count particles with non-finite state or outside the box.
 __global__ void k_validate(const InstDesc* __restrict__ Ip, uint32_t par, uint32_t n, uint32_t* bad) {
@@ -1718,16 +1849,31 @@ int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* cursor, bool clear_i
   return 0;
 }
 
-void scatter(const InstDesc* d, uint32_t par, uint32_t grid, hipStream_t st, uint32_t n_inst) {
-  hipLaunchKernelGGL(k_scatter, dim3(grid, n_inst), dim3(256), 0, st, d, par);
+StepScan step_scan_plan(uint32_t max_cells, uint32_t max_faces) {
+  StepScan p;
+  p.n_cell = blocks_for(max_cells > 0 ? max_cells : 1u, kScanTile);
+  p.n_face = blocks_for(max_faces, kScanTile);
+  p.small = max_cells <= kScanSmall;
+  return p;
 }
 
-void step_scan(const InstDesc* d, uint32_t n_inst, uint32_t which, uint32_t max_n, uint32_t* scratch,
-               hipStream_t st) {
-  uint32_t tiles = blocks_for(max_n > 0 ? max_n : 1u, kScanTile);
-  hipLaunchKernelGGL(k_bscan_reduce, dim3(tiles, n_inst), dim3(kScanThreads), 0, st, d, which, scratch);
-  hipLaunchKernelGGL(k_bscan_tiles, dim3(1, n_inst), dim3(kScanThreads), 0, st, d, which, scratch);
-  hipLaunchKernelGGL(k_bscan_apply, dim3(tiles, n_inst), dim3(kScanThreads), 0, st, d, which, scratch);
+void step_scan(const InstDesc* d, const StepScan& p, uint32_t* ts, hipStream_t st, uint32_t n_inst) {
+  if (p.small) {
+    hipLaunchKernelGGL(k_scan_small, dim3(p.n_cell + p.n_face + 1, n_inst), dim3(kSmallThreads), 0, st, d, p.n_cell,
+                       p.n_face, ts, p.words());
+    return;
+  }
+  hipLaunchKernelGGL(k_scan_reduce_step, dim3(p.n_cell + p.n_face, n_inst), dim3(kScanThreads), 0, st, d, p.n_cell, ts,
+                     p.words());
+  hipLaunchKernelGGL(k_scan_apply_step, dim3(p.n_cell + 1, n_inst), dim3(kScanThreads), 0, st, d, p.n_cell, ts,
+                     p.words());
+}
+
+uint32_t scatter_blocks(const InstDesc& I) { return I.n_scatter_wg + blocks_for(I.n_face_cells, kScanTile); }
+
+void scatter(const InstDesc* d, uint32_t par, uint32_t blocks, const uint2* map, const StepScan& p, const uint32_t* ts,
+             hipStream_t st) {
+  hipLaunchKernelGGL(k_scatter, dim3(blocks), dim3(256), 0, st, d, par, map, ts + p.n_cell, p.words());
 }
 
 uint64_t op_sort_work_words(uint32_t n, uint32_t n_cells) {
@@ -1773,10 +1919,20 @@ int op_sort(const uint32_t* keys, uint32_t n, uint32_t n_cells, uint32_t* perm, 
   return 0;
 }
 
-void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t grid, hipStream_t st, uint32_t n_inst) {
-  hipLaunchKernelGGL(k_defer_list, dim3(grid, n_inst), dim3(kTileThreads), 0, st, d);
-  hipLaunchKernelGGL(k_walls, dim3(grid, n_inst), dim3(kTileThreads), 0, st, d, opar, flags);
-  hipLaunchKernelGGL(k_wall_sum, dim3(1, n_inst), dim3(kTileThreads), 0, st, d);
+uint32_t wall_blocks(const InstDesc& I) {
+  return (I.defer_bits ? I.n_wall_wg : 0u) + (I.n_face_cells ? I.n_inj_wg : 0u);
+}
+
+void defer_list(const InstDesc* d, uint32_t grid, hipStream_t st, uint32_t n_inst) {
+  if (grid) hipLaunchKernelGGL(k_defer_list, dim3(grid, n_inst), dim3(kTileThreads), 0, st, d);
+}
+
+void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, const uint2* map, hipStream_t st) {
+  if (blocks) hipLaunchKernelGGL(k_walls, dim3(blocks), dim3(kTileThreads), 0, st, d, opar, flags, map);
+}
+
+void wall_sum(const InstDesc* d, hipStream_t st) {
+  hipLaunchKernelGGL(k_wall_sum, dim3(1), dim3(kTileThreads), 0, st, d);
 }
 
 void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t n_vwg, hipStream_t st,
@@ -1806,16 +1962,6 @@ void load_count(const InstDesc* d, uint32_t n_streams, const float* fn, hipStrea
 void load_generate(const InstDesc* d, uint32_t par, uint32_t n_streams, const float* fu, const float* fv,
                    const float* fw, const float* fT, hipStream_t st) {
   hipLaunchKernelGGL(k_load_generate, dim3(blocks_for(n_streams, 256)), dim3(256), 0, st, d, par, fu, fv, fw, fT);
-}
-
-void inject_count(const InstDesc* d, uint32_t n_threads, hipStream_t st, uint32_t n_inst) {
-  if (!n_threads) return;
-  hipLaunchKernelGGL(k_inject_count, dim3(blocks_for(n_threads, 256), n_inst), dim3(256), 0, st, d);
-}
-
-void inject_generate(const InstDesc* d, uint32_t opar, uint32_t n_threads, hipStream_t st, uint32_t n_inst) {
-  if (!n_threads) return;
-  hipLaunchKernelGGL(k_inject_generate, dim3(blocks_for(n_threads, 256), n_inst), dim3(256), 0, st, d, opar);
 }
 
 void sample_cells(const InstDesc* d, uint32_t par, uint32_t mode, uint32_t ncells, hipStream_t st) {

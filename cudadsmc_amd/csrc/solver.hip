@@ -39,35 +39,11 @@ const char* global_error() { return g_err.c_str(); }
 
 using namespace dsmc_host;
 
-// A second stream (default priority) on which the freestream injection runs
-// beside the wall pass: both only add to the cell counts, injection writes
-// the slots after the sorted ones and the wall pass deferred slots below
-// them, so they may overlap; the main stream waits for the injection before
-// the next step. Under graph capture the side stream joins the capture
-// through the fork event.
-struct SideStream {
-  hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-  hipError_t create() {
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
-    return e;
-  }
-  ~SideStream() {
-    if (s) (void)hipStreamSynchronize(s);
-    if (fork) (void)hipEventDestroy(fork);
-    if (join) (void)hipEventDestroy(join);
-    if (s) (void)hipStreamDestroy(s);
-  }
-};
-
 struct dsmc_solver {
   std::string err;
   dsmc_settings s{};
   bool inited = false, have_state = false;
   hipStream_t stream = nullptr;
-  SideStream side;
   InstDesc h{};
   InstDesc* d_desc = nullptr;
   std::vector<void*> bufs;      // lifetime of the handle
@@ -94,12 +70,21 @@ struct dsmc_solver {
   // costs more than the global atomics it saves). No result depends on
   // either choice.
   double ppc_exp = 0.0;
+  // Scatter grid: tiles are ranked by up to 4096 workgroups (fewer tiles per
+  // pass fill the GPU); without tiles a workgroup takes 1024 slots per pass.
+  void set_scatter_grid() {
+    const uint32_t wg = std::min<uint32_t>((h.cap + 255u) / 256u, 4096u);
+    h.n_scatter_wg = scatter_grid ? scatter_grid : h.tile_dyn ? wg : std::min<uint32_t>((h.cap + 1023u) / 1024u, wg);
+  }
   void set_tile_schedule() { h.tile_dyn = (double)h.tile_cells * ppc_exp >= 512.0 ? 1u : 0u; }
   bool sampling = false;
   uint64_t sample_steps0 = 0;
   double acc_snap[kAccSlots] = {0};
-  uint32_t* scan_scratch = nullptr;
-  uint32_t scatter_grid = 0;
+  uint32_t* scan_scratch = nullptr;  // of the loading's scan
+  dsmc_launch::StepScan scan;        // of the step, with its tile sums
+  uint32_t* scan_ts = nullptr;
+  uint32_t n_loaded = 0;      // particles when the wall pass's grid was chosen
+  uint32_t scatter_grid = 0;  // as set by the user (0: by the engine)
   uint32_t ppc = 0;
   float ntc_init = 0.0f;
   bool timing = false;
@@ -177,6 +162,10 @@ struct dsmc_solver {
 
 namespace {
 
+// The wall pass reads the bitmask directly up to this capacity, with at most
+// this many workgroups (also over the members of a batch).
+constexpr uint32_t kWallDirectCap = 2u << 20, kWallDirectWg = 4096;
+
 const double kPi = 3.14159265358979323846;
 
 // Gamma function for the VHS constant (Lanczos approximation, g = 7).
@@ -227,7 +216,6 @@ int dsmc_create(int solver_type, dsmc_solver** out) {
     return set_global_error(DSMC_ERR_DEVICE, std::string("no HIP device: ") + hipGetErrorString(e));
   auto* h = new dsmc_solver();
   e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = h->side.create();
   if (e != hipSuccess) {
     delete h;
     return set_global_error(DSMC_ERR_DEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
@@ -482,8 +470,6 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
     HIPC(hipMemcpyAsync(I.taus, ts.data(), ts.size() * 4, hipMemcpyHostToDevice, st));
   }
   HIPC(hipStreamSynchronize(st));
-  // grid-stride scatter: 256 positions per workgroup and pass
-  h->scatter_grid = std::min<uint32_t>((cap + 255) / 256, 4096u);
   if (phys) {
     // F_n and the inflow per face for the whole box; dsmc_set_geometry
     // redoes both for the fluid volume
@@ -664,7 +650,7 @@ static std::vector<uint32_t> tile_locality_order(uint32_t X, uint32_t Y, uint32_
 }
 
 namespace {
-uint32_t wall_grid(const InstDesc& I);
+void wall_grid(InstDesc& I, uint32_t n, bool direct);
 }  // namespace
 
 static int finish_loading(dsmc_solver* h, uint32_t n, uint32_t* n_out) {
@@ -688,9 +674,13 @@ static int finish_loading(dsmc_solver* h, uint32_t n, uint32_t* n_out) {
     CHECK_RC(h->alloc(&I.defer_bits, words));
     HIPC(hipMemsetAsync(I.defer_bits, 0, words * 8, st));
     CHECK_RC(h->alloc(&I.defer_list, I.cap));
-    I.n_wall_wg = wall_grid(I);
-    CHECK_RC(h->alloc(&I.wall_part, (size_t)I.n_wall_wg * 4));
-    HIPC(hipMemsetAsync(I.wall_part, 0, (size_t)I.n_wall_wg * 4 * sizeof(long long), st));
+    wall_grid(I, n, false);  // a batch may run the member in this form
+    I.n_wall_part = I.n_wall_wg;
+    wall_grid(I, n, true);
+    I.n_wall_part = std::max(I.n_wall_part, I.n_wall_wg);
+    h->n_loaded = n;
+    CHECK_RC(h->alloc(&I.wall_part, (size_t)I.n_wall_part * 4));
+    HIPC(hipMemsetAsync(I.wall_part, 0, (size_t)I.n_wall_part * 4 * sizeof(long long), st));
     CHECK_RC(h->alloc(&I.wall_acc, 4));
     HIPC(hipMemsetAsync(I.wall_acc, 0, 4 * sizeof(double), st));
     // fixed-point units of the wall sums, from the largest of the speeds
@@ -705,6 +695,12 @@ static int finish_loading(dsmc_solver* h, uint32_t n, uint32_t* n_out) {
     I.wall_unit[1] = (double)I.mass * vref * vref / std::ldexp(1.0, 34);
     CHECK_RC(h->upload_desc());
   }
+  if (!h->scan_ts) {  // cells and open faces are fixed from here on
+    h->scan = dsmc_launch::step_scan_plan(I.ncells, I.n_face_cells);
+    CHECK_RC(h->alloc(&h->scan_ts, h->scan.words()));
+  }
+  h->set_scatter_grid();
+  CHECK_RC(h->upload_desc());
   uint32_t ctr[2] = {n, n};
   HIPC(hipMemcpyAsync(I.ctr, ctr, 8, hipMemcpyHostToDevice, st));
   HIPC(hipMemsetAsync(I.count, 0, (size_t)I.ncells * 4, st));
@@ -740,6 +736,7 @@ static int setup_injection(dsmc_solver* h) {
     I.face_off[f + 1] = total;
   }
   I.n_face_cells = total;
+  I.n_inj_wg = (std::min(I.n_streams, total) + kTileThreads - 1u) / kTileThreads;
   if (total && !I.face_count) CHECK_RC(h->alloc(&I.face_count, (size_t)total + 1));
   return DSMC_OK;
 }
@@ -941,6 +938,10 @@ int dsmc_get_fields(dsmc_solver* h, float* n, float* u, float* v, float* w, floa
 
 static int sum_acc(dsmc_solver* h, double out[kAccSlots]) {
   InstDesc& I = h->h;
+  if (I.wall_acc) {  // the last step's wall sums are folded by the next one, or here
+    dsmc_launch::wall_sum(h->d_desc, h->stream);
+    HIPC(hipGetLastError());
+  }
   std::vector<long long> acc((size_t)I.n_vwg * kAccSlots);
   HIPC(hipMemcpyAsync(acc.data(), I.wg_acc, acc.size() * 8, hipMemcpyDeviceToHost, h->stream));
   double tacc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1382,6 +1383,8 @@ int dsmc_set_scatter_grid(dsmc_solver* h, uint32_t blocks) {
   if (!h->inited) return h->fail(DSMC_ERR_STATE, "not initialised");
   if (blocks == 0 || blocks > 65535) return h->fail(DSMC_ERR_INVALID, "scatter grid must be in [1, 65535]");
   h->scatter_grid = blocks;
+  h->set_scatter_grid();
+  CHECK_RC(h->upload_desc());
   for (auto& g : h->graphs) (void)hipGraphExecDestroy(g.second);
   h->graphs.clear();
   return DSMC_OK;
@@ -1570,44 +1573,38 @@ uint32_t step_flags(const dsmc_solver* h, uint64_t stepno, bool* sample) {
   return flags;
 }
 
-// Enqueue the kernels of one step reading buffer `par` (no host sync, no
-// memsets: safe to capture in a HIP graph).
-// Workgroups of the wall pass (both launches): one wave per chunk of 64
-// bitmask words for small instances, at most 1024 workgroups (about what
-// the GPU keeps resident at the pass's occupancy); grid-stride beyond.
-uint32_t wall_grid(const InstDesc& I) {
-  const uint64_t chunks = ((uint64_t)I.cap / 64 + 2 + 63) / 64;
-  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, (chunks + 3) / 4));
+// Form and workgroups of the wall pass for n loaded particles. direct (small
+// instances only): the bitmask is read by a wave per word of 64 slots (a few
+// more than are loaded; grid-stride beyond). Else the deferred particles are
+// compacted first: one wave per chunk of 64 words, at most 1024 workgroups
+// (about what the GPU keeps resident at the pass's occupancy).
+void wall_grid(InstDesc& I, uint32_t n, bool direct) {
+  const uint64_t words = (uint64_t)I.cap / 64 + 2;
+  I.wall_direct = direct && I.cap <= kWallDirectCap ? 1u : 0u;
+  const uint64_t wg = I.wall_direct ? std::min<uint64_t>({(n + n / 8u) / 256u + 1u, (words + 3) / 4, kWallDirectWg})
+                                    : std::min<uint64_t>(1024, ((words + 63) / 64 + 3) / 4);
+  I.n_wall_wg = (uint32_t)std::max<uint64_t>(1, wg);
 }
 
+// Enqueue the kernels of one step reading buffer `par` (no host sync, no
+// memsets: safe to capture in a HIP graph).
 int enqueue_step(dsmc_solver* h, uint32_t par, uint32_t flags, hipEvent_t* ev) {
   InstDesc& I = h->h;
   hipStream_t st = h->stream;
   if (ev) HIPC(hipEventRecord(ev[0], st));
-  dsmc_launch::step_scan(h->d_desc, 1, 0, I.ncells, h->scan_scratch, st);
+  dsmc_launch::step_scan(h->d_desc, h->scan, h->scan_ts, st);
   if (ev) HIPC(hipEventRecord(ev[1], st));
-  dsmc_launch::scatter(h->d_desc, par, h->scatter_grid, st);
+  dsmc_launch::scatter(h->d_desc, par, dsmc_launch::scatter_blocks(I), nullptr, h->scan, h->scan_ts, st);
   if (ev) HIPC(hipEventRecord(ev[2], st));
   dsmc_launch::tile(I.mode, h->d_desc, par, flags, I.n_vwg, st);
   if (ev) HIPC(hipEventRecord(ev[3], st));
-  // injection beside the wall pass (a phase timer then sees only the part
-  // of the injection that outlasts the wall pass)
-  const bool overlap = I.defer_bits && I.n_face_cells;
-  auto inject = [&](hipStream_t s) {
-    dsmc_launch::inject_count(h->d_desc, std::min(I.n_streams, I.n_face_cells), s);
-    dsmc_launch::step_scan(h->d_desc, 1, 1, I.n_face_cells, h->scan_scratch, s);
-    dsmc_launch::inject_generate(h->d_desc, par ^ 1u, std::min(I.n_streams, I.n_face_cells), s);
-  };
-  if (overlap) {
-    HIPC(hipEventRecord(h->side.fork, st));
-    HIPC(hipStreamWaitEvent(h->side.s, h->side.fork, 0));
-    inject(h->side.s);
-    HIPC(hipEventRecord(h->side.join, h->side.s));
-  }
-  if (I.defer_bits) dsmc_launch::walls(h->d_desc, par ^ 1u, flags, I.n_wall_wg, st);
-  if (ev) HIPC(hipEventRecord(ev[4], st));
-  if (overlap) HIPC(hipStreamWaitEvent(st, h->side.join, 0));
-  else if (I.n_face_cells) inject(st);
+  // the injection runs in the wall pass's launch: with a body both count as
+  // walls, without one as injection
+  const uint32_t n_wall = I.defer_bits ? I.n_wall_wg : 0u;
+  if (ev && !n_wall) HIPC(hipEventRecord(ev[4], st));
+  if (!I.wall_direct) dsmc_launch::defer_list(h->d_desc, n_wall, st);
+  dsmc_launch::walls(h->d_desc, par ^ 1u, flags, dsmc_launch::wall_blocks(I), nullptr, st);
+  if (ev && n_wall) HIPC(hipEventRecord(ev[4], st));
   if (ev) HIPC(hipEventRecord(ev[5], st));
   return DSMC_OK;
 }
@@ -1670,12 +1667,16 @@ struct dsmc_batch {
   std::vector<dsmc_solver*> hs;
   std::string err;
   hipStream_t stream = nullptr;
-  SideStream side;
   hipEvent_t ev = nullptr;
   InstDesc* d_descs = nullptr;
   uint32_t* scratch = nullptr;
-  uint32_t n = 0, mode = 0, max_cells = 0, max_faces = 0, max_vwg = 0, max_inj_threads = 0, scatter_grid = 0;
-  uint32_t wall_grid = 0;
+  uint32_t n = 0, mode = 0, max_cells = 0, max_faces = 0, max_vwg = 0, list_grid = 0;
+  dsmc_launch::StepScan scan;
+  // blocks of the scatter and of the wall pass, {instance, its block} each
+  // (the wall pass's follow the scatter's), and what they were made for
+  uint2* d_map = nullptr;
+  uint32_t scatter_blocks = 0, wall_blocks = 0;
+  std::vector<uint32_t> map_of;
   bool use_graphs = true;
   std::map<uint64_t, hipGraphExec_t> graphs;
   ~dsmc_batch() {
@@ -1683,6 +1684,7 @@ struct dsmc_batch {
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
     if (d_descs) (void)hipFree(d_descs);
     if (scratch) (void)hipFree(scratch);
+    if (d_map) (void)hipFree(d_map);
     if (ev) (void)hipEventDestroy(ev);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -1702,27 +1704,55 @@ int batch_hip(dsmc_batch* b, hipError_t e, const char* what) {
 
 int enqueue_batch_step(dsmc_batch* b, uint32_t par, uint32_t flags) {
   hipStream_t st = b->stream;
-  dsmc_launch::step_scan(b->d_descs, b->n, 0, b->max_cells, b->scratch, st);
-  dsmc_launch::scatter(b->d_descs, par, b->scatter_grid, st, b->n);
+  dsmc_launch::step_scan(b->d_descs, b->scan, b->scratch, st, b->n);
+  dsmc_launch::scatter(b->d_descs, par, b->scatter_blocks, b->d_map, b->scan, b->scratch, st);
   dsmc_launch::tile(b->mode, b->d_descs, par, flags, b->max_vwg, st, b->n);
-  // injection beside the wall pass, as for one solver
-  const bool overlap = b->wall_grid && b->max_faces;
-  auto inject = [&](hipStream_t s) {
-    dsmc_launch::inject_count(b->d_descs, b->max_inj_threads, s, b->n);
-    dsmc_launch::step_scan(b->d_descs, b->n, 1, b->max_faces, b->scratch, s);
-    dsmc_launch::inject_generate(b->d_descs, par ^ 1u, b->max_inj_threads, s, b->n);
-  };
-  hipError_t e = hipSuccess;
-  if (overlap) {
-    e = hipEventRecord(b->side.fork, st);
-    if (e == hipSuccess) e = hipStreamWaitEvent(b->side.s, b->side.fork, 0);
-    if (e == hipSuccess) inject(b->side.s);
-    if (e == hipSuccess) e = hipEventRecord(b->side.join, b->side.s);
+  dsmc_launch::defer_list(b->d_descs, b->list_grid, st, b->n);
+  dsmc_launch::walls(b->d_descs, par ^ 1u, flags, b->wall_blocks, b->d_map + b->scatter_blocks, st);
+  return DSMC_OK;
+}
+
+// The members' descriptors as the batch runs them: the wall pass reads the
+// bitmasks directly only where all members together are small.
+std::vector<InstDesc> batch_descs(dsmc_batch* b) {
+  std::vector<InstDesc> d;
+  uint64_t wg = 0;
+  for (auto* h : b->hs) {
+    d.push_back(h->h);
+    if (h->h.defer_bits) wg += h->h.n_wall_wg;
   }
-  if (b->wall_grid) dsmc_launch::walls(b->d_descs, par ^ 1u, flags, b->wall_grid, st, b->n);
-  if (overlap && e == hipSuccess) e = hipStreamWaitEvent(st, b->side.join, 0);
-  else if (!overlap && b->max_faces) inject(st);
-  if (e != hipSuccess) return b->fail(DSMC_ERR_DEVICE, std::string("batch side stream: ") + hipGetErrorString(e));
+  for (uint32_t i = 0; i < b->n; ++i)
+    if (d[i].defer_bits && wg > kWallDirectWg) wall_grid(d[i], b->hs[i]->n_loaded, false);
+  return d;
+}
+
+// The block maps of the descriptors' grids; captured steps hold the old ones,
+// so they are dropped with them.
+int batch_maps(dsmc_batch* b, const std::vector<InstDesc>& descs) {
+  std::vector<uint32_t> of;
+  for (const InstDesc& d : descs) {
+    of.push_back(dsmc_launch::scatter_blocks(d));
+    of.push_back(dsmc_launch::wall_blocks(d));
+    of.push_back(d.defer_bits && !d.wall_direct ? d.n_wall_wg : 0u);
+  }
+  if (of == b->map_of) return DSMC_OK;
+  std::vector<uint2> map;
+  for (int k = 0; k < 2; ++k) {
+    for (uint32_t i = 0; i < b->n; ++i)
+      for (uint32_t q = 0; q < of[3 * i + k]; ++q) map.push_back(make_uint2(i, q));
+    (k ? b->wall_blocks : b->scatter_blocks) = (uint32_t)map.size() - (k ? b->scatter_blocks : 0u);
+  }
+  BHIP(hipStreamSynchronize(b->stream));
+  for (auto& g : b->graphs) (void)hipGraphExecDestroy(g.second);
+  b->graphs.clear();
+  if (b->d_map) (void)hipFree(b->d_map);
+  b->d_map = nullptr;
+  b->map_of.clear();
+  BHIP(hipMalloc(&b->d_map, map.size() * sizeof(uint2)));
+  BHIP(hipMemcpy(b->d_map, map.data(), map.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  b->list_grid = 0;
+  for (uint32_t i = 0; i < b->n; ++i) b->list_grid = std::max(b->list_grid, of[3 * i + 2]);
+  b->map_of = of;
   return DSMC_OK;
 }
 
@@ -1751,15 +1781,12 @@ int dsmc_batch_create(dsmc_solver* const* hs, uint32_t n, dsmc_batch** out) {
     b->max_cells = std::max(b->max_cells, h->h.ncells);
     b->max_faces = std::max(b->max_faces, h->h.n_face_cells);
     b->max_vwg = std::max(b->max_vwg, h->h.n_vwg);
-    b->max_inj_threads = std::max(b->max_inj_threads, std::min(h->h.n_streams, h->h.n_face_cells));
-    b->scatter_grid = std::max(b->scatter_grid, h->scatter_grid);
-    if (h->h.defer_bits) b->wall_grid = std::max(b->wall_grid, h->h.n_wall_wg);
   }
+  b->scan = dsmc_launch::step_scan_plan(b->max_cells, b->max_faces);
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = b->side.create();
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&b->d_descs, sizeof(InstDesc) * n);
-  if (e == hipSuccess) e = hipMalloc(&b->scratch, sizeof(uint32_t) * n * (dsmc_launch::kScanMaxTiles + 1));
+  if (e == hipSuccess) e = hipMalloc(&b->scratch, sizeof(uint32_t) * n * b->scan.words());
   if (e != hipSuccess) {
     delete b;
     return set_global_error(DSMC_ERR_DEVICE, std::string("batch allocation: ") + hipGetErrorString(e));
@@ -1792,6 +1819,8 @@ int dsmc_batch_run(dsmc_batch* b, uint32_t steps) {
   dsmc_solver* h0 = b->hs[0];
   for (auto* h : b->hs)
     if (h->par != h0->par || h->steps != h0->steps) return b->fail(DSMC_ERR_STATE, "batch members drifted apart");
+  std::vector<InstDesc> descs = batch_descs(b);
+  CHECK_RC(batch_maps(b, descs));
   // order after each member's queued work, refresh the descriptors
   for (auto* h : b->hs) {
     BHIP(hipEventRecord(b->ev, h->stream));
@@ -1800,10 +1829,8 @@ int dsmc_batch_run(dsmc_batch* b, uint32_t steps) {
   // Sampling: in PHYSICS mode each member samples while its own sampling is
   // on (sample_on in its descriptor); launches carry the sample flag when any
   // member samples. REFERENCE members share the every-Nth-step schedule.
-  std::vector<InstDesc> descs(b->n);
   bool any_sampling = false;
   for (uint32_t i = 0; i < b->n; ++i) {
-    descs[i] = b->hs[i]->h;
     descs[i].sample_on = (!b->hs[i]->physics() || b->hs[i]->sampling) ? 1u : 0u;
     any_sampling = any_sampling || b->hs[i]->sampling;
   }

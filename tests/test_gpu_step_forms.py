@@ -1,0 +1,64 @@
+"""The forms that a step takes by the size of an instance: the scan of one or
+two launches at its limits, several blocks of freestream faces, the wall pass
+from the bitmask or from the compacted list (GPU)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import cudadsmc_amd as dm
+
+from helpers import small_physics_settings
+from test_gpu_batch import make
+from test_gpu_parity import _compare_state, _mirror
+
+pytestmark = pytest.mark.gpu
+
+
+# cells: one block of 4096; not a multiple of four; the most of the one-launch scan (16 blocks, 10240 faces in three
+# blocks); two launches with an odd rest; a long thin box with more faces than cells
+@pytest.mark.parametrize("dims,n", [((16, 16, 16), 20000), ((17, 13, 19), 9000), ((64, 32, 32), 40000),
+                                    ((65, 33, 31), 40000), ((5000, 1, 1), 20000)])
+def test_step_forms_match_oracle(dims, n):
+    print(f"step forms dims={dims} n={n}", flush=True)
+    s = small_physics_settings(dims=dims, n_target=n)
+    sol = dm.Solver()
+    sol.Init(s)
+    mesh = dm.icosphere((0.07, 0.05, 0.05), 0.02, 2)
+    sol.SetModel(mesh, grid=(6, 6, 6))
+    o = _mirror(sol, mesh)
+    sol.InitSystemState((1500.0, 0.0, 0.0))
+    o.load((1500.0, 0.0, 0.0))
+    for k in range(5):
+        sol.RunBenchmarkSimulationStep(s.dt)
+        o.step(sample=False)
+        assert np.array_equal(sol.cell_start(), o.cell_start()), k
+        _compare_state(sol, o, f"step {k + 1}")
+    assert np.array_equal(sol.ntc_state(), o.ntc())
+    sol.close()
+
+
+def test_wall_forms_give_the_same_walls():
+    """Members of a batch that is large as a whole take the list, the same
+    solvers on their own the bitmask: state and wall sums agree, also where
+    the forms alternate and the host reads the sums in between."""
+    args = [(1 + i, 100000 + 1000 * i, 900.0 + 100.0 * i, 0.015 + 0.001 * i) for i in range(12)]
+    alone = [make(*a) for a in args]
+    members = [make(*a) for a in args]
+    batch = dm.Batch(members)
+    for steps in (3, 2):
+        for a, m in zip(alone, members):
+            a.DoBenchmark(steps + 1, a.settings.dt)
+        batch.run(steps)
+        for i, m in enumerate(members):
+            m.RunBenchmarkSimulationStep(m.settings.dt)  # from the bitmask, after the list
+            if i % 3 == 0:
+                m.drag()
+    for a, m in zip(alone, members):
+        p, q = a.particles(), m.particles()
+        for k in ("pos", "vel", "key"):
+            assert np.array_equal(p[k], q[k]), k
+        assert np.any(a.drag() != 0.0) and np.array_equal(a.drag(), m.drag())
+        assert np.array_equal(m.drag(), m.drag())  # a second read folds nothing twice
+        a.close()
+    batch.close()
