@@ -220,13 +220,13 @@ class Solver:
         return int(s.grid_dim[0]) * int(s.grid_dim[1]) * int(s.grid_dim[2])
 
     def cell_stats(self) -> np.ndarray:
-        arr = (CellStats * self.n_cells)()
-        self._c(lib().dsmc_get_cell_stats(self._h, arr, self.n_cells))
-        return np.frombuffer(arr, dtype=np.float64).reshape(self.n_cells, 5).copy()
+        arr = np.empty((self.n_cells, 5), np.float64)
+        self._c(lib().dsmc_get_cell_stats(self._h, arr.ctypes.data_as(C.POINTER(CellStats)), self.n_cells))
+        return arr
 
     def fields(self) -> dict:
         C_ = self.n_cells
-        out = {k: np.zeros(C_, np.float32) for k in ("n", "u", "v", "w", "T")}
+        out = {k: np.empty(C_, np.float32) for k in ("n", "u", "v", "w", "T")}
         self._c(lib().dsmc_get_fields(self._h, *[_fp(out[k]) for k in ("n", "u", "v", "w", "T")], C_))
         return out
 

@@ -57,8 +57,11 @@ void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32
 uint32_t wall_blocks(const InstDesc& I);
 void defer_list(const InstDesc* d, uint32_t grid, hipStream_t st, uint32_t n_inst = 1);
 void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, const uint2* map, hipStream_t st);
-// Folds the wall sums of the last step into wall_acc (before a host read).
-void wall_sum(const InstDesc* d, hipStream_t st);
+// For host reads: folds the wall sums of the last step into wall_acc and sums
+// the collision counters (2 * kAccSlots values, see k_totals).
+void totals(const InstDesc* d, long long* out, hipStream_t st);
+// n, u, v, w, T of the samples as float [5][ncells].
+void fields(const InstDesc* d, uint32_t mode, uint32_t ncells, double samples, double kb, float* out, hipStream_t st);
 void load_reference(const InstDesc* d, uint32_t par, uint32_t ppc, uint32_t n_threads, float sux, float suy,
                     float suz, float temp, hipStream_t st);
 void move_zero(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st);

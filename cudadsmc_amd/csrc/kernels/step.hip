@@ -1596,11 +1596,58 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __res
   }
 }
 
-// Folds the wall sums that no step has folded yet, for a host read of the
-// totals.
-__global__ void __launch_bounds__(kTileThreads) k_wall_sum(const InstDesc* __restrict__ Ip) {
+// The totals that the host reads: the wall sums that no step has folded yet
+// into wall_acc, and the sums over the workgroups' collision counters, as
+// 64-bit sums of their low and high halves (out[2 k], out[2 k + 1] of slot k:
+// exact, the host puts them together in 128 bits).
+__global__ void __launch_bounds__(kTileThreads) k_totals(const InstDesc* __restrict__ Ip, long long* out) {
+  const InstDesc& I = *Ip;
   __shared__ long long s_red[kTileThreads / 64 * 4];
-  fold_walls<kTileThreads>(*Ip, s_red);
+  __shared__ long long s_sum[kTileThreads / kAccSlots][2 * kAccSlots];
+  if (I.wall_part) fold_walls<kTileThreads>(I, s_red);
+  const uint32_t k = threadIdx.x % kAccSlots, r = threadIdx.x / kAccSlots;
+  long long lo = 0, hi = 0;
+  for (uint32_t w = r; w < I.n_vwg; w += kTileThreads / kAccSlots) {
+    const long long v = gmem(I.wg_acc)[w * kAccSlots + k];
+    lo += (long long)((unsigned long long)v & 0xFFFFFFFFull);
+    hi += v >> 32;
+  }
+  s_sum[r][2 * k] = lo;
+  s_sum[r][2 * k + 1] = hi;
+  __syncthreads();
+  if (threadIdx.x < 2 * kAccSlots) {
+    long long t = 0;
+    for (uint32_t q = 0; q < kTileThreads / kAccSlots; ++q) t += s_sum[q][threadIdx.x];
+    out[threadIdx.x] = t;
+  }
+}
+
+// Fields of the samples (ProcessAndOutputStatistics, dsmc_base.cu:104-163), one
+// lane per cell: n, u, v, w, T in double from the sums, stored as float
+// [5][ncells], so that 20 bytes per cell travel to the host and not 40.
+template <class T>
+__global__ void __launch_bounds__(256) k_fields(const InstDesc* __restrict__ Ip, double samples, double kb, float* out) {
+  const InstDesc& I = *Ip;
+  const uint32_t c = blockIdx.x * 256u + threadIdx.x, C = I.ncells;
+  if (c >= C) return;
+  const gptr<const T> S = gmem<const T>(reinterpret_cast<const T*>(I.samp));
+  const double N = S[c], sx = S[(size_t)C + c], sy = S[2 * (size_t)C + c], sz = S[3 * (size_t)C + c],
+               s2 = S[4 * (size_t)C + c];
+  const double fr = I.fluid_frac ? (double)I.fluid_frac[c] : 1.0;
+  const double vol = (double)I.cell_volume * fr;
+  const double dens = vol > 0.0 ? (double)I.fnum * N / (vol * samples) : 0.0;
+  double ux = 0.0, uy = 0.0, uz = 0.0, tt = 0.0;
+  if (N > 0.0) {
+    ux = sx / N;
+    uy = sy / N;
+    uz = sz / N;
+    tt = (double)I.mass * (s2 / N - (ux * ux + uy * uy + uz * uz)) / (3.0 * kb);
+  }
+  out[c] = (float)dens;
+  out[(size_t)C + c] = (float)ux;
+  out[2 * (size_t)C + c] = (float)uy;
+  out[3 * (size_t)C + c] = (float)uz;
+  out[4 * (size_t)C + c] = (float)tt;
 }
 
 // =================================================================== loading
@@ -1931,8 +1978,15 @@ void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, co
   if (blocks) hipLaunchKernelGGL(k_walls, dim3(blocks), dim3(kTileThreads), 0, st, d, opar, flags, map);
 }
 
-void wall_sum(const InstDesc* d, hipStream_t st) {
-  hipLaunchKernelGGL(k_wall_sum, dim3(1), dim3(kTileThreads), 0, st, d);
+void totals(const InstDesc* d, long long* out, hipStream_t st) {
+  hipLaunchKernelGGL(k_totals, dim3(1), dim3(kTileThreads), 0, st, d, out);
+}
+
+void fields(const InstDesc* d, uint32_t mode, uint32_t ncells, double samples, double kb, float* out, hipStream_t st) {
+  if (mode == kModePhysics)
+    hipLaunchKernelGGL(k_fields<double>, dim3(blocks_for(ncells, 256)), dim3(256), 0, st, d, samples, kb, out);
+  else
+    hipLaunchKernelGGL(k_fields<float>, dim3(blocks_for(ncells, 256)), dim3(256), 0, st, d, samples, kb, out);
 }
 
 void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t n_vwg, hipStream_t st,

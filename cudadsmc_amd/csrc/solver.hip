@@ -39,6 +39,26 @@ const char* global_error() { return g_err.c_str(); }
 
 using namespace dsmc_host;
 
+// Pinned buffer of host reads, two halves filled in turn: one for the process
+// (reads wait for their data anyway), held while solvers exist.
+struct Staging {
+  static constexpr size_t kHalf = 2u << 20;
+  std::mutex mu;
+  char* p = nullptr;
+  int users = 0;
+  void enter() {
+    std::lock_guard<std::mutex> lock(mu);
+    ++users;
+  }
+  void leave() {
+    std::lock_guard<std::mutex> lock(mu);
+    if (--users > 0 || !p) return;
+    (void)hipHostFree(p);
+    p = nullptr;
+  }
+};
+static Staging g_staging;
+
 struct dsmc_solver {
   std::string err;
   dsmc_settings s{};
@@ -90,6 +110,9 @@ struct dsmc_solver {
   bool timing = false;
   double t_ms[6] = {0, 0, 0, 0, 0, 0};  // summed ms: scan, scatter, tile, inject, whole step, walls
   uint64_t timed_steps = 0;
+  hipEvent_t read_ev[2] = {nullptr, nullptr};  // the halves of a host read
+  float* d_fields = nullptr;                   // fields on their way to the host
+  long long* d_totals = nullptr;               // totals, likewise
   std::vector<hipEvent_t> ev_pool;   // 5 events per timed step, resolved lazily
   size_t ev_used = 0;
   uint32_t debug_flags = 0;
@@ -130,14 +153,52 @@ struct dsmc_solver {
     free_geom();
     for (void* p : bufs) (void)hipFree(p);
     for (auto& e : ev_pool) (void)hipEventDestroy(e);
+    for (auto& e : read_ev)
+      if (e) (void)hipEventDestroy(e);
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
     if (stream) (void)hipStreamDestroy(stream);
+    g_staging.leave();
   }
+  dsmc_solver() { g_staging.enter(); }
   int upload_desc() { return hip(hipMemcpyAsync(d_desc, &h, sizeof(h), hipMemcpyHostToDevice, stream), "desc upload"); }
+  // Device memory to the host: consume(data, offset, bytes) for consecutive
+  // parts, each copied to a pinned half-buffer while the one before is
+  // consumed (a copy to pageable memory goes through the driver's own staging
+  // at a third of the rate).
+  template <class F>
+  int read_back(const void* src, size_t bytes, F consume) {
+    std::lock_guard<std::mutex> lock(g_staging.mu);
+    if (!g_staging.p) {
+      void* q = nullptr;
+      const hipError_t e = hipHostMalloc(&q, 2 * Staging::kHalf, hipHostMallocPortable);
+      if (e != hipSuccess) return hip(e, "hipHostMalloc");
+      g_staging.p = static_cast<char*>(q);
+    }
+    auto issue = [&](size_t off) {
+      const int half = (int)(off / Staging::kHalf % 2);
+      const size_t n = std::min(Staging::kHalf, bytes - off);
+      hipError_t e = hipMemcpyAsync(g_staging.p + half * Staging::kHalf, static_cast<const char*>(src) + off, n,
+                                    hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipEventRecord(read_ev[half], stream);
+      return hip(e, "read back");
+    };
+    int rc = bytes ? issue(0) : DSMC_OK;
+    for (size_t off = 0; off < bytes && rc == DSMC_OK; off += Staging::kHalf) {
+      if (off + Staging::kHalf < bytes) rc = issue(off + Staging::kHalf);
+      const int half = (int)(off / Staging::kHalf % 2);
+      const int rc2 = hip(hipEventSynchronize(read_ev[half]), "read back");
+      if (rc == DSMC_OK) rc = rc2;
+      if (rc == DSMC_OK) consume(g_staging.p + half * Staging::kHalf, off, std::min(Staging::kHalf, bytes - off));
+    }
+    if (rc != DSMC_OK) (void)hipStreamSynchronize(stream);  // no copy into the halves stays in flight
+    return rc;
+  }
+  int read_to(void* dst, const void* src, size_t bytes) {
+    return read_back(src, bytes, [&](const char* p, size_t off, size_t n) { std::memcpy((char*)dst + off, p, n); });
+  }
   uint32_t get_ctr(int i) {
     uint32_t v = 0;
-    (void)hipMemcpyAsync(&v, h.ctr + i, 4, hipMemcpyDeviceToHost, stream);
-    (void)hipStreamSynchronize(stream);
+    (void)read_to(&v, h.ctr + i, 4);
     return v;
   }
   bool physics() const { return s.mode == DSMC_MODE_PHYSICS; }
@@ -216,6 +277,8 @@ int dsmc_create(int solver_type, dsmc_solver** out) {
     return set_global_error(DSMC_ERR_DEVICE, std::string("no HIP device: ") + hipGetErrorString(e));
   auto* h = new dsmc_solver();
   e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
+  for (auto& ev : h->read_ev)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
   if (e != hipSuccess) {
     delete h;
     return set_global_error(DSMC_ERR_DEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
@@ -885,74 +948,60 @@ int dsmc_get_cell_stats(dsmc_solver* h, dsmc_cell_stats* out, uint32_t n) {
   InstDesc& I = h->h;
   if (n < I.ncells) return h->fail(DSMC_ERR_INVALID, "need %u cells", I.ncells);
   const uint32_t C = I.ncells;
-  std::vector<double> buf((size_t)5 * C);
-  HIPC(hipMemcpyAsync(buf.data(), I.samp, buf.size() * 8, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
-  const float* f = reinterpret_cast<const float*>(buf.data());
-  for (uint32_t c = 0; c < C; ++c) {
-    if (h->physics()) {
-      out[c].num_in_sample = buf[c];
-      out[c].xyz_sum[0] = buf[C + c];
-      out[c].xyz_sum[1] = buf[2 * (size_t)C + c];
-      out[c].xyz_sum[2] = buf[3 * (size_t)C + c];
-      out[c].vel_mag = buf[4 * (size_t)C + c];
-    } else {
-      out[c].num_in_sample = f[c];
-      out[c].xyz_sum[0] = f[C + c];
-      out[c].xyz_sum[1] = f[2 * (size_t)C + c];
-      out[c].xyz_sum[2] = f[3 * (size_t)C + c];
-      out[c].vel_mag = f[4 * (size_t)C + c];
+  double* const o = &out[0].num_in_sample;  // five doubles per cell, in the order of the sums
+  static_assert(sizeof(dsmc_cell_stats) == 5 * sizeof(double), "packed cell statistics");
+  auto split = [&](auto* p, size_t i0, size_t count) {
+    for (size_t q = 0; q < count;) {
+      const size_t k = (i0 + q) / C, c = (i0 + q) % C, m = std::min(count - q, C - c);
+      for (size_t e = 0; e < m; ++e) o[5 * (c + e) + k] = (double)p[q + e];
+      q += m;
     }
-  }
-  return DSMC_OK;
+  };
+  if (h->physics())
+    return h->read_back(I.samp, (size_t)5 * C * 8, [&](const char* p, size_t off, size_t nb) {
+      split(reinterpret_cast<const double*>(p), off / 8, nb / 8);
+    });
+  return h->read_back(I.samp, (size_t)5 * C * 4, [&](const char* p, size_t off, size_t nb) {
+    split(reinterpret_cast<const float*>(p), off / 4, nb / 4);
+  });
 }
 
 int dsmc_get_fields(dsmc_solver* h, float* n, float* u, float* v, float* w, float* T, uint32_t nc) {
   if (!h) return set_global_error(DSMC_ERR_INVALID, "null handle");
   InstDesc& I = h->h;
   if (nc < I.ncells) return h->fail(DSMC_ERR_INVALID, "need %u cells", I.ncells);
-  std::vector<dsmc_cell_stats> cs(I.ncells);
-  CHECK_RC(dsmc_get_cell_stats(h, cs.data(), I.ncells));
+  if (!h->inited) return h->fail(DSMC_ERR_STATE, "not initialised");
+  const size_t C = I.ncells;
+  if (!h->d_fields) CHECK_RC(h->alloc(&h->d_fields, 5 * C));
   const double S = h->samples > 0 ? (double)h->samples : 1.0;
   const double kb = h->physics() ? kBoltz : (double)kBoltzRef;
-  for (uint32_t c = 0; c < I.ncells; ++c) {
-    double N = cs[c].num_in_sample;
-    double fr = (h->physics() && !h->frac.empty()) ? h->frac[c] : 1.0;
-    double vol = (double)I.cell_volume * fr;
-    double dens = vol > 0.0 ? (double)I.fnum * N / (vol * S) : 0.0;
-    double ux = 0, uy = 0, uz = 0, tt = 0;
-    if (N > 0) {
-      ux = cs[c].xyz_sum[0] / N;
-      uy = cs[c].xyz_sum[1] / N;
-      uz = cs[c].xyz_sum[2] / N;
-      tt = (double)I.mass * (cs[c].vel_mag / N - (ux * ux + uy * uy + uz * uz)) / (3.0 * kb);
+  dsmc_launch::fields(h->d_desc, I.mode, I.ncells, S, kb, h->d_fields, h->stream);
+  HIPC(hipGetLastError());
+  float* const dst[5] = {n, u, v, w, T};
+  return h->read_back(h->d_fields, 5 * C * 4, [&](const char* p, size_t off, size_t bytes) {
+    const float* f = reinterpret_cast<const float*>(p);
+    for (size_t i = off / 4, end = (off + bytes) / 4; i < end;) {
+      const size_t k = i / C, c = i % C, m = std::min(end - i, C - c);
+      if (dst[k]) std::memcpy(dst[k] + c, f, m * 4);
+      f += m;
+      i += m;
     }
-    if (n) n[c] = (float)dens;
-    if (u) u[c] = (float)ux;
-    if (v) v[c] = (float)uy;
-    if (w) w[c] = (float)uz;
-    if (T) T[c] = (float)tt;
-  }
-  return DSMC_OK;
+  });
 }
 
 static int sum_acc(dsmc_solver* h, double out[kAccSlots]) {
   InstDesc& I = h->h;
-  if (I.wall_acc) {  // the last step's wall sums are folded by the next one, or here
-    dsmc_launch::wall_sum(h->d_desc, h->stream);
-    HIPC(hipGetLastError());
-  }
-  std::vector<long long> acc((size_t)I.n_vwg * kAccSlots);
-  HIPC(hipMemcpyAsync(acc.data(), I.wg_acc, acc.size() * 8, hipMemcpyDeviceToHost, h->stream));
+  // the collision counters' sums, then the wall totals, in one small buffer
+  constexpr size_t kWords = 2 * kAccSlots;
+  if (!h->d_totals) CHECK_RC(h->alloc(&h->d_totals, kWords));
+  dsmc_launch::totals(h->d_desc, h->d_totals, h->stream);
+  HIPC(hipGetLastError());
+  long long acc[kWords];
   double tacc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (I.wall_acc) HIPC(hipMemcpyAsync(tacc, I.wall_acc, sizeof(tacc), hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(acc, h->d_totals, sizeof(acc)));
+  if (I.wall_acc) CHECK_RC(h->read_to(tacc, I.wall_acc, sizeof(tacc)));
   // the workgroups' integer counters summed exactly (128-bit), converted once
-  for (int k = 0; k < kAccSlots; ++k) {
-    __int128 t = 0;
-    for (uint32_t w = 0; w < I.n_vwg; ++w) t += acc[(size_t)w * kAccSlots + k];
-    out[k] = (double)t;
-  }
+  for (int k = 0; k < kAccSlots; ++k) out[k] = (double)((__int128)acc[2 * k + 1] * ((__int128)1 << 32) + acc[2 * k]);
   out[kAccCr] /= kCrScale;
   // wall forces and heat of the wall pass
   for (int k = 0; k < 4; ++k) out[kAccFx + k] += tacc[k];
@@ -966,8 +1015,7 @@ int dsmc_get_collision_stats(dsmc_solver* h, double out[4]) {
   if (!h->physics()) {
     // GetStatistics (dsmc_kernel.cu:840-854): sum of the per-cell counters
     std::vector<float4> cs(I.ncells);
-    HIPC(hipMemcpyAsync(cs.data(), I.cstat, cs.size() * sizeof(float4), hipMemcpyDeviceToHost, h->stream));
-    HIPC(hipStreamSynchronize(h->stream));
+    CHECK_RC(h->read_to(cs.data(), I.cstat, cs.size() * sizeof(float4)));
     double a = 0, b = 0, c = 0;
     for (auto& x : cs) {
       a += x.x;
@@ -1139,9 +1187,7 @@ int dsmc_get_counts(dsmc_solver* h, uint64_t* steps, uint32_t* n_particles, uint
       InstDesc& I = h->h;
       uint32_t stored = h->get_ctr(0);
       std::vector<uint32_t> keys(stored);
-      if (stored)
-        HIPC(hipMemcpyAsync(keys.data(), I.key[h->par], (size_t)stored * 4, hipMemcpyDeviceToHost, h->stream));
-      HIPC(hipStreamSynchronize(h->stream));
+      CHECK_RC(h->read_to(keys.data(), I.key[h->par], (size_t)stored * 4));
       uint32_t live = 0;
       for (uint32_t k : keys) live += k != kInvalidKey;
       *n_particles = live;
@@ -1177,20 +1223,13 @@ int dsmc_get_particles(dsmc_solver* h, float* pos, float* vel, uint32_t* keys, u
   uint32_t n = h->get_ctr(0);
   if (n_out) *n_out = n;
   if (cap < n) return pos || vel || keys ? h->fail(DSMC_ERR_CAPACITY, "need room for %u particles", n) : DSMC_OK;
-  hipStream_t st = h->stream;
-  uint32_t p = h->par;
-  if (pos) {
-    HIPC(hipMemcpyAsync(pos, I.px[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-    HIPC(hipMemcpyAsync(pos + cap, I.py[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-    HIPC(hipMemcpyAsync(pos + 2 * (size_t)cap, I.pz[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
+  const uint32_t p = h->par;
+  const float* const from[6] = {I.px[p], I.py[p], I.pz[p], I.vx[p], I.vy[p], I.vz[p]};
+  for (size_t k = 0; k < 6; ++k) {
+    float* const to = k < 3 ? pos : vel;
+    if (to) CHECK_RC(h->read_to(to + (k % 3) * cap, from[k], (size_t)n * 4));
   }
-  if (vel) {
-    HIPC(hipMemcpyAsync(vel, I.vx[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-    HIPC(hipMemcpyAsync(vel + cap, I.vy[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-    HIPC(hipMemcpyAsync(vel + 2 * (size_t)cap, I.vz[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-  }
-  if (keys) HIPC(hipMemcpyAsync(keys, I.key[p], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-  HIPC(hipStreamSynchronize(st));
+  if (keys) CHECK_RC(h->read_to(keys, I.key[p], (size_t)n * 4));
   if (keys)
     for (uint32_t i = 0; i < n; ++i) keys[i] = key_cell(keys[i]);  // without the wall pass's mark
   return DSMC_OK;
@@ -1223,8 +1262,7 @@ int dsmc_get_cell_start(dsmc_solver* h, uint32_t* out, uint32_t n) {
   if (!h || !out) return set_global_error(DSMC_ERR_INVALID, "null argument");
   InstDesc& I = h->h;
   if (n < I.ncells + 1) return h->fail(DSMC_ERR_INVALID, "need %u entries", I.ncells + 1);
-  HIPC(hipMemcpyAsync(out, I.cell_start, ((size_t)I.ncells + 1) * 4, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(out, I.cell_start, ((size_t)I.ncells + 1) * 4));
   return DSMC_OK;
 }
 
@@ -1232,8 +1270,7 @@ int dsmc_get_perm(dsmc_solver* h, uint32_t* out, uint32_t n) {
   if (!h || !out) return set_global_error(DSMC_ERR_INVALID, "null argument");
   InstDesc& I = h->h;
   uint32_t m = std::min(n, I.cap);
-  HIPC(hipMemcpyAsync(out, I.perm, (size_t)m * 4, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(out, I.perm, (size_t)m * 4));
   return DSMC_OK;
 }
 
@@ -1241,8 +1278,7 @@ int dsmc_get_hit_counts(dsmc_solver* h, uint32_t* out, uint32_t n) {
   if (!h || !out) return set_global_error(DSMC_ERR_INVALID, "null argument");
   InstDesc& I = h->h;
   uint32_t m = std::min(n, I.cap);
-  HIPC(hipMemcpyAsync(out, I.hits, (size_t)m * 4, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(out, I.hits, (size_t)m * 4));
   return DSMC_OK;
 }
 
@@ -1250,8 +1286,7 @@ int dsmc_get_ntc_state(dsmc_solver* h, float* out, uint32_t n) {
   if (!h || !out) return set_global_error(DSMC_ERR_INVALID, "null argument");
   InstDesc& I = h->h;
   if (n < I.ncells) return h->fail(DSMC_ERR_INVALID, "need %u cells", I.ncells);
-  HIPC(hipMemcpyAsync(out, I.ntc, (size_t)I.ncells * 8, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(out, I.ntc, (size_t)I.ncells * 8));
   return DSMC_OK;
 }
 
@@ -1261,8 +1296,7 @@ int dsmc_get_rng_state(dsmc_solver* h, uint32_t* out, uint32_t n) {
   size_t need = (size_t)kMtWords * I.n_streams;
   if (n < need) return h->fail(DSMC_ERR_INVALID, "need %zu words", need);
   std::vector<uint32_t> tmp(need);
-  HIPC(hipMemcpyAsync(tmp.data(), I.mt_state, need * 4, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(tmp.data(), I.mt_state, need * 4));
   for (uint32_t s = 0; s < I.n_streams; ++s)
     for (uint32_t w = 0; w < kMtWords; ++w) out[(size_t)s * kMtWords + w] = tmp[(size_t)w * I.n_streams + s];
   return DSMC_OK;
@@ -1299,8 +1333,7 @@ int dsmc_get_taus_state(dsmc_solver* h, uint32_t* out, uint32_t n) {
   InstDesc& I = h->h;
   if (!I.taus) return h->fail(DSMC_ERR_STATE, "no Hybrid-Taus state (REFERENCE mode with mt = 0 only)");
   if (n < 4u * I.ncells) return h->fail(DSMC_ERR_INVALID, "need %u words", 4u * I.ncells);
-  HIPC(hipMemcpyAsync(out, I.taus, (size_t)16 * I.ncells, hipMemcpyDeviceToHost, h->stream));
-  HIPC(hipStreamSynchronize(h->stream));
+  CHECK_RC(h->read_to(out, I.taus, (size_t)16 * I.ncells));
   return DSMC_OK;
 }
 

@@ -62,3 +62,43 @@ def test_wall_forms_give_the_same_walls():
         assert np.array_equal(m.drag(), m.drag())  # a second read folds nothing twice
         a.close()
     batch.close()
+
+
+@pytest.mark.parametrize("mode", [dm.MODE_PHYSICS, dm.MODE_REFERENCE])
+def test_fields_from_the_sums(mode):
+    """Fields computed on the GPU against the same formulas on the sums, both
+    read through the staging halves (several rounds of them in PHYSICS)."""
+    if mode == dm.MODE_PHYSICS:
+        s = small_physics_settings(dims=(128, 64, 32), n_target=60000)
+        steps, kb = 3, 1.380649e-23
+    else:
+        from helpers import small_reference_settings
+
+        s = small_reference_settings(geometry=False)
+        s.sample_every = 2
+        steps, kb = 4, float(np.float32(1.3806e-23))
+    sol = dm.Solver()
+    sol.Init(s)
+    if mode == dm.MODE_PHYSICS:
+        sol.SetModel(dm.icosphere((0.07, 0.05, 0.05), 0.02, 2), grid=(6, 6, 6))
+        frac = sol.fluid_fraction().astype(np.float64)
+    else:
+        frac = 1.0
+    sol.InitSystemState(tuple(s.stream_velocity))
+    sol.set_sampling(True)
+    sol.DoBenchmark(steps, s.dt)
+    samples = sol.counts()[2]
+    N, sx, sy, sz, s2 = sol.cell_stats().T
+    d = sol.derived()
+    vol = float(d["cell_volume"]) * frac
+    safe, on = np.maximum(N, 1.0), N > 0
+    want = {"n": np.where(vol > 0, float(d["fnum"]) * N / np.where(vol > 0, vol * samples, 1.0), 0.0)}
+    u = {k: np.where(on, a / safe, 0.0) for k, a in (("u", sx), ("v", sy), ("w", sz))}
+    want.update(u)
+    T = float(np.float32(s.molmass)) * (s2 / safe - (u["u"] ** 2 + u["v"] ** 2 + u["w"] ** 2)) / (3.0 * kb)
+    want["T"] = np.where(on, T, 0.0)
+    assert samples > 0 and on.any()
+    got = sol.fields()
+    for k, w in want.items():
+        np.testing.assert_array_equal(got[k], w.astype(np.float32), err_msg=k)
+    sol.close()
