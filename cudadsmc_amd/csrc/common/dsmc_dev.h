@@ -30,6 +30,9 @@ __host__ __device__ inline uint32_t key_cell(uint32_t k) { return k >= kDeferred
 constexpr uint32_t kTileCells = 256;    // most cells per tile (one lane per cell)
 constexpr uint32_t kTileThreads = 256;  // threads of the tile kernel
 constexpr uint32_t kLdsCap = 2048;      // particles staged in LDS per tile
+// Narrow tiles (one wave each): most cells, particles staged in LDS, and
+// tiles that a wave takes in one launch.
+constexpr uint32_t kNarrowCells = 64, kNarrowCap = 496, kNarrowWalk = 4;
 constexpr uint32_t kMaxCap = 1u << 30;   // particles per instance: 4-byte arrays stay below 4 GiB
 constexpr uint32_t kMtWords = 20;       // 19 window words + 1 spare (zero)
 constexpr uint32_t kRefMtStreams = 65536;  // the reference's MT_RNG_COUNT (MersenneTwister.h:31)
@@ -157,7 +160,7 @@ struct InstDesc {
   double wall_unit[2];  // value of one fixed-point unit: m v_ref / 2^36 (momentum), m v_ref^2 / 2^34 (energy)
   double* wall_acc;     // PHYSICS with a body: wall {Fx, Fy, Fz, heat} sums over the steps [4]
   uint32_t wall_key[2]; // Philox key of the wall re-emission draws
-  long long* wg_acc;    // [n_vwg][kAccSlots] collision counters per workgroup (integers, see CollAcc)
+  long long* wg_acc;    // [workgroups][kAccSlots] collision counters per workgroup (integers, see CollAcc)
   uint32_t* hits;       // per sorted particle wall hits (debug, may be null)
   // ---- RNG
   uint32_t* taus;       // REFERENCE with mt = 0: Hybrid-Taus state per cell, 4 words (else null)
@@ -166,10 +169,13 @@ struct InstDesc {
   const uint32_t* mt_b;
   const uint32_t* mt_c;
   uint32_t n_streams;
-  uint32_t n_vwg;       // virtual workgroups of the tile kernel = n_streams / 256
+  uint32_t n_vwg;       // virtual workgroups of the tile kernel = n_streams / 256 (n_tile_wg of wide tiles)
   // ---- injection face cells
   uint32_t n_face_cells;
   uint32_t* face_count; // [n_face_cells + 1] counts then offsets
+  // ---- tile kernel's launch
+  uint32_t tile_narrow;   // small tiles of few particles: a wave takes a tile (else a workgroup)
+  uint32_t n_tile_wg;     // workgroups of the tile kernel
 };
 
 // Global-memory view of a pointer held in a descriptor. Pointers loaded from

@@ -48,8 +48,10 @@ void scatter(const InstDesc* d, uint32_t par, uint32_t blocks, const uint2* map,
 uint64_t op_sort_work_words(uint32_t n, uint32_t n_cells);
 int op_sort(const uint32_t* keys, uint32_t n, uint32_t n_cells, uint32_t* perm, uint32_t* cell_start,
             uint32_t* work, hipStream_t st);
-void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t n_vwg, hipStream_t st,
-          uint32_t n_inst = 1);
+// The tile kernel of instances with (narrow) or without tile_narrow: blocks =
+// the sum of their n_tile_wg, map as for the scatter.
+void tile(uint32_t mode, bool narrow, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t blocks,
+          const uint2* map, hipStream_t st);
 // PHYSICS: the wall pass over the particles the tile kernel deferred (opar =
 // the buffer it wrote) and the inflow; blocks and map as for the scatter.
 // Before it, instances that are not wall_direct compact the deferred
@@ -59,7 +61,7 @@ void defer_list(const InstDesc* d, uint32_t grid, hipStream_t st, uint32_t n_ins
 void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, const uint2* map, hipStream_t st);
 // For host reads: folds the wall sums of the last step into wall_acc and sums
 // the collision counters (2 * kAccSlots values, see k_totals).
-void totals(const InstDesc* d, long long* out, hipStream_t st);
+void totals(const InstDesc* d, uint32_t n_acc, long long* out, hipStream_t st);
 // n, u, v, w, T of the samples as float [5][ncells].
 void fields(const InstDesc* d, uint32_t mode, uint32_t ncells, double samples, double kb, float* out, hipStream_t st);
 void load_reference(const InstDesc* d, uint32_t par, uint32_t ppc, uint32_t n_threads, float sux, float suy,

@@ -780,18 +780,54 @@ using dsmc_launch::kFlagSample;
 using dsmc_launch::kFlagKeepPerm;
 using dsmc_launch::kFlagHits;
 
-constexpr uint32_t kMoveBatch = 6;  // rounds of 256 positions whose loads are issued together
-// PHYSICS: rounds of 256 permutation entries of the next tile loaded into
-// registers during this tile's move (the next tile's first phase then only
-// stores them to LDS)
-constexpr uint32_t kPermPrefetch = 6;
+// A tile is worked by NT threads: a workgroup (wide), or one wave of it
+// (narrow: tiles of few particles, see k_tile).
+template <uint32_t NT>
+struct TileShape {
+  static constexpr bool kWide = NT == kTileThreads;
+  static constexpr uint32_t kCells = kWide ? kTileCells : kNarrowCells;
+  static constexpr uint32_t kCap = kWide ? kLdsCap : kNarrowCap;  // particles staged in LDS
+  static constexpr uint32_t kMoveBatch = kWide ? 6 : 4;  // rounds of NT positions whose loads are issued together
+  // PHYSICS: rounds of NT permutation entries of the next tile loaded into
+  // registers during this tile's move (the next tile's first phase then only
+  // stores them to LDS)
+  static constexpr uint32_t kPermPrefetch = kWide ? 6 : 4;
+};
+
+// Pops a tile from a queue. The address comes from a vector register that the
+// compiler cannot see through: an atomic that it knows to be uniform it makes
+// for the whole wave, with a wait for the result right behind it (the wide
+// kernel was 1.4 % slower at 33.5 million particles).
+__device__ __forceinline__ uint32_t queue_pop(gptr<uint32_t> queue) {
+  uint32_t at = 0u;
+  asm volatile("" : "+v"(at));
+  return gatomic_add(gelem(queue, at), 1u);
+}
+
+// Thread of the tile.
+template <uint32_t NT>
+__device__ __forceinline__ uint32_t tile_tid() {
+  return TileShape<NT>::kWide ? threadIdx.x : lane_id();
+}
+
+// Between the phases of a tile: a wave's own LDS and memory operations are in
+// order, only the compiler has to keep them so.
+template <uint32_t NT>
+__device__ __forceinline__ void tile_sync() {
+  if (TileShape<NT>::kWide) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
 
 // LDS of the PHYSICS NTC rounds.
 struct NtcLds {
-  uint32_t* off;   // [kTileCells] each cell's first item of the round
-  uint32_t* nmax;  // [kTileCells] (sigma c_r)max at the round's start (float bits)
-  uint32_t* rmax;  // [kTileCells] largest sigma c_r seen so far (float bits)
-  uint8_t* icell;  // [kTileThreads] cell of each of the round's first kTileThreads items
+  uint32_t* off;   // [cells] each cell's first item of the round
+  uint32_t* nmax;  // [cells] (sigma c_r)max at the round's start (float bits)
+  uint32_t* rmax;  // [cells] largest sigma c_r seen so far (float bits)
+  uint8_t* icell;  // [NT] cell of each of the round's first NT items
   uint32_t* red;   // [8] wave totals of the scan, then the waves' largest round counts
 };
 
@@ -804,12 +840,13 @@ struct NtcLds {
 // (sigma c_r)max and collided independently; the maximum then takes the
 // round's largest sigma c_r. Draws: Philox4x32-10 under key
 // (seed, kNtcKey1) at counter (cell, step, round, item).
+template <uint32_t NT>
 __device__ __forceinline__ void tile_ntc_rounds(const InstDesc& I, uint32_t c0, uint32_t nc, uint32_t p0,
                                                 const uint32_t* s_start, float* vx, float* vy, float* vz,
                                                 float2& nt, float frac, uint32_t stepno, const NtcLds& L,
                                                 CollAcc& acc) {
   using namespace dsmc_pairing;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / 64u;
+  const uint32_t tid = tile_tid<NT>(), lane = lane_id(), wid = tid / 64u;
   uint32_t n = 0u, M = 0u;
   if (tid < nc) {
     n = s_start[tid + 1] - s_start[tid];
@@ -844,10 +881,10 @@ __device__ __forceinline__ void tile_ntc_rounds(const InstDesc& I, uint32_t c0, 
     }
     if (lane == 63) L.red[wid] = x;
     if (r == 0u && lane == 0) L.red[4 + wid] = R;
-    __syncthreads();
+    tile_sync<NT>();
     uint32_t base = 0u, total = 0u;
 #pragma unroll
-    for (uint32_t w = 0; w < kTileThreads / 64; ++w) {
+    for (uint32_t w = 0; w < NT / 64; ++w) {
       const uint32_t t = L.red[w];
       base += w < wid ? t : 0u;
       total += t;
@@ -857,12 +894,12 @@ __device__ __forceinline__ void tile_ntc_rounds(const InstDesc& I, uint32_t c0, 
     const uint32_t off = base + x - m;
     if (tid < nc) {
       L.off[tid] = off;
-      for (uint32_t q = off; q < off + m && q < kTileThreads; ++q) L.icell[q] = (uint8_t)tid;
+      for (uint32_t q = off; q < off + m && q < NT; ++q) L.icell[q] = (uint8_t)tid;
     }
-    __syncthreads();
-    for (uint32_t it = tid; it < total; it += kTileThreads) {
+    tile_sync<NT>();
+    for (uint32_t it = tid; it < total; it += NT) {
       uint32_t c;
-      if (it < kTileThreads) {
+      if (it < NT) {
         c = L.icell[it];
       } else {  // the last cell whose first item is at or before it
         uint32_t lo = 0u, hi = nc - 1u;
@@ -895,23 +932,25 @@ __device__ __forceinline__ void tile_ntc_rounds(const InstDesc& I, uint32_t c0, 
         scatter_uv(vx, vy, vz, i, j, mag, dsmc_rng::px_unit(d.v[1]), dsmc_rng::px_unit(d.v[2]));
       }
     }
-    __syncthreads();
+    tile_sync<NT>();
     if (tid < nc) L.nmax[tid] = L.rmax[tid];
   }
   if (tid < nc) nt.x = __uint_as_float(L.rmax[tid]);
 }
 
-template <uint32_t MODE, bool LDS>
+template <uint32_t MODE, bool LDS, uint32_t NT>
 __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint32_t flags, uint32_t tile,
                                           uint32_t c0, uint32_t nc, uint32_t p0, uint32_t np,
                                           const uint32_t* s_start, const uint8_t* s_nearc, uint32_t& tile_n,
                                           gptr<uint32_t> queue, uint32_t qx, bool per_xcd, uint32_t e_static,
                                           uint32_t* s_pop,
-                                          uint32_t* sn_start, uint8_t* sn_nearc, uint32_t (&pf)[kPermPrefetch],
+                                          uint32_t* sn_start, uint8_t* sn_nearc, uint32_t (&pf)[TileShape<NT>::kPermPrefetch],
                                           uint32_t* s_raw,
                                           uint32_t* s_perm, uint8_t* s_owner, float* s_vx, float* s_vy,
                                           float* s_vz, uint32_t stepno, const NtcLds& ntl, CollAcc& cacc) {
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = tile_tid<NT>();
+  constexpr uint32_t kBatch = TileShape<NT>::kMoveBatch, kPf = TileShape<NT>::kPermPrefetch;
+  constexpr uint32_t kCap = TileShape<NT>::kCap;
   const uint32_t opar = par ^ 1u;
   const gptr<const float> ipx = gmem<const float>(I.px[par]);
   const gptr<const float> ipy = gmem<const float>(I.py[par]);
@@ -938,25 +977,25 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
   // next element of its fixed sequence
   const bool dyn = I.tile_dyn != 0u;
   uint32_t popped = 0u;
-  if (dyn && tid == 0) popped = gatomic_add(queue, 1u);
+  if (dyn && tid == 0) popped = queue_pop(queue);
   // (1) raw permutation of the tile and the owning cell of each position
   if (LDS) {
     if (MODE == kModePhysics) {
 #pragma unroll
-      for (uint32_t k = 0; k < kPermPrefetch; ++k)
-        if (tid + k * kTileThreads < np) raw[tid + k * kTileThreads] = pf[k];
-      for (uint32_t q = tid + kPermPrefetch * kTileThreads; q < np; q += kTileThreads) raw[q] = *gelem(gmem(I.perm), p0 + q);
+      for (uint32_t k = 0; k < kPf; ++k)
+        if (tid + k * NT < np) raw[tid + k * NT] = pf[k];
+      for (uint32_t q = tid + kPf * NT; q < np; q += NT) raw[q] = *gelem(gmem(I.perm), p0 + q);
     } else {
-      for (uint32_t q = tid; q < np; q += kTileThreads) raw[q] = *gelem(gmem(I.perm), p0 + q);
+      for (uint32_t q = tid; q < np; q += NT) raw[q] = *gelem(gmem(I.perm), p0 + q);
     }
   }
   if (tid < nc) {
     uint32_t a = s_start[tid] - p0, b = s_start[tid + 1] - p0;
     for (uint32_t q = a; q < b; ++q) own[q] = (uint8_t)tid;
   }
-  __syncthreads();
+  tile_sync<NT>();
   // (2) rank of each entry among its cell's entries -> stable order
-  for (uint32_t q = tid; q < np; q += kTileThreads) {
+  for (uint32_t q = tid; q < np; q += NT) {
     uint32_t c = own[q];
     uint32_t a = s_start[c] - p0, b = s_start[c + 1] - p0;
     uint32_t v = raw[q];
@@ -973,7 +1012,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     srt[a + r0 + r1 + r2 + r3] = v;
   }
   if (dyn && tid == 0) *s_pop = popped;
-  __syncthreads();
+  tile_sync<NT>();
   {
     const uint32_t jn = tile_queue_pos(dyn ? *s_pop : e_static, qx, per_xcd);
     tile_n = jn < I.ntiles ? (I.tile_order ? gmem(I.tile_order)[jn] : jn) : kInvalidKey;
@@ -992,13 +1031,13 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     }
   };
   if (tid >= np) load_cell_state();
-  // (3) gather velocities in sorted order; the loads of kMoveBatch positions
+  // (3) gather velocities in sorted order; the loads of kBatch positions
   // are issued before any store so that their latencies overlap
-  for (uint32_t q0 = tid; q0 < np; q0 += kMoveBatch * kTileThreads) {
-    float gx[kMoveBatch], gy[kMoveBatch], gz[kMoveBatch];
+  for (uint32_t q0 = tid; q0 < np; q0 += kBatch * NT) {
+    float gx[kBatch], gy[kBatch], gz[kBatch];
 #pragma unroll
-    for (uint32_t k = 0; k < kMoveBatch; ++k) {
-      const uint32_t q = q0 + k * kTileThreads;
+    for (uint32_t k = 0; k < kBatch; ++k) {
+      const uint32_t q = q0 + k * NT;
       gx[k] = gy[k] = gz[k] = 0.0f;
       if (q < np) {
         const uint32_t src = srt[q];
@@ -1009,8 +1048,8 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     }
     if (q0 == tid) load_cell_state();
 #pragma unroll
-    for (uint32_t k = 0; k < kMoveBatch; ++k) {
-      const uint32_t q = q0 + k * kTileThreads;
+    for (uint32_t k = 0; k < kBatch; ++k) {
+      const uint32_t q = q0 + k * NT;
       if (q < np) {
         vx[q] = gx[k];
         vy[q] = gy[k];
@@ -1018,7 +1057,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
       }
     }
   }
-  __syncthreads();
+  tile_sync<NT>();
   // Every load issued so far has arrived (the velocity gather waited for
   // them); saying so here keeps the compiler from waiting for the next
   // tile's loads below at the first use of an older one in the NTC phase.
@@ -1067,7 +1106,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     // the NTC's clamp of it right after its load, whose wait then comes
     // before the velocity gather instead of after it
     asm volatile("" : "+v"(frac_pf));
-    tile_ntc_rounds(I, c0, nc, p0, s_start, vx, vy, vz, ntc_state, frac_pf, stepno, ntl, cacc);
+    tile_ntc_rounds<NT>(I, c0, nc, p0, s_start, vx, vy, vz, ntc_state, frac_pf, stepno, ntl, cacc);
   }
   if (tile_n != kInvalidKey) {
     sn_start[tid] = nx_start;
@@ -1081,7 +1120,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
   // with the offsets that share this LDS)
   ntl.off[tid] = 0u;
   if (tid == 0) gmem(I.tile_p0)[tile] = p0;
-  __syncthreads();
+  tile_sync<NT>();
   // the next tile's first permutation entries (its offsets are in LDS now),
   // requested with the first batch of position gathers and waited for with
   // them, so that no later wait (the next tile's first use of pf comes after
@@ -1091,27 +1130,27 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
       const uint32_t p0n = sn_start[0];
       const uint32_t npn = sn_start[ncn] - p0n;
 #pragma unroll
-      for (uint32_t k = 0; k < kPermPrefetch; ++k) {
-        const uint32_t q = tid + k * kTileThreads;
-        pf[k] = (npn <= kLdsCap && q < npn) ? *gelem(gmem(I.perm), p0n + q) : 0u;
+      for (uint32_t k = 0; k < kPf; ++k) {
+        const uint32_t q = tid + k * NT;
+        pf[k] = (npn <= kCap && q < npn) ? *gelem(gmem(I.perm), p0n + q) : 0u;
       }
     }
   };
   // (5) move, walls, box faces, next key; rounds keep waves converged for
   // the aggregated counting
-  const uint32_t rounds = (np + kTileThreads - 1u) / kTileThreads;
+  const uint32_t rounds = (np + NT - 1u) / NT;
   if (rounds == 0u) {
     load_pf();
     wait_vmem();
   }
-  for (uint32_t r0 = 0; r0 < rounds; r0 += kMoveBatch) {
+  for (uint32_t r0 = 0; r0 < rounds; r0 += kBatch) {
     if (r0 == 0u) load_pf();
-    // positions of up to kMoveBatch rounds in flight before the first store
-    float bx[kMoveBatch], by[kMoveBatch], bz[kMoveBatch];
-    uint32_t bsrc[kMoveBatch];
+    // positions of up to kBatch rounds in flight before the first store
+    float bx[kBatch], by[kBatch], bz[kBatch];
+    uint32_t bsrc[kBatch];
 #pragma unroll
-    for (uint32_t k = 0; k < kMoveBatch; ++k) {
-      const uint32_t q = (r0 + k) * kTileThreads + tid;
+    for (uint32_t k = 0; k < kBatch; ++k) {
+      const uint32_t q = (r0 + k) * NT + tid;
       bsrc[k] = 0u;
       bx[k] = by[k] = bz[k] = 0.0f;
       if (q < np) {
@@ -1124,9 +1163,9 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     }
     wait_vmem();
 #pragma unroll
-    for (uint32_t k = 0; k < kMoveBatch; ++k) {
+    for (uint32_t k = 0; k < kBatch; ++k) {
     if (r0 + k >= rounds) break;  // uniform over the workgroup
-    uint32_t q = (r0 + k) * kTileThreads + tid;
+    uint32_t q = (r0 + k) * NT + tid;
     uint32_t key = kInvalidKey;
     // REFERENCE: the wall flights of the wavefront run together (every lane
     // takes part, with or without a particle)
@@ -1176,7 +1215,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
       // mark the wave's deferred slots in the bitmask the wall pass reads
       const uint64_t m = __ballot(key == kDeferredKey);
       if (m && lane_id() == 0) {
-        const uint32_t s0 = p0 + (r0 + k) * kTileThreads + (tid & ~63u);
+        const uint32_t s0 = p0 + (r0 + k) * NT + (tid & ~63u);
         const uint32_t sh = s0 & 63u;
         const gptr<unsigned long long> wb = gmem(I.defer_bits) + s0 / 64u;
         __hip_atomic_fetch_or(wb, (unsigned long long)(m << sh), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1190,7 +1229,7 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
 
   // (6) sampling of the post-move velocities, one lane per cell
   if ((flags & kFlagSample) && I.sample_on) {
-    __syncthreads();
+    tile_sync<NT>();
     if (tid < nc) {
       uint32_t c = c0 + tid;
       uint32_t a = s_start[tid] - p0, b = s_start[tid + 1] - p0;
@@ -1228,73 +1267,46 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
   }
 }
 
-template <uint32_t MODE>
-__global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __restrict__ Ip, uint32_t par, uint32_t flags) {
-  const InstDesc& I = Ip[blockIdx.y];
-  if (blockIdx.x >= I.n_vwg) return;  // batched launches size the grid for the largest instance
-  // cell offsets and near flags of the current tile and of the next one
-  __shared__ uint32_t s_start[2][kTileCells + 1];
-  __shared__ uint8_t s_nearc[2][kTileCells];
-  __shared__ uint32_t s_raw[kLdsCap];
-  __shared__ uint32_t s_perm[kLdsCap];
-  __shared__ uint8_t s_owner[kLdsCap];
-  __shared__ float s_vx[kLdsCap];
-  __shared__ float s_vy[kLdsCap];
-  __shared__ double s_red[kTileThreads / 64][kAccSlots];
-  // PHYSICS NTC rounds (the item-cell table shares s_red, used only at the end)
-  __shared__ uint32_t s_ntc_off[kTileCells];
-  __shared__ uint32_t s_ntc_nmax[kTileCells];
-  __shared__ uint32_t s_ntc_rmax[kTileCells];
-  __shared__ uint32_t s_ntc_red[8];
-  static_assert(sizeof(s_red) >= kTileThreads, "item-cell table must fit in s_red");
-  const NtcLds ntl = {s_ntc_off, s_ntc_nmax, s_ntc_rmax, reinterpret_cast<uint8_t*>(&s_red[0][0]), s_ntc_red};
-  // The raw permutation is dead once the rank sort has run (phase 2), so
-  // the z velocities reuse its space: 35 KB of LDS, four workgroups per CU.
-  float* const s_vz = reinterpret_cast<float*>(s_raw);
+// LDS of one tile. The raw permutation is dead once the rank sort has run
+// (phase 2), so the z velocities reuse its space.
+struct TileLds {
+  static constexpr uint32_t kStart = kTileCells + 4;
+  uint32_t* start;  // [cells + 1] cell offsets of the current tile, and kStart further of the next one
+  uint8_t* near;    // [cells] PHYSICS: near flags, likewise (kTileCells further)
+  uint32_t* raw;    // [kCap] and so are the others
+  uint32_t* perm;
+  uint8_t* owner;
+  float* vx;
+  float* vy;
+  NtcLds ntc;
+};
 
-  const uint32_t tid = threadIdx.x;
-  const uint32_t vw = blockIdx.x;
-  const uint32_t stepno = gmem(I.ctr)[4];  // this step's number (counter of the PHYSICS draws)
-  if (vw == 0 && tid == 0) {
-    I.ctr[0] = I.ctr[1];
-    I.tile_p0[I.ntiles] = I.ctr[1];  // the slots this launch stores in tile order
-  }
-  // tiles come from the XCD's queue (dynamic schedule) or, for instances
-  // whose tiles are small, as the fixed sequence of elements vw / 8,
-  // vw / 8 + G / 8, ... of that queue (no atomic per tile)
-  __shared__ uint32_t s_pop;
-  const bool per_xcd = I.n_vwg % 8u == 0u;
-  const uint32_t qx = per_xcd ? vw % 8u : 0u;
-  const uint32_t e_stride = per_xcd ? I.n_vwg / 8u : I.n_vwg;
-  const gptr<uint32_t> queue = gmem(I.ctr) + kTileQueueCtr + qx;
-  uint32_t e = per_xcd ? vw / 8u : vw;
-  if (I.tile_dyn) {
-    if (tid == 0) s_pop = gatomic_add(queue, 1u);
-    __syncthreads();
-    e = s_pop;
-  }
-  const uint32_t j = tile_queue_pos(e, qx, per_xcd);
-  if (j >= I.ntiles) return;  // no tile: this workgroup's counters stay as they are
-  CollAcc cacc = {0ull, 0ull, 0ll};
-  uint32_t tile = kInvalidKey;
+// Walk over tiles: `tile` first, then the positions that tile_body finds next
+// (queue, or e_stride further along the fixed sequence; single: none).
+template <uint32_t MODE, uint32_t NT>
+__device__ __forceinline__ void tile_walk(const InstDesc& I, uint32_t par, uint32_t flags, uint32_t tile, uint32_t e,
+                                          uint32_t e_stride, uint32_t qx, bool per_xcd, gptr<uint32_t> queue,
+                                          uint32_t* s_pop, uint32_t stepno, const TileLds& L, CollAcc& cacc,
+                                          uint32_t* over) {
+  using S = TileShape<NT>;
+  const uint32_t tid = tile_tid<NT>();
+  float* const vz = reinterpret_cast<float*>(L.raw);
   {
-    tile = I.tile_order ? gmem(I.tile_order)[j] : j;
     const uint32_t c0 = tile * I.tile_cells;
     const uint32_t nc = min(I.tile_cells, I.ncells - c0);
-    s_start[0][tid] = gmem(I.cell_start)[c0 + min(tid, nc)];
-    if (tid == 0) s_start[0][nc] = gmem(I.cell_start)[c0 + nc];
-    if (MODE == kModePhysics)
-      s_nearc[0][tid] = (I.near_cell && tid < nc) ? gmem(I.near_cell)[c0 + tid] : (uint8_t)255;
+    L.start[tid] = gmem(I.cell_start)[c0 + min(tid, nc)];
+    if (tid == 0) L.start[nc] = gmem(I.cell_start)[c0 + nc];
+    if (MODE == kModePhysics) L.near[tid] = (I.near_cell && tid < nc) ? gmem(I.near_cell)[c0 + tid] : (uint8_t)255;
   }
-  __syncthreads();
-  uint32_t pf[kPermPrefetch];
-  if (MODE == kModePhysics && tile != kInvalidKey) {
+  tile_sync<NT>();
+  uint32_t pf[S::kPermPrefetch];
+  if (MODE == kModePhysics) {
     const uint32_t nc = min(I.tile_cells, I.ncells - tile * I.tile_cells);
-    const uint32_t p0 = s_start[0][0], np = s_start[0][nc] - p0;
+    const uint32_t p0 = L.start[0], np = L.start[nc] - p0;
 #pragma unroll
-    for (uint32_t k = 0; k < kPermPrefetch; ++k) {
-      const uint32_t q = tid + k * kTileThreads;
-      pf[k] = (np <= kLdsCap && q < np) ? *gelem(gmem(I.perm), p0 + q) : 0u;
+    for (uint32_t k = 0; k < S::kPermPrefetch; ++k) {
+      const uint32_t q = tid + k * NT;
+      pf[k] = (np <= S::kCap && q < np) ? *gelem(gmem(I.perm), p0 + q) : 0u;
     }
   }
   wait_vmem();  // the first tile needs them now; later tiles find theirs arrived
@@ -1303,42 +1315,141 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __rest
     e += e_stride;                  // the next element of the fixed sequence
     const uint32_t c0 = tile * I.tile_cells;
     const uint32_t nc = min(I.tile_cells, I.ncells - c0);
-    const uint32_t p0 = s_start[b][0];
-    const uint32_t np = s_start[b][nc] - p0;
-    if (np <= kLdsCap)
-      tile_body<MODE, true>(I, par, flags, tile, c0, nc, p0, np, s_start[b], s_nearc[b], tile_n, queue, qx,
-                            per_xcd, e, &s_pop, s_start[b ^ 1u],
-                            s_nearc[b ^ 1u], pf, s_raw, s_perm, s_owner, s_vx, s_vy, s_vz, stepno, ntl, cacc);
+    uint32_t *const start = L.start + b * L.kStart, *const start_n = L.start + (b ^ 1u) * L.kStart;
+    uint8_t *const near = L.near + b * kTileCells, *const near_n = L.near + (b ^ 1u) * kTileCells;
+    const uint32_t p0 = start[0], np = start[nc] - p0;
+    // a narrow tile above its capacity is left to the whole workgroup: the
+    // wave takes it as empty and only finds the next one
+    const bool fits = np <= S::kCap;
+    if (!S::kWide && !fits && tid == 0) over[atomicAdd(over, 1u) + 1u] = tile;
+    if (fits || !S::kWide)
+      tile_body<MODE, true, NT>(I, par, flags, tile, c0, fits ? nc : 0u, p0, fits ? np : 0u, start, near, tile_n,
+                                queue, qx, per_xcd, e, s_pop, start_n, near_n, pf, L.raw, L.perm, L.owner, L.vx, L.vy, vz, stepno, L.ntc, cacc);
     else
-      tile_body<MODE, false>(I, par, flags, tile, c0, nc, p0, np, s_start[b], s_nearc[b], tile_n, queue, qx,
-                            per_xcd, e, &s_pop, s_start[b ^ 1u],
-                             s_nearc[b ^ 1u], pf, s_raw, s_perm, s_owner, s_vx, s_vy, s_vz, stepno, ntl, cacc);
-    __syncthreads();
-    if (I.tile_dyn && tid < nc) gmem(I.local_cnt)[c0 + tid] = s_ntc_off[tid];
+      tile_body<MODE, false, NT>(I, par, flags, tile, c0, nc, p0, np, start, near, tile_n, queue, qx,
+                                 per_xcd, e, s_pop, start_n, near_n, pf, L.raw, L.perm, L.owner, L.vx,
+                                 L.vy, vz, stepno, L.ntc, cacc);
+    tile_sync<NT>();
+    if (I.tile_dyn && tid < nc) gmem(I.local_cnt)[c0 + tid] = L.ntc.off[tid];
     tile = tile_n;
+  }
+}
+
+// A workgroup takes one tile after the other; where tiles hold few particles
+// (NARROW, instances with tile_narrow), each of its waves takes its own:
+// the phases of such a tile are too short to feed 256 threads, and what bounds
+// it is the latency of its chain of loads, of which four times as many are in
+// flight this way, without a barrier between the phases. Tiles that turn out
+// too full for a wave's LDS are done by the workgroup at the end.
+template <uint32_t MODE, bool NARROW>
+__global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __restrict__ Ip, uint32_t par, uint32_t flags,
+                                                      const uint2* map) {
+  const uint2 blk = block_of(map);
+  const InstDesc& I = Ip[blk.x];
+  // 40.7 KB, four workgroups per CU. Arrays of their own, so that the compiler
+  // can tell them apart (one struct of them: 1.5 % slower); a wave's share
+  // where tiles are narrow.
+  __shared__ uint32_t s_start[2 * TileLds::kStart];
+  __shared__ uint8_t s_nearc[2 * kTileCells];
+  __shared__ uint32_t s_raw[kLdsCap];
+  __shared__ uint32_t s_perm[kLdsCap];
+  __shared__ uint8_t s_owner[kLdsCap];
+  __shared__ float s_vx[kLdsCap];
+  __shared__ float s_vy[kLdsCap];
+  __shared__ uint32_t s_ntc_off[kTileCells];
+  __shared__ uint32_t s_ntc_nmax[kTileCells];
+  __shared__ uint32_t s_ntc_rmax[kTileCells];
+  __shared__ uint32_t s_ntc_red[NARROW ? 8 * (kTileThreads / 64) : 8];
+  // the NTC rounds' item-cell table, and the counters' sums at the end
+  __shared__ long long s_red[kTileThreads / 8];
+  static_assert(4u * kNarrowCap <= kLdsCap && 4u * kNarrowCells <= kTileCells && 4u * (kNarrowCells + 1u) <= TileLds::kStart,
+                "four narrow tiles share a wide tile's LDS");
+  const auto lds_of = [&](uint32_t cells, uint32_t cap, uint32_t k) {  // the k-th of tiles of this size
+    TileLds L;
+    L.start = s_start + k * (cells + 1u);
+    L.near = s_nearc + k * cells;
+    L.raw = s_raw + k * cap;
+    L.perm = s_perm + k * cap;
+    L.owner = s_owner + k * cap;
+    L.vx = s_vx + k * cap;
+    L.vy = s_vy + k * cap;
+    L.ntc.off = s_ntc_off + k * cells;
+    L.ntc.nmax = s_ntc_nmax + k * cells;
+    L.ntc.rmax = s_ntc_rmax + k * cells;
+    L.ntc.icell = reinterpret_cast<uint8_t*>(s_red) + k * cells;
+    L.ntc.red = s_ntc_red + k * 8u;
+    return L;
+  };
+  __shared__ uint32_t s_pop;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t vw = blk.y;
+  const uint32_t stepno = gmem(I.ctr)[4];  // this step's number (counter of the PHYSICS draws)
+  if (vw == 0 && tid == 0) {
+    I.ctr[0] = I.ctr[1];
+    I.tile_p0[I.ntiles] = I.ctr[1];  // the slots this launch stores in tile order
+  }
+  // tiles come from the XCD's queue (dynamic schedule) or, for instances
+  // whose tiles are small, as the fixed sequence of elements vw / 8,
+  // vw / 8 + G / 8, ... of that queue (no atomic per tile); narrow: with a
+  // walker per wave
+  const bool per_xcd = I.n_tile_wg % 8u == 0u;
+  const uint32_t qx = per_xcd ? vw % 8u : 0u;
+  const uint32_t wgs = per_xcd ? I.n_tile_wg / 8u : I.n_tile_wg;
+  const gptr<uint32_t> queue = gmem(I.ctr) + kTileQueueCtr + qx;
+  uint32_t e = per_xcd ? vw / 8u : vw;
+  CollAcc cacc = {0ull, 0ull, 0ll};
+  auto tile_at = [&](uint32_t el) {
+    const uint32_t j = tile_queue_pos(el, qx, per_xcd);
+    return j >= I.ntiles ? kInvalidKey : I.tile_order ? gmem(I.tile_order)[j] : j;
+  };
+  if constexpr (NARROW) {
+    constexpr uint32_t kW = kTileThreads / 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64u);
+    __shared__ uint32_t s_over[kNarrowWalk * kW + 1u];  // count, tiles
+    if (tid == 0) s_over[0] = 0u;
+    __syncthreads();
+    e = e * kW + wave;
+    const uint32_t tile = tile_at(e);
+    if (tile != kInvalidKey)
+      tile_walk<MODE, 64>(I, par, flags, tile, e, wgs * kW, qx, per_xcd, queue, &s_pop, stepno,
+                          lds_of(kNarrowCells, kNarrowCap, wave), cacc, s_over);
+    __syncthreads();
+    for (uint32_t k = 0; k < s_over[0]; ++k) {
+      tile_walk<MODE, kTileThreads>(I, par, flags, s_over[k + 1u], kInvalidKey / 2u, 0u, 0u, false, queue, &s_pop, stepno,
+                                    lds_of(kTileCells, kLdsCap, 0u), cacc, nullptr);
+      __syncthreads();
+    }
+  } else {
+    if (I.tile_dyn) {
+      if (tid == 0) s_pop = queue_pop(queue);
+      __syncthreads();
+      e = s_pop;
+    }
+    const uint32_t tile = tile_at(e);
+    if (tile == kInvalidKey) return;  // no tile: this workgroup's counters stay as they are
+    tile_walk<MODE, kTileThreads>(I, par, flags, tile, e, wgs, qx, per_xcd, queue, &s_pop, stepno, lds_of(kTileCells, kLdsCap, 0u), cacc,
+                                  nullptr);
   }
 
   // per-workgroup collision counters (integers: exact in any order)
   if (MODE == kModePhysics) {
+    __syncthreads();
     long long v[3] = {(long long)cacc.sel, (long long)cacc.coll, cacc.cr};
-    long long* red = reinterpret_cast<long long*>(&s_red[0][0]);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       long long x = v[k];
       for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
-      if (lane_id() == 0) red[(tid / 64) * 3 + k] = x;
+      if (lane_id() == 0) s_red[(tid / 64) * 3 + k] = x;
     }
     __syncthreads();
     if (tid < 3) {
       long long t = 0;
-      for (uint32_t w = 0; w < kTileThreads / 64; ++w) t += red[w * 3 + tid];
+      for (uint32_t w = 0; w < kTileThreads / 64; ++w) t += s_red[w * 3 + tid];
       gmem(I.wg_acc)[vw * kAccSlots + tid] += t;
     }
   }
 }
 
-template __global__ void k_tile<kModeReference>(const InstDesc*, uint32_t, uint32_t);
-template __global__ void k_tile<kModePhysics>(const InstDesc*, uint32_t, uint32_t);
 
 // =============================================================== wall pass
 // PHYSICS: the particles the tile kernel deferred (key kDeferredKey, state
@@ -1599,15 +1710,17 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_walls(const InstDesc* __res
 // The totals that the host reads: the wall sums that no step has folded yet
 // into wall_acc, and the sums over the workgroups' collision counters, as
 // 64-bit sums of their low and high halves (out[2 k], out[2 k + 1] of slot k:
-// exact, the host puts them together in 128 bits).
-__global__ void __launch_bounds__(kTileThreads) k_totals(const InstDesc* __restrict__ Ip, long long* out) {
+// exact, the host puts them together in 128 bits). n_acc: the tile kernel's
+// workgroups so far.
+__global__ void __launch_bounds__(kTileThreads) k_totals(const InstDesc* __restrict__ Ip, uint32_t n_acc, long long* out) {
   const InstDesc& I = *Ip;
   __shared__ long long s_red[kTileThreads / 64 * 4];
   __shared__ long long s_sum[kTileThreads / kAccSlots][2 * kAccSlots];
   if (I.wall_part) fold_walls<kTileThreads>(I, s_red);
   const uint32_t k = threadIdx.x % kAccSlots, r = threadIdx.x / kAccSlots;
   long long lo = 0, hi = 0;
-  for (uint32_t w = r; w < I.n_vwg; w += kTileThreads / kAccSlots) {
+#pragma unroll 8
+  for (uint32_t w = r; w < n_acc; w += kTileThreads / kAccSlots) {
     const long long v = gmem(I.wg_acc)[w * kAccSlots + k];
     lo += (long long)((unsigned long long)v & 0xFFFFFFFFull);
     hi += v >> 32;
@@ -1978,8 +2091,8 @@ void walls(const InstDesc* d, uint32_t opar, uint32_t flags, uint32_t blocks, co
   if (blocks) hipLaunchKernelGGL(k_walls, dim3(blocks), dim3(kTileThreads), 0, st, d, opar, flags, map);
 }
 
-void totals(const InstDesc* d, long long* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_totals, dim3(1), dim3(kTileThreads), 0, st, d, out);
+void totals(const InstDesc* d, uint32_t n_acc, long long* out, hipStream_t st) {
+  hipLaunchKernelGGL(k_totals, dim3(1), dim3(kTileThreads), 0, st, d, n_acc, out);
 }
 
 void fields(const InstDesc* d, uint32_t mode, uint32_t ncells, double samples, double kb, float* out, hipStream_t st) {
@@ -1989,12 +2102,12 @@ void fields(const InstDesc* d, uint32_t mode, uint32_t ncells, double samples, d
     hipLaunchKernelGGL(k_fields<float>, dim3(blocks_for(ncells, 256)), dim3(256), 0, st, d, samples, kb, out);
 }
 
-void tile(uint32_t mode, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t n_vwg, hipStream_t st,
-          uint32_t n_inst) {
-  if (mode == kModeReference)
-    hipLaunchKernelGGL(k_tile<kModeReference>, dim3(n_vwg, n_inst), dim3(kTileThreads), 0, st, d, par, flags);
-  else
-    hipLaunchKernelGGL(k_tile<kModePhysics>, dim3(n_vwg, n_inst), dim3(kTileThreads), 0, st, d, par, flags);
+void tile(uint32_t mode, bool narrow, const InstDesc* d, uint32_t par, uint32_t flags, uint32_t blocks,
+          const uint2* map, hipStream_t st) {
+  if (!blocks) return;
+  const auto k = mode == kModeReference ? (narrow ? k_tile<kModeReference, true> : k_tile<kModeReference, false>)
+                                        : (narrow ? k_tile<kModePhysics, true> : k_tile<kModePhysics, false>);
+  hipLaunchKernelGGL(k, dim3(blocks), dim3(kTileThreads), 0, st, d, par, flags, map);
 }
 
 void load_reference(const InstDesc* d, uint32_t par, uint32_t ppc, uint32_t n_threads, float sux, float suy,

@@ -96,14 +96,42 @@ struct dsmc_solver {
     const uint32_t wg = std::min<uint32_t>((h.cap + 255u) / 256u, 4096u);
     h.n_scatter_wg = scatter_grid ? scatter_grid : h.tile_dyn ? wg : std::min<uint32_t>((h.cap + 1023u) / 1024u, wg);
   }
-  void set_tile_schedule() { h.tile_dyn = (double)h.tile_cells * ppc_exp >= 512.0 ? 1u : 0u; }
+  // Tiles of at most kNarrowCells cells that expect few particles are taken
+  // by single waves: the more tiles there are (also over the members of a
+  // batch) for the 1024 workgroups that the GPU holds, the fuller they may be
+  // before four waves on one tile finish sooner. Measured, us per step with
+  // waves / workgroups on 64-cell tiles: 1024 tiles of 10 particles 40.2 /
+  // 40.8, of 98 45.0 / 44.4, of 195 51 / 49, of 293 58 / 53; 8192 of 128 92 /
+  // 130, of 256 108 / 148; 65536 of mixed members (the 64-instance ensemble,
+  // tile kernel alone) 407 / 366 / 347 / 328 with limits of 200 / 300 / 400 /
+  // 480, 733 with workgroups only. Never with the tile queues, which serve
+  // workgroups.
+  static double narrow_limit(uint64_t tiles) { return tiles < 2048u ? 64.0 : tiles < 4096u ? 200.0 : tiles < 32768u ? 300.0 : 480.0; }
+  static bool is_narrow(const InstDesc& d, double per_tile, uint64_t tiles) {
+    return !d.tile_dyn && d.tile_cells <= kNarrowCells && per_tile <= narrow_limit(tiles);
+  }
+  // From 8192 tiles a wave takes two of them (the second's data load during
+  // the first: 92 us per step, with one each 95).
+  void set_tile_schedule() {
+    h.tile_dyn = (double)h.tile_cells * ppc_exp >= 512.0 ? 1u : 0u;
+    h.tile_narrow = is_narrow(h, (double)h.tile_cells * ppc_exp, h.ntiles) ? 1u : 0u;
+    h.n_tile_wg = h.tile_narrow ? narrow_wg(h.ntiles, h.ntiles < 8192u ? 1u : 2u) : h.n_vwg;
+    n_acc_wg = std::max(n_acc_wg, h.n_tile_wg);
+  }
+  // Workgroups for narrow tiles with at most `walk` of them per wave (the
+  // XCDs' shares of the tiles are whole patches: the fullest XCD decides).
+  static uint32_t narrow_wg(uint32_t ntiles, uint32_t walk) {
+    const uint32_t share = (ntiles + 8u * kTilePatch - 1u) / (8u * kTilePatch) * kTilePatch;  // of one XCD
+    return 8u * ((share + 4u * walk - 1u) / (4u * walk));
+  }
+  uint32_t n_acc_wg = 0;  // workgroups of the tile kernel so far (slots of wg_acc in use)
   bool sampling = false;
   uint64_t sample_steps0 = 0;
   double acc_snap[kAccSlots] = {0};
   uint32_t* scan_scratch = nullptr;  // of the loading's scan
   dsmc_launch::StepScan scan;        // of the step, with its tile sums
   uint32_t* scan_ts = nullptr;
-  uint32_t n_loaded = 0;      // particles when the wall pass's grid was chosen
+  uint32_t n_loaded = 0;      // particles loaded
   uint32_t scatter_grid = 0;  // as set by the user (0: by the engine)
   uint32_t ppc = 0;
   float ntc_init = 0.0f;
@@ -226,6 +254,10 @@ namespace {
 // The wall pass reads the bitmask directly up to this capacity, with at most
 // this many workgroups (also over the members of a batch).
 constexpr uint32_t kWallDirectCap = 2u << 20, kWallDirectWg = 4096;
+
+// A batch with more tiles than this walks its narrow ones (kNarrowWalk per
+// wave).
+constexpr uint32_t kNarrowWalkTiles = 8192;
 
 const double kPi = 3.14159265358979323846;
 
@@ -384,7 +416,7 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   // four per resident workgroup (c1, 64x32x32, 100k particles: 0.123 ms per
   // step with 64-cell tiles, 0.132 with 256, 0.149 with 32; c2, 128x64x64,
   // 1M particles: 0.155 ms with 128-cell tiles, 0.171 with 256, 0.182 with
-  // 64), and to 32 cells where such a tile still expects 512 particles (the
+  // 64, all with a workgroup per tile), and to 32 cells where such a tile still expects 512 particles (the
   // reference's 32x32x32 benchmark case with 17 per cell: 0.135 ms per step
   // with 32-cell tiles, 0.143 with 64).
   {
@@ -394,11 +426,12 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
     uint32_t tc = kTileCells;
     while (tc > 32u && tc * ppc_exp > 0.5 * kLdsCap) tc >>= 1;
     while (tc > 64u && (C + tc - 1) / tc < 4096u) tc >>= 1;
+    // sparse tiles for single waves (see dsmc_solver::narrow_limit)
+    if (tc > kNarrowCells && C >= 4096u * kNarrowCells && kNarrowCells * ppc_exp <= 300.0) tc = kNarrowCells;
     if (tc == 64u && (C + tc - 1) / tc < 4096u && 32.0 * ppc_exp >= 512.0) tc = 32u;
     I.tile_cells = tc;
     I.ntiles = (C + tc - 1) / tc;
     h->ppc_exp = ppc_exp;
-    h->set_tile_schedule();
   }
   // RNG streams = 256 x the tile kernel's workgroups. By default one tile
   // per workgroup up to 1024 workgroups (small grids fill the GPU), else
@@ -428,6 +461,7 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   I.cap = cap;
   I.n_streams = ns;
   I.n_vwg = ns / kTileThreads;
+  h->set_tile_schedule();
   h->s = s;
 
   // ---- device buffers
@@ -452,7 +486,9 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   CHECK_RC(h->alloc(&I.cstat, C));
   CHECK_RC(h->alloc(&I.samp, (size_t)5 * C));
   CHECK_RC(h->alloc(&I.ctr, 16));
-  CHECK_RC(h->alloc(&I.wg_acc, (size_t)I.n_vwg * kAccSlots));
+  // room for the narrow tiles' workgroups of any tile size
+  const size_t acc = (size_t)std::max(I.n_vwg, dsmc_solver::narrow_wg((C + 31u) / 32u, 1u)) * kAccSlots;
+  CHECK_RC(h->alloc(&I.wg_acc, acc));
   CHECK_RC(h->alloc(&I.mt_state, (size_t)kMtWords * ns));
   uint32_t *ma, *mb, *mc, *seeds;
   CHECK_RC(h->alloc(&ma, ns));
@@ -470,7 +506,7 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   HIPC(hipMemsetAsync(I.cstat, 0, (size_t)C * sizeof(float4), st));
   HIPC(hipMemsetAsync(I.samp, 0, (size_t)5 * C * 8, st));
   HIPC(hipMemsetAsync(I.ctr, 0, 64, st));
-  HIPC(hipMemsetAsync(I.wg_acc, 0, (size_t)I.n_vwg * kAccSlots * 8, st));
+  HIPC(hipMemsetAsync(I.wg_acc, 0, acc * 8, st));
   HIPC(hipMemsetAsync(I.hits, 0, (size_t)cap * 4, st));
   // ---- RNG parameters and seeds
   std::vector<uint32_t> ra, rb, rc;
@@ -741,7 +777,6 @@ static int finish_loading(dsmc_solver* h, uint32_t n, uint32_t* n_out) {
     I.n_wall_part = I.n_wall_wg;
     wall_grid(I, n, true);
     I.n_wall_part = std::max(I.n_wall_part, I.n_wall_wg);
-    h->n_loaded = n;
     CHECK_RC(h->alloc(&I.wall_part, (size_t)I.n_wall_part * 4));
     HIPC(hipMemsetAsync(I.wall_part, 0, (size_t)I.n_wall_part * 4 * sizeof(long long), st));
     CHECK_RC(h->alloc(&I.wall_acc, 4));
@@ -762,6 +797,7 @@ static int finish_loading(dsmc_solver* h, uint32_t n, uint32_t* n_out) {
     h->scan = dsmc_launch::step_scan_plan(I.ncells, I.n_face_cells);
     CHECK_RC(h->alloc(&h->scan_ts, h->scan.words()));
   }
+  h->n_loaded = n;
   h->set_scatter_grid();
   CHECK_RC(h->upload_desc());
   uint32_t ctr[2] = {n, n};
@@ -994,7 +1030,7 @@ static int sum_acc(dsmc_solver* h, double out[kAccSlots]) {
   // the collision counters' sums, then the wall totals, in one small buffer
   constexpr size_t kWords = 2 * kAccSlots;
   if (!h->d_totals) CHECK_RC(h->alloc(&h->d_totals, kWords));
-  dsmc_launch::totals(h->d_desc, h->d_totals, h->stream);
+  dsmc_launch::totals(h->d_desc, h->n_acc_wg, h->d_totals, h->stream);
   HIPC(hipGetLastError());
   long long acc[kWords];
   double tacc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1629,7 +1665,7 @@ int enqueue_step(dsmc_solver* h, uint32_t par, uint32_t flags, hipEvent_t* ev) {
   if (ev) HIPC(hipEventRecord(ev[1], st));
   dsmc_launch::scatter(h->d_desc, par, dsmc_launch::scatter_blocks(I), nullptr, h->scan, h->scan_ts, st);
   if (ev) HIPC(hipEventRecord(ev[2], st));
-  dsmc_launch::tile(I.mode, h->d_desc, par, flags, I.n_vwg, st);
+  dsmc_launch::tile(I.mode, I.tile_narrow != 0u, h->d_desc, par, flags, I.n_tile_wg, nullptr, st);
   if (ev) HIPC(hipEventRecord(ev[3], st));
   // the injection runs in the wall pass's launch: with a body both count as
   // walls, without one as injection
@@ -1696,6 +1732,8 @@ int run_graph_pair(dsmc_solver* h, uint32_t f1, uint32_t f2) {
 // Several instances advanced by the same kernel launches (grid.y = instance):
 // the batched-ensemble step. Every instance keeps its own buffers, RNG
 // streams, dt and descriptor; the batch holds the descriptor array.
+enum BatchMap { kMapScatter = 0, kMapTile, kMapNarrow, kMapWalls, kMaps };
+
 struct dsmc_batch {
   std::vector<dsmc_solver*> hs;
   std::string err;
@@ -1703,12 +1741,12 @@ struct dsmc_batch {
   hipEvent_t ev = nullptr;
   InstDesc* d_descs = nullptr;
   uint32_t* scratch = nullptr;
-  uint32_t n = 0, mode = 0, max_cells = 0, max_faces = 0, max_vwg = 0, list_grid = 0;
+  uint32_t n = 0, mode = 0, max_cells = 0, max_faces = 0, list_grid = 0;
   dsmc_launch::StepScan scan;
-  // blocks of the scatter and of the wall pass, {instance, its block} each
-  // (the wall pass's follow the scatter's), and what they were made for
+  // blocks of the launches that need different numbers for each instance:
+  // {instance, its block} of each, and the grids that the maps were made for
   uint2* d_map = nullptr;
-  uint32_t scatter_blocks = 0, wall_blocks = 0;
+  uint32_t first[kMaps] = {}, blocks[kMaps] = {};
   std::vector<uint32_t> map_of;
   bool use_graphs = true;
   std::map<uint64_t, hipGraphExec_t> graphs;
@@ -1738,43 +1776,62 @@ int batch_hip(dsmc_batch* b, hipError_t e, const char* what) {
 int enqueue_batch_step(dsmc_batch* b, uint32_t par, uint32_t flags) {
   hipStream_t st = b->stream;
   dsmc_launch::step_scan(b->d_descs, b->scan, b->scratch, st, b->n);
-  dsmc_launch::scatter(b->d_descs, par, b->scatter_blocks, b->d_map, b->scan, b->scratch, st);
-  dsmc_launch::tile(b->mode, b->d_descs, par, flags, b->max_vwg, st, b->n);
+  dsmc_launch::scatter(b->d_descs, par, b->blocks[kMapScatter], b->d_map + b->first[kMapScatter], b->scan, b->scratch, st);
+  dsmc_launch::tile(b->mode, false, b->d_descs, par, flags, b->blocks[kMapTile], b->d_map + b->first[kMapTile], st);
+  dsmc_launch::tile(b->mode, true, b->d_descs, par, flags, b->blocks[kMapNarrow], b->d_map + b->first[kMapNarrow], st);
   dsmc_launch::defer_list(b->d_descs, b->list_grid, st, b->n);
-  dsmc_launch::walls(b->d_descs, par ^ 1u, flags, b->wall_blocks, b->d_map + b->scatter_blocks, st);
+  dsmc_launch::walls(b->d_descs, par ^ 1u, flags, b->blocks[kMapWalls], b->d_map + b->first[kMapWalls], st);
   return DSMC_OK;
 }
 
 // The members' descriptors as the batch runs them: the wall pass reads the
-// bitmasks directly only where all members together are small.
+// bitmasks directly only where all members together are small, and narrow
+// tiles are walked where they fill the GPU without (a walker loads the next
+// tile's data during this one's phases).
 std::vector<InstDesc> batch_descs(dsmc_batch* b) {
   std::vector<InstDesc> d;
-  uint64_t wg = 0;
+  uint64_t wall = 0, tiles = 0;
   for (auto* h : b->hs) {
     d.push_back(h->h);
-    if (h->h.defer_bits) wg += h->h.n_wall_wg;
+    if (h->h.defer_bits) wall += h->h.n_wall_wg;
+    tiles += h->h.ntiles;
   }
-  for (uint32_t i = 0; i < b->n; ++i)
-    if (d[i].defer_bits && wg > kWallDirectWg) wall_grid(d[i], b->hs[i]->n_loaded, false);
+  for (uint32_t i = 0; i < b->n; ++i) {
+    if (d[i].defer_bits && wall > kWallDirectWg) wall_grid(d[i], b->hs[i]->n_loaded, false);
+    if (!dsmc_solver::is_narrow(d[i], (double)d[i].tile_cells * b->hs[i]->ppc_exp, tiles)) continue;
+    d[i].tile_narrow = 1u;
+    d[i].n_tile_wg = dsmc_solver::narrow_wg(d[i].ntiles, tiles > kNarrowWalkTiles ? kNarrowWalk : 1u);
+    b->hs[i]->n_acc_wg = std::max(b->hs[i]->n_acc_wg, d[i].n_tile_wg);
+  }
   return d;
 }
 
-// The block maps of the descriptors' grids; captured steps hold the old ones,
-// so they are dropped with them.
+// The block maps of the descriptors' grids, fullest members first (the last
+// blocks to start are then short); captured steps hold the old ones, so they
+// are dropped with them.
 int batch_maps(dsmc_batch* b, const std::vector<InstDesc>& descs) {
-  std::vector<uint32_t> of;
+  std::vector<uint32_t> of, order;
+  uint32_t list_grid = 0;
   for (const InstDesc& d : descs) {
     of.push_back(dsmc_launch::scatter_blocks(d));
+    of.push_back(d.tile_narrow ? 0u : d.n_tile_wg);
+    of.push_back(d.tile_narrow ? d.n_tile_wg : 0u);
     of.push_back(dsmc_launch::wall_blocks(d));
-    of.push_back(d.defer_bits && !d.wall_direct ? d.n_wall_wg : 0u);
+    if (d.defer_bits && !d.wall_direct) list_grid = std::max(list_grid, d.n_wall_wg);
+    order.push_back((uint32_t)order.size());
   }
+  of.push_back(list_grid);
   if (of == b->map_of) return DSMC_OK;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](uint32_t x, uint32_t y) { return b->hs[x]->n_loaded > b->hs[y]->n_loaded; });
   std::vector<uint2> map;
-  for (int k = 0; k < 2; ++k) {
-    for (uint32_t i = 0; i < b->n; ++i)
-      for (uint32_t q = 0; q < of[3 * i + k]; ++q) map.push_back(make_uint2(i, q));
-    (k ? b->wall_blocks : b->scatter_blocks) = (uint32_t)map.size() - (k ? b->scatter_blocks : 0u);
+  for (int k = 0; k < kMaps; ++k) {
+    b->first[k] = (uint32_t)map.size();
+    for (uint32_t i : order)
+      for (uint32_t q = 0; q < of[kMaps * i + k]; ++q) map.push_back(make_uint2(i, q));
+    b->blocks[k] = (uint32_t)map.size() - b->first[k];
   }
+  b->list_grid = list_grid;
   BHIP(hipStreamSynchronize(b->stream));
   for (auto& g : b->graphs) (void)hipGraphExecDestroy(g.second);
   b->graphs.clear();
@@ -1783,8 +1840,6 @@ int batch_maps(dsmc_batch* b, const std::vector<InstDesc>& descs) {
   b->map_of.clear();
   BHIP(hipMalloc(&b->d_map, map.size() * sizeof(uint2)));
   BHIP(hipMemcpy(b->d_map, map.data(), map.size() * sizeof(uint2), hipMemcpyHostToDevice));
-  b->list_grid = 0;
-  for (uint32_t i = 0; i < b->n; ++i) b->list_grid = std::max(b->list_grid, of[3 * i + 2]);
   b->map_of = of;
   return DSMC_OK;
 }
@@ -1813,7 +1868,6 @@ int dsmc_batch_create(dsmc_solver* const* hs, uint32_t n, dsmc_batch** out) {
   for (auto* h : b->hs) {
     b->max_cells = std::max(b->max_cells, h->h.ncells);
     b->max_faces = std::max(b->max_faces, h->h.n_face_cells);
-    b->max_vwg = std::max(b->max_vwg, h->h.n_vwg);
   }
   b->scan = dsmc_launch::step_scan_plan(b->max_cells, b->max_faces);
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);

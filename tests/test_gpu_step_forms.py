@@ -102,3 +102,68 @@ def test_fields_from_the_sums(mode):
     for k, w in want.items():
         np.testing.assert_array_equal(got[k], w.astype(np.float32), err_msg=k)
     sol.close()
+
+
+def _narrow_pair(tile_cells, crowd, seed=11, dims=(64, 64, 32), n=60000):
+    """Two equal solvers, tiles of `tile_cells` (taken by single waves) and of
+    128 cells (by workgroups). `crowd` of the particles are put into the first
+    32 cells: more than a wave's share of the LDS, or than all of it."""
+    out = []
+    for tc in (tile_cells, 128):
+        s = small_physics_settings(dims=dims, n_target=n)
+        s.seed = seed
+        sol = dm.Solver()
+        sol.Init(s)
+        sol.set_tile_cells(tc)
+        sol.SetModel(dm.icosphere((0.07, 0.05, 0.05), 0.02, 2), grid=(8, 8, 8))
+        sol.InitSystemState((1500.0, 0.0, 0.0))
+        if crowd:
+            p = sol.particles()
+            pos, vel = p["pos"].copy(), p["vel"].copy()
+            k = np.random.default_rng(seed).choice(pos.shape[1], crowd, replace=False)
+            pos[:, k] *= np.array([[0.48], [0.96 / dims[1]], [0.96 / dims[2]]], np.float32)
+            vel[:, k] *= np.float32(0.02)
+            sol.set_particles(pos, vel)
+        out.append(sol)
+    return out
+
+
+def _assert_same_run(a, b):
+    p, q = a.particles(), b.particles()
+    for k in ("pos", "vel", "key"):
+        assert np.array_equal(p[k], q[k]), k
+    assert np.array_equal(a.ntc_state(), b.ntc_state())
+    assert np.array_equal(a.cell_stats(), b.cell_stats())
+    assert np.array_equal(a.collision_stats(), b.collision_stats())
+    assert np.array_equal(a.drag(), b.drag())
+
+
+@pytest.mark.parametrize("tile_cells", [32, 64])
+@pytest.mark.parametrize("crowd", [0, 497, 1500, 5000])
+def test_narrow_tiles_match_wide_tiles(tile_cells, crowd):
+    print(f"narrow tiles of {tile_cells} cells, crowd {crowd}", flush=True)
+    a, b = _narrow_pair(tile_cells, crowd)
+    for sol in (a, b):
+        sol.set_sampling(True)
+        sol.DoBenchmark(4, sol.settings.dt)
+    start = a.cell_start()
+    assert crowd == 0 or start[32] > 0.9 * crowd  # still crowded after the steps
+    _assert_same_run(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("members", [1, 3])  # 4096 tiles: one per wave; 12288: a wave walks over four
+def test_narrow_tiles_in_a_batch(members):
+    pairs = [_narrow_pair(32, 900 * i, seed=5 + i) for i in range(members)]
+    extra = _narrow_pair(256, 0, seed=3, dims=(16, 12, 11), n=40000)  # a member taken by workgroups
+    batch = dm.Batch([p[0] for p in pairs] + [extra[0]])
+    batch.set_sampling(True)
+    batch.run(4)
+    batch.synchronize()
+    for a, b in pairs + [extra]:
+        b.set_sampling(True)
+        b.DoBenchmark(4, b.settings.dt)
+        _assert_same_run(a, b)
+        b.close()
+    batch.close()
