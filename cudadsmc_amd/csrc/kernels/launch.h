@@ -16,11 +16,9 @@ void mt_generate(const uint32_t* a, const uint32_t* b, const uint32_t* c, const 
 void cell_ids(const InstDesc& I, const float* x, const float* y, const float* z, uint32_t n, uint32_t* keys,
               hipStream_t st);
 void keys_count(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st);
-// Exclusive scan of in[0..n) into out[0..n] (out[n] = total); cursor gets a
-// copy of the offsets when non-null; in is cleared when clear_in; total_out
-// (device) receives the total. scratch: kScanMaxTiles + 1 uint32.
-int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* cursor, bool clear_in, uint32_t* scratch,
-         uint32_t* total_out, hipStream_t st);
+// Exclusive scan of in[0..n) into out[0..n] (out[n] = total); in is cleared,
+// total_out (device) receives the total. scratch: kScanMaxTiles uint32.
+int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* scratch, uint32_t* total_out, hipStream_t st);
 // Step kernels take an array of n_inst descriptors (grid.y = instance).
 //
 // Scan of the step: cell offsets and the inflow numbers of the freestream

@@ -38,6 +38,13 @@ constexpr uint32_t kScanTile = kScanThreads * kScanItems;  // 4096
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
+// Between phases of one wave: its own LDS and memory operations are in order,
+// only the compiler has to keep them so.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ void mt_load(const InstDesc& I, uint32_t s, Mt& m) {
   const gptr<uint32_t> st = gmem(I.mt_state);
 #pragma unroll
@@ -155,18 +162,9 @@ __global__ void k_keys_count(const InstDesc* __restrict__ Ip, uint32_t par, uint
   count_keys(gmem(I.count), key);
 }
 
-// Plain counting of arbitrary keys (sort operator); keys >= n_cells are
-// dropped.
-__global__ void k_count_keys(const uint32_t* keys, uint32_t n, uint32_t n_cells, uint32_t* cnt) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t key = i < n ? keys[i] : kInvalidKey;
-  count_keys(gmem(cnt), key < n_cells ? key : kInvalidKey);
-}
-
 // ====================================================================== scan
 // Exclusive scan of uint32 counts in three passes (tile sums, scan of the
-// tile sums, tile scan). Optionally copies the offsets into a cursor array,
-// clears the counts and stores the total.
+// tile sums, tile scan); clears the counts and stores the total.
 __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const uint32_t* in, uint32_t n, uint32_t* tile_sums) {
   __shared__ uint32_t red[kScanThreads / 64];
   uint32_t base = blockIdx.x * kScanTile;
@@ -241,12 +239,11 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_tiles(uint32_t* tile_sums
     if (i < n_tiles) tile_sums[i] = off;
     off += v[k];
   }
-  if (threadIdx.x == 0 && total_out) *total_out = total;
+  if (threadIdx.x == 0) *total_out = total;
 }
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_apply(uint32_t* in, uint32_t n, const uint32_t* tile_sums,
-                                                            uint32_t* out, uint32_t* cursor, uint32_t clear_in,
-                                                            const uint32_t* total) {
+                                                            uint32_t* out, const uint32_t* total) {
   __shared__ uint32_t sh[kScanThreads / 64 + 1];
   uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
@@ -264,8 +261,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(uint32_t* in, uint3
     uint32_t i = base + k;
     if (i < n) {
       out[i] = off;
-      if (cursor) cursor[i] = off;
-      if (clear_in) in[i] = 0u;
+      in[i] = 0u;
     }
     off += v[k];
   }
@@ -688,91 +684,227 @@ __global__ void __launch_bounds__(256) k_scatter(const InstDesc* __restrict__ Ip
 }
 
 // ============================================================ sort operator
-// Stable LSD radix sort of (key, storage index) pairs, 8 bits per pass: the
-// permutation of SortParticlesIndices' thrust::sort_by_key
-// (dsmc_kernel.cu:2033-2051). Keys >= n_cells (dropped particles) sort as
-// n_cells, after every valid key. A pass is a per-block digit histogram
-// (hist[digit * nblocks + block]), an exclusive scan of it, and a scatter in
-// which each block ranks its 4096 keys stably: rounds of 256 positions in
-// order, waves in order within a round, lanes in order within a wave (peers
-// of equal digit found with eight ballots).
-constexpr uint32_t kRsThreads = 256;
-constexpr uint32_t kRsRounds = 16;
-constexpr uint32_t kRsTile = kRsThreads * kRsRounds;  // 4096 keys per block
+// Stable LSD radix sort of (key, storage index) pairs: the permutation of
+// SortParticlesIndices' thrust::sort_by_key (dsmc_kernel.cu:2033-2051). Keys
+// >= n_cells (dropped particles) sort as n_cells, after every valid key.
+//
+// A pass takes up to 10 bits (2^20 keys of 2^19 cells: two passes) in three
+// launches: each block counts its keys' digits (table[digit * nblocks +
+// block]), k_rs_scan turns each digit's row into offsets and leaves the row's
+// total, and k_rs_scatter ranks its keys and moves them. Latency bounds it at
+// this size, so a block has 16 waves, of which each ranks a run of consecutive
+// keys by itself (peers of equal digit found with a ballot per bit, counts of
+// the earlier rounds in LDS of its own), and the block sorts its keys in LDS
+// first, so that its stores are runs. The cell offsets come from the sorted
+// keys (k_rs_cells). 2^20 keys, 128x64x64 cells: 55 us; with 8 bits per
+// pass, four waves per block and barriers in each of 16 rounds, a scan of three
+// launches over the table, and offsets from atomic counts 128 us.
+constexpr uint32_t kRsThreads = 1024, kRsWaves = kRsThreads / 64;
+constexpr uint32_t kRsMaxBits = 10, kRsMaxDigits = 1u << kRsMaxBits;
+constexpr uint32_t kRsCells = 1024;   // cells per block of k_rs_cells
+constexpr uint32_t kRsStage = 4096;   // keys of them that it takes into LDS
+static_assert(kRsMaxDigits <= kRsThreads, "a thread per digit");
 
 __device__ __forceinline__ uint32_t rs_key(const uint32_t* keys, uint32_t i, uint32_t n_cells, bool raw) {
   const uint32_t k = keys[i];
   return raw ? (k < n_cells ? k : n_cells) : k;
 }
 
+// R: keys per thread
+template <uint32_t R>
 __global__ void __launch_bounds__(kRsThreads) k_rs_hist(const uint32_t* keys, uint32_t n, uint32_t n_cells,
-                                                        uint32_t raw, uint32_t shift, uint32_t nblocks,
-                                                        uint32_t* hist) {
-  __shared__ uint32_t s_h[256];
-  const uint32_t tid = threadIdx.x, b = blockIdx.x;
+                                                        uint32_t raw, uint32_t shift, uint32_t digits,
+                                                        uint32_t nblocks, uint32_t* table) {
+  __shared__ uint32_t s_h[kRsMaxDigits];
+  const uint32_t tid = threadIdx.x, base = blockIdx.x * (kRsThreads * R);
+  uint32_t k[R];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = base + r * kRsThreads + tid;
+    k[r] = i < n ? rs_key(keys, i, n_cells, raw != 0u) : 0u;
+  }
   s_h[tid] = 0u;
   __syncthreads();
-  const uint32_t base = b * kRsTile;
-  for (uint32_t r = 0; r < kRsRounds; ++r) {
-    const uint32_t i = base + r * kRsThreads + tid;
-    if (i < n) atomicAdd(&s_h[(rs_key(keys, i, n_cells, raw != 0u) >> shift) & 255u], 1u);
-  }
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r)
+    if (base + r * kRsThreads + tid < n) atomicAdd(&s_h[(k[r] >> shift) & (digits - 1u)], 1u);
   __syncthreads();
-  hist[(size_t)tid * nblocks + b] = s_h[tid];
+  if (tid < digits) table[(size_t)tid * nblocks + blockIdx.x] = s_h[tid];
 }
 
+// Block d: row d of the table to exclusive offsets, in place, its total to tot[d].
+__global__ void __launch_bounds__(kScanThreads) k_rs_scan(uint32_t* table, uint32_t nblocks, uint32_t* tot) {
+  __shared__ __align__(8) uint32_t sh[4 * 2 * kScanThreads / 64];
+  uint32_t* row = table + (size_t)blockIdx.x * nblocks;
+  uint32_t carry = 0u;
+  for (uint32_t b0 = 0; b0 < nblocks; b0 += 4u * kScanThreads) {
+    const uint32_t base = b0 + 4u * threadIdx.x;
+    uint32_t v[4], sum = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      v[k] = base + k < nblocks ? row[base + k] : 0u;
+      sum += v[k];
+    }
+    uint32_t total, none;
+    uint32_t off = carry + block_scan_sum<kScanThreads / 64>(sum, 0u, total, none, sh);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (base + k < nblocks) row[base + k] = off;
+      off += v[k];
+    }
+    carry += total;
+    __syncthreads();  // sh is used again
+  }
+  if (threadIdx.x == 0) tot[blockIdx.x] = carry;
+}
+
+template <uint32_t R>
 __global__ void __launch_bounds__(kRsThreads) k_rs_scatter(const uint32_t* keys, const uint32_t* vals, uint32_t n,
                                                            uint32_t n_cells, uint32_t raw, uint32_t shift,
-                                                           uint32_t nblocks, const uint32_t* offs,
-                                                           uint32_t* keys_out, uint32_t* vals_out) {
-  __shared__ uint32_t s_run[256];              // this block's keys of each digit in earlier rounds
-  __shared__ uint32_t s_wc[kRsThreads / 64][256];  // keys of each digit per wave in this round
-  const uint32_t tid = threadIdx.x, b = blockIdx.x, lane = lane_id(), w = tid / 64u;
-  s_run[tid] = 0u;
+                                                           uint32_t bits, uint32_t nblocks, const uint32_t* table,
+                                                           const uint32_t* tot, uint32_t* keys_out,
+                                                           uint32_t* vals_out) {
+  __shared__ uint16_t s_wc[kRsWaves][kRsMaxDigits];  // a wave's keys of each digit, then the earlier waves'
+  __shared__ uint32_t s_k[kRsThreads * R], s_v[kRsThreads * R];
+  __shared__ uint32_t s_first[kRsMaxDigits];  // first place of the digit in the block
+  __shared__ uint32_t s_dst[kRsMaxDigits];    // its first place in the result, less s_first
+  __shared__ uint32_t s_part[2][kRsWaves];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid / 64u;
+  const uint32_t base = blockIdx.x * (kRsThreads * R), digits = 1u << bits, mask = digits - 1u;
+  uint32_t k[R], v[R];
 #pragma unroll
-  for (uint32_t k = 0; k < kRsThreads / 64; ++k) s_wc[k][tid] = 0u;
-  const uint32_t dbase = offs[(size_t)tid * nblocks + b];  // block's first slot of digit tid
-  __shared__ uint32_t s_base[256];
-  s_base[tid] = dbase;
-  __syncthreads();
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = base + w * (64u * R) + r * 64u + lane;
+    k[r] = i < n ? rs_key(keys, i, n_cells, raw != 0u) : 0u;
+    v[r] = i < n ? (vals ? vals[i] : i) : 0u;
+  }
+  const uint32_t g_tot = tid < digits ? tot[tid] : 0u;
+  const uint32_t g_row = tid < digits ? table[(size_t)tid * nblocks + blockIdx.x] : 0u;
+  for (uint32_t d = lane; d < digits; d += 64u) s_wc[w][d] = 0u;
   const uint64_t below = (1ull << lane) - 1ull;
-  const uint32_t base = b * kRsTile;
-  for (uint32_t r = 0; r < kRsRounds; ++r) {
-    const uint32_t i = base + r * kRsThreads + tid;
-    const bool valid = i < n;
-    const uint32_t k = valid ? rs_key(keys, i, n_cells, raw != 0u) : 0u;
-    const uint32_t v = valid ? (vals ? vals[i] : i) : 0u;
-    const uint32_t d = (k >> shift) & 255u;
+  uint32_t rank[R];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const bool valid = base + w * (64u * R) + r * 64u + lane < n;
+    const uint32_t d = (k[r] >> shift) & mask;
     uint64_t peers = __ballot(valid);
+    for (uint32_t bit = 0; bit < bits; ++bit) {
+      const bool one = (d >> bit) & 1u;
+      const uint64_t m = __ballot(one);
+      peers &= one ? m : ~m;
+    }
+    wave_sync();  // the round before has stored its counts
+    const uint32_t at = (uint32_t)__popcll(peers & below), had = s_wc[w][d];
+    wave_sync();
+    if (valid && at == 0u) s_wc[w][d] = (uint16_t)(had + (uint32_t)__popcll(peers));
+    rank[r] = had + at;
+  }
+  __syncthreads();
+  uint32_t cnt = 0u;
+  if (tid < digits) {
 #pragma unroll
-    for (uint32_t bit = 0; bit < 8; ++bit) {
-      const uint64_t m = __ballot((d >> bit) & 1u);
-      peers &= ((d >> bit) & 1u) ? m : ~m;
+    for (uint32_t q = 0; q < kRsWaves; ++q) {
+      const uint32_t c = s_wc[q][tid];
+      s_wc[q][tid] = (uint16_t)cnt;
+      cnt += c;
     }
-    const uint32_t rank = (uint32_t)__popcll(peers & below);
-    if (valid && rank == 0u) s_wc[w][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t off = s_run[d] + rank;
-      for (uint32_t k2 = 0; k2 < w; ++k2) off += s_wc[k2][d];
-      const uint32_t dst = s_base[d] + off;
-      keys_out[dst] = k;
-      vals_out[dst] = v;
-    }
-    __syncthreads();
-    uint32_t t = 0u;
+  }
+  // exclusive scans over the digits, of the block's counts and of all keys'
+  uint32_t x = cnt, y = g_tot;
 #pragma unroll
-    for (uint32_t k2 = 0; k2 < kRsThreads / 64; ++k2) {
-      t += s_wc[k2][tid];
-      s_wc[k2][tid] = 0u;
-    }
-    s_run[tid] += t;
-    __syncthreads();
+  for (uint32_t o = 1; o < 64u; o <<= 1) {
+    const uint32_t xo = __shfl_up(x, o), yo = __shfl_up(y, o);
+    if (lane >= o) x += xo, y += yo;
+  }
+  if (lane == 63u) s_part[0][w] = x, s_part[1][w] = y;
+  __syncthreads();
+  uint32_t px = 0u, py = 0u;
+#pragma unroll
+  for (uint32_t q = 0; q < kRsWaves; ++q) {
+    px += q < w ? s_part[0][q] : 0u;
+    py += q < w ? s_part[1][q] : 0u;
+  }
+  if (tid < digits) {
+    const uint32_t first = px + x - cnt;
+    s_first[tid] = first;
+    s_dst[tid] = py + y - g_tot + g_row - first;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    if (base + w * (64u * R) + r * 64u + lane >= n) continue;
+    const uint32_t d = (k[r] >> shift) & mask;
+    const uint32_t at = s_first[d] + s_wc[w][d] + rank[r];
+    s_k[at] = k[r];
+    s_v[at] = v[r];
+  }
+  __syncthreads();
+  const uint32_t m = min(n - base, kRsThreads * R);
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = r * kRsThreads + tid;
+    if (i >= m) continue;
+    const uint32_t kk = s_k[i], dst = s_dst[(kk >> shift) & mask] + i;
+    keys_out[dst] = kk;
+    vals_out[dst] = s_v[i];
   }
 }
 
-__global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
+// First place in the sorted keys whose key is not below v, found by a wave in
+// steps of 64 places (2^20 keys: four rounds of loads).
+__device__ __forceinline__ uint32_t rs_lower_bound(const uint32_t* keys, uint32_t n, uint32_t v) {
+  uint32_t lo = 0u, len = n;  // the place is in [lo, lo + len]
+  while (len) {
+    const uint32_t step = (len + 63u) / 64u;
+    const uint32_t at = (lane_id() + 1u) * step;
+    const uint32_t hit = (uint32_t)__popcll(__ballot(at <= len && keys[lo + at - 1u] < v)) * step;
+    lo += hit;
+    len = min(step - 1u, len - hit);
+  }
+  return lo;
+}
+
+// cell_start[c] = keys below c, for c in [0, n_cells], kRsCells cells per
+// block: their stretch of the keys, then a search in it per cell, in LDS where
+// the stretch is short.
+__global__ void __launch_bounds__(256) k_rs_cells(const uint32_t* keys, uint32_t n, uint32_t n_cells,
+                                                  uint32_t* cell_start) {
+  __shared__ uint32_t s_k[kRsStage];
+  __shared__ uint32_t s_end[2];
+  constexpr uint32_t kPer = kRsCells / 256u;
+  const uint32_t tid = threadIdx.x, c0 = blockIdx.x * kRsCells, w = tid / 64u;
+  if (w < 2u) {
+    const uint32_t at = rs_lower_bound(keys, n, c0 + w * kRsCells);
+    if (lane_id() == 0u) s_end[w] = at;
+  }
+  __syncthreads();
+  const uint32_t lo = s_end[0], len = s_end[1] - lo;
+  uint32_t at[kPer];
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) at[k] = 0u;
+  // at[k]: keys of the stretch below the cell, the largest power of two first
+  const uint32_t top = len ? 1u << (31u - (uint32_t)__clz((int)len)) : 0u;
+  auto search = [&](auto key) {
+    for (uint32_t step = top; step; step >>= 1) {
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t q = at[k] + step;
+        if (q <= len && key(q - 1u) < c0 + k * 256u + tid) at[k] = q;
+      }
+    }
+  };
+  if (len <= kRsStage) {
+    for (uint32_t q = tid; q < len; q += 256u) s_k[q] = keys[lo + q];
+    __syncthreads();
+    search([&](uint32_t q) { return s_k[q]; });
+  } else {
+    search([&](uint32_t q) { return keys[lo + q]; });
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t c = c0 + k * 256u + tid;
+    if (c <= n_cells) cell_start[c] = lo + at[k];
+  }
 }
 
 // ====================================================================== tile
@@ -810,15 +942,13 @@ __device__ __forceinline__ uint32_t tile_tid() {
   return TileShape<NT>::kWide ? threadIdx.x : lane_id();
 }
 
-// Between the phases of a tile: a wave's own LDS and memory operations are in
-// order, only the compiler has to keep them so.
+// Between the phases of a tile.
 template <uint32_t NT>
 __device__ __forceinline__ void tile_sync() {
   if (TileShape<NT>::kWide) {
     __syncthreads();
   } else {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
   }
 }
 
@@ -1997,15 +2127,12 @@ void keys_count(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st) {
   hipLaunchKernelGGL(k_keys_count, dim3(blocks_for(n, 256)), dim3(256), 0, st, d, par, n);
 }
 
-int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* cursor, bool clear_in, uint32_t* scratch,
-         uint32_t* total_out, hipStream_t st) {
+int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* scratch, uint32_t* total_out, hipStream_t st) {
   uint32_t tiles = blocks_for(n > 0 ? n : 1u, kScanTile);
   if (tiles > kScanMaxTiles) return -1;
-  uint32_t* total = total_out ? total_out : scratch + kScanMaxTiles;
   hipLaunchKernelGGL(k_scan_reduce, dim3(tiles), dim3(kScanThreads), 0, st, in, n, scratch);
-  hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, st, scratch, tiles, total);
-  hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(kScanThreads), 0, st, in, n, scratch, out, cursor,
-                     clear_in ? 1u : 0u, total);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, st, scratch, tiles, total_out);
+  hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(kScanThreads), 0, st, in, n, scratch, out, total_out);
   return 0;
 }
 
@@ -2037,45 +2164,45 @@ void scatter(const InstDesc* d, uint32_t par, uint32_t blocks, const uint2* map,
 }
 
 uint64_t op_sort_work_words(uint32_t n, uint32_t n_cells) {
-  const uint64_t nb = blocks_for(n > 0 ? n : 1u, kRsTile);
+  const uint64_t nb = blocks_for(n > 0 ? n : 1u, 4096u);
   return (uint64_t)n_cells + 2ull * (256ull * nb + 1ull) + (kScanMaxTiles + 1ull) + 3ull * n;
 }
 
 int op_sort(const uint32_t* keys, uint32_t n, uint32_t n_cells, uint32_t* perm, uint32_t* cell_start,
             uint32_t* work, hipStream_t st) {
-  const uint32_t nb = blocks_for(n > 0 ? n : 1u, kRsTile);
-  if ((uint64_t)n_cells > (uint64_t)kScanMaxTiles * kScanTile || 256ull * nb > (uint64_t)kScanMaxTiles * kScanTile)
-    return -1;
-  uint32_t* cnt = work;
-  uint32_t* hist = cnt + n_cells;
-  uint32_t* offs = hist + (256u * nb + 1u);
-  uint32_t* scr = offs + (256u * nb + 1u);
-  uint32_t* ka = scr + (kScanMaxTiles + 1u);
-  uint32_t* kb = ka + n;
-  uint32_t* vt = kb + n;
-  // cell offsets: counts of the valid keys and their exclusive scan
-  if (n_cells) hipLaunchKernelGGL(k_fill_u32, dim3(std::min<uint32_t>(blocks_for(n_cells, 256), 4096u)), dim3(256),
-                                  0, st, cnt, n_cells, 0u);
-  if (n) hipLaunchKernelGGL(k_count_keys, dim3(blocks_for(n, 256)), dim3(256), 0, st, keys, n, n_cells, cnt);
-  if (scan(cnt, n_cells, cell_start, nullptr, true, scr, nullptr, st)) return -1;
-  if (!n) return 0;
+  constexpr uint64_t kMost = (uint64_t)kScanMaxTiles * kScanTile;
+  if ((uint64_t)n_cells > kMost || (n + 4095ull) / 4096ull * 256ull > kMost) return -1;
   // radix passes over the bits of n_cells (the largest mapped key)
   uint32_t bits = 1;
   while (bits < 32 && (n_cells >> bits) != 0u) ++bits;
-  const uint32_t passes = (bits + 7u) / 8u;
+  const uint32_t passes = blocks_for(bits, kRsMaxBits), per = blocks_for(bits, passes), digits = 1u << per;
+  // 4096 keys per block (2^18, 2^20 and 2^25 keys of 65536 cells: 43, 56 and
+  // 626 us, with 8192 54, 71 and 750), 8192 where the table does not fit the
+  // workspace (at most 2^10 digits, so that of 8192 always does).
+  const uint64_t words = op_sort_work_words(n, n_cells) - 3ull * n;
+  const auto table_words = [&](uint32_t r) { return (uint64_t)digits * (blocks_for(n, kRsThreads * r) + 1u); };
+  const bool small = table_words(4u) <= words;
+  const uint32_t nb = blocks_for(n, kRsThreads * (small ? 4u : 8u));
+  uint32_t* ka = work;
+  uint32_t* kb = ka + n;
+  uint32_t* vt = kb + n;
+  uint32_t* tot = vt + n;
+  uint32_t* table = tot + digits;
   const uint32_t* kin = keys;
   const uint32_t* vin = nullptr;
-  for (uint32_t p = 0; p < passes; ++p) {
+  for (uint32_t p = 0; p < (n ? passes : 0u); ++p) {
     const uint32_t raw = p == 0 ? 1u : 0u;
     uint32_t* kout = (p & 1u) ? kb : ka;
     uint32_t* vout = ((passes - 1u - p) & 1u) ? vt : perm;  // the last pass writes perm
-    hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(kRsThreads), 0, st, kin, n, n_cells, raw, 8u * p, nb, hist);
-    if (scan(hist, 256u * nb, offs, nullptr, false, scr, nullptr, st)) return -1;
-    hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(kRsThreads), 0, st, kin, vin, n, n_cells, raw, 8u * p, nb,
-                       offs, kout, vout);
+    hipLaunchKernelGGL((small ? k_rs_hist<4> : k_rs_hist<8>), dim3(nb), dim3(kRsThreads), 0, st, kin, n, n_cells, raw,
+                       per * p, digits, nb, table);
+    hipLaunchKernelGGL(k_rs_scan, dim3(digits), dim3(kScanThreads), 0, st, table, nb, tot);
+    hipLaunchKernelGGL((small ? k_rs_scatter<4> : k_rs_scatter<8>), dim3(nb), dim3(kRsThreads), 0, st, kin, vin, n,
+                       n_cells, raw, per * p, per, nb, table, tot, kout, vout);
     kin = kout;
     vin = vout;
   }
+  hipLaunchKernelGGL(k_rs_cells, dim3(n_cells / kRsCells + 1u), dim3(256), 0, st, kin, n, n_cells, cell_start);
   return 0;
 }
 

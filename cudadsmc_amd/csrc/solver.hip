@@ -877,7 +877,7 @@ int dsmc_init_state(dsmc_solver* h, float ux, float uy, float uz, uint32_t* n_ou
   CHECK_RC(setup_injection(h));
   CHECK_RC(h->upload_desc());
   dsmc_launch::load_count(h->d_desc, I.n_streams, nullptr, st);
-  if (dsmc_launch::scan(I.count, I.ncells, I.cell_start, nullptr, true, h->scan_scratch, I.ctr + 1, st))
+  if (dsmc_launch::scan(I.count, I.ncells, I.cell_start, h->scan_scratch, I.ctr + 1, st))
     return h->fail(DSMC_ERR_CAPACITY, "too many cells to scan");
   uint32_t n = h->get_ctr(1);
   if (n > I.cap) return h->fail(DSMC_ERR_CAPACITY, "capacity %u < %u particles", I.cap, n);
@@ -908,7 +908,7 @@ int dsmc_init_state_from_fields(dsmc_solver* h, const float* fn, const float* fu
     HIPC(hipMemcpyAsync(d[k], src[k], (size_t)n_cells * 4, hipMemcpyHostToDevice, st));
   }
   dsmc_launch::load_count(h->d_desc, I.n_streams, d[0], st);
-  if (dsmc_launch::scan(I.count, I.ncells, I.cell_start, nullptr, true, h->scan_scratch, I.ctr + 1, st))
+  if (dsmc_launch::scan(I.count, I.ncells, I.cell_start, h->scan_scratch, I.ctr + 1, st))
     return h->fail(DSMC_ERR_CAPACITY, "too many cells to scan");
   uint32_t n = h->get_ctr(1);
   if (n > I.cap) return h->fail(DSMC_ERR_CAPACITY, "capacity %u < %u particles", I.cap, n);
