@@ -961,6 +961,12 @@ __device__ __forceinline__ uint32_t queue_pop(gptr<uint32_t> queue) {
   return gatomic_add(gelem(queue, at), 1u);
 }
 
+// Cells of at least this many particles are ranked in steps of 16: the launch
+// waits for such a cell's tile, whose ranks take n^2 comparisons (REFERENCE
+// benchmark case, which gathers 1100 of its 557k particles in one cell: 174 ->
+// 124 us, without such a cell 75 us as before).
+constexpr uint32_t kFullCell = 64;
+
 // Thread of the tile.
 template <uint32_t NT>
 __device__ __forceinline__ uint32_t tile_tid() {
@@ -1157,6 +1163,17 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
     // four independent reads per iteration: dense cells are long loops
     uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
     uint32_t j = a;
+    if (LDS && TileShape<NT>::kWide && __builtin_expect(b - a >= kFullCell, 0)) {  // 16 reads
+      for (; j & 3u; ++j) r0 += raw[j] < v ? 1u : 0u;
+      for (; j + 16u <= b; j += 16u) {
+        const uint4* const w = reinterpret_cast<const uint4*>(raw + j);
+        const uint4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+        r0 += (w0.x < v ? 1u : 0u) + (w1.x < v ? 1u : 0u) + (w2.x < v ? 1u : 0u) + (w3.x < v ? 1u : 0u);
+        r1 += (w0.y < v ? 1u : 0u) + (w1.y < v ? 1u : 0u) + (w2.y < v ? 1u : 0u) + (w3.y < v ? 1u : 0u);
+        r2 += (w0.z < v ? 1u : 0u) + (w1.z < v ? 1u : 0u) + (w2.z < v ? 1u : 0u) + (w3.z < v ? 1u : 0u);
+        r3 += (w0.w < v ? 1u : 0u) + (w1.w < v ? 1u : 0u) + (w2.w < v ? 1u : 0u) + (w3.w < v ? 1u : 0u);
+      }
+    }
     for (; j + 4u <= b; j += 4u) {
       r0 += raw[j] < v ? 1u : 0u;
       r1 += raw[j + 1u] < v ? 1u : 0u;
@@ -1507,7 +1524,7 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __rest
   // where tiles are narrow.
   __shared__ uint32_t s_start[2 * TileLds::kStart];
   __shared__ uint8_t s_nearc[2 * kTileCells];
-  __shared__ uint32_t s_raw[kLdsCap];
+  __shared__ __align__(16) uint32_t s_raw[kLdsCap];
   __shared__ uint32_t s_perm[kLdsCap];
   __shared__ uint8_t s_owner[kLdsCap];
   __shared__ float s_vx[kLdsCap];

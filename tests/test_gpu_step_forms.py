@@ -17,10 +17,10 @@ pytestmark = pytest.mark.gpu
 
 # cells: one block of 4096; not a multiple of four; the most of the one-launch scan (16 blocks, 10240 faces in three
 # blocks); two launches with an odd rest; a long thin box with more faces than cells; the second and the fourth with
-# tile queues, whose cells' counts come from two arrays
+# tile queues, whose cells' counts come from two arrays; one tile of 16 cells with about 94 particles each
 @pytest.mark.parametrize("dims,n", [((16, 16, 16), 20000), ((17, 13, 19), 9000), ((64, 32, 32), 40000),
                                     ((65, 33, 31), 40000), ((5000, 1, 1), 20000),
-                                    ((17, 13, 19), 60000), ((65, 33, 31), 600000)])
+                                    ((17, 13, 19), 60000), ((65, 33, 31), 600000), ((4, 2, 2), 1500)])
 def test_step_forms_match_oracle(dims, n):
     print(f"step forms dims={dims} n={n}", flush=True)
     s = small_physics_settings(dims=dims, n_target=n)
