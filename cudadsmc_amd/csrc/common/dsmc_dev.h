@@ -4,7 +4,8 @@
 //   particles  x,y,z,vx,vy,vz : float[cap], double-buffered (parity = step & 1)
 //   keys                      : uint32[cap] per buffer (cell of the particle,
 //                               0xFFFFFFFF = removed)
-//   count                     : uint32[ncells]      next-step counting
+//   count                     : uint32[ncells]      next-step counting (PHYSICS with tile queues: without
+//                                                   the particles in local_cnt)
 //   cursor                    : uint32[ncells]      scatter: next free sorted position of each cell
 //   local_cnt                 : uint32[ncells]      particles moved into the cell from its own tile
 //   tile_p0                   : uint32[ntiles + 1]  first stored slot of each tile's particles

@@ -6,21 +6,19 @@
 // SampleCellStatistics sequence (include/gpu_dsmc.inl:221-274).
 //
 //  * Keys of the next step are computed by the move itself and counted per
-//    cell with wave-aggregated atomics, so the "sort" is a counting sort:
-//    an exclusive scan of the counts gives the cell offsets
-//    (cellStartEnd of FindCellBoundariesDev, dsmc_kernel.cu:1734-1787). The
-//    counting atomics return each particle's rank in its cell, which is
-//    kept, so the scatter that builds the permutation needs no atomics.
+//    cell, so the "sort" is a counting sort: an exclusive scan of the counts
+//    gives the cell offsets (cellStartEnd of FindCellBoundariesDev,
+//    dsmc_kernel.cu:1734-1787) and the scatter places each particle in its
+//    cell's segment.
 //  * The tile kernel owns a tile of consecutive cells: it restores the stable
 //    order inside each cell segment (ascending storage index, i.e. the
 //    permutation of a stable sort_by_key, dsmc_kernel.cu:2048), gathers the
-//    particles (the REORDER gather, :1777-1786), runs the NTC loop one lane
-//    per cell out of LDS (:1002-1089), moves each particle with walls and
-//    box faces (:1596-1657), writes the next key and samples per cell
-//    (:856-890).
-//  * RNG (PHYSICS): stream s = 256 * virtual_workgroup + lane; the tile
-//    kernel runs a fixed grid of n_streams/256 workgroups, each walking a
-//    fixed sequence of tiles, so a cell always draws from the same stream.
+//    particles (the REORDER gather, :1777-1786), runs the NTC out of LDS (one
+//    lane per cell in REFERENCE mode, :1002-1089, rounds of disjoint pairs
+//    in PHYSICS mode), moves each particle with walls and box faces
+//    (:1596-1657), writes the next key and samples per cell (:856-890).
+//  * RNG: PHYSICS draws are counter-based (Philox keyed by cell, slot and
+//    step), so no result depends on which wave takes a tile.
 //    REFERENCE mode keeps the reference's layout: cell c collides with
 //    stream c and loading thread t draws from stream t.
 #include <hip/hip_runtime.h>

@@ -416,9 +416,10 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   // four per resident workgroup (c1, 64x32x32, 100k particles: 0.123 ms per
   // step with 64-cell tiles, 0.132 with 256, 0.149 with 32; c2, 128x64x64,
   // 1M particles: 0.155 ms with 128-cell tiles, 0.171 with 256, 0.182 with
-  // 64, all with a workgroup per tile), and to 32 cells where such a tile still expects 512 particles (the
-  // reference's 32x32x32 benchmark case with 17 per cell: 0.135 ms per step
-  // with 32-cell tiles, 0.143 with 64).
+  // 64, all with a workgroup per tile), and to 32 cells where such a tile
+  // still expects 512 particles (the reference's 32x32x32 benchmark case with
+  // 17 per cell: 0.135 ms per step with 32-cell tiles, 0.143 with 64).
+  uint32_t stream_tiles;
   {
     double ppc_exp = phys ? (s.target_particles ? (double)s.target_particles / C : (double)s.density *
                              I.cell_volume / (double)s.fnum)
@@ -426,14 +427,17 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
     uint32_t tc = kTileCells;
     while (tc > 32u && tc * ppc_exp > 0.5 * kLdsCap) tc >>= 1;
     while (tc > 64u && (C + tc - 1) / tc < 4096u) tc >>= 1;
-    // sparse tiles for single waves (see dsmc_solver::narrow_limit)
-    if (tc > kNarrowCells && C >= 4096u * kNarrowCells && kNarrowCells * ppc_exp <= 300.0) tc = kNarrowCells;
     if (tc == 64u && (C + tc - 1) / tc < 4096u && 32.0 * ppc_exp >= 512.0) tc = 32u;
+    // The streams go by these tiles, which a workgroup takes. Sparse tiles for
+    // single waves (see dsmc_solver::narrow_limit) leave them as they are, and
+    // with them the particles that the loading draws.
+    stream_tiles = (C + tc - 1) / tc;
+    if (tc > kNarrowCells && C >= 4096u * kNarrowCells && kNarrowCells * ppc_exp <= 300.0) tc = kNarrowCells;
     I.tile_cells = tc;
     I.ntiles = (C + tc - 1) / tc;
     h->ppc_exp = ppc_exp;
   }
-  // RNG streams = 256 x the tile kernel's workgroups. By default one tile
+  // RNG streams = 256 x the (wide) tile kernel's workgroups. By default one tile
   // per workgroup up to 1024 workgroups (small grids fill the GPU), else
   // about eight tiles per workgroup, at most 4096 workgroups: enough
   // workgroups to balance tiles of uneven cost (walls, dense cells) over the
@@ -441,7 +445,7 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   // written) stays small next to the particle traffic.
   uint32_t ns = s.n_streams;
   if (!ns) {
-    uint32_t wg = std::max(std::min(I.ntiles, 1024u), (I.ntiles + 7u) / 8u);
+    uint32_t wg = std::max(std::min(stream_tiles, 1024u), (stream_tiles + 7u) / 8u);
     ns = std::min(wg, 4096u) * kTileThreads;
   }
   ns = round_up(ns, kTileThreads);

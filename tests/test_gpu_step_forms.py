@@ -169,3 +169,17 @@ def test_narrow_tiles_in_a_batch(members):
         _assert_same_run(a, b)
         b.close()
     batch.close()
+
+
+# 128-cell tiles would be 8000: 1024 workgroups; 256-cell tiles 32768: 4096
+@pytest.mark.parametrize("dims,n,streams", [((160, 80, 80), 4000000, 1024 * 256), ((512, 128, 128), 8000000, 4096 * 256)])
+def test_narrow_tiles_keep_the_streams(dims, n, streams):
+    """The random-number streams, and so the particles that a case loads, do
+    not go by the size of tiles that single waves take."""
+    s = small_physics_settings(dims=dims, n_target=n)
+    s.n_streams = 0
+    sol = dm.Solver()
+    sol.Init(s)
+    layout = sol.layout()
+    assert layout["tile_cells"] == 64 and layout["n_streams"] == streams
+    sol.close()
