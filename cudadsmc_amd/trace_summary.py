@@ -6,15 +6,19 @@ over a range of steps of the main workload.
 The bench runs the main workload first (loading, warm-up, timed steps, then
 the developed-flow and sampling blocks), then the ensemble and the c1/c2
 lines. Step kernels of the main workload are picked by the tile kernel's
-grid (Grid_Size_X = G threads, Grid_Size_Y = Y: 1 for one solver, the
-member count for a batch); --skip drops the first N such steps and --take
-keeps the next K.
+grid (Grid_Size_X = G threads, for a batch those of all its members;
+Grid_Size_Y = Y: the member count in traces of builds before the batch's block
+maps); --skip drops the first N such steps and --take keeps the next K.
 """
 from __future__ import annotations
 
 import argparse
 import csv
 from collections import defaultdict
+
+
+# the launch that starts a step: the scan of the cell counts
+FIRST = ("k_scan_small", "k_scan_reduce_step", "k_bscan_reduce")
 
 
 def main() -> None:
@@ -30,12 +34,11 @@ def main() -> None:
         if r["Kernel_Name"].startswith("void "):
             r["Kernel_Name"] = r["Kernel_Name"][5:]
     rows.sort(key=lambda r: int(r["Start_Timestamp"]))
-    # step boundaries: each k_bscan_reduce launch with which=0 starts a step;
-    # a step of the main workload is the run of kernels up to the next one,
-    # identified by its tile kernel's grid
+    # a step is the run of kernels from one scan to the next, and one of the
+    # main workload is identified by its tile kernel's grid
     steps, cur = [], []
     for r in rows:
-        if r["Kernel_Name"].startswith("k_bscan_reduce") and cur and any(x["Kernel_Name"].startswith("k_tile") for x in cur):
+        if r["Kernel_Name"].startswith(FIRST) and cur and any(x["Kernel_Name"].startswith("k_tile") for x in cur):
             steps.append(cur)
             cur = []
         cur.append(r)
