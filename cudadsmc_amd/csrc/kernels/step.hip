@@ -1103,7 +1103,8 @@ __device__ __forceinline__ void tile_body(const InstDesc& I, uint32_t par, uint3
                                           const uint32_t* s_start, const uint8_t* s_nearc, uint32_t& tile_n,
                                           gptr<uint32_t> queue, uint32_t qx, bool per_xcd, uint32_t e_static,
                                           uint32_t* s_pop,
-                                          uint32_t* sn_start, uint8_t* sn_nearc, uint32_t (&pf)[TileShape<NT>::kPermPrefetch],
+                                          uint32_t* sn_start, uint8_t* sn_nearc,
+                                          uint32_t (&pf)[TileShape<NT>::kPermPrefetch],
                                           uint32_t* s_raw,
                                           uint32_t* s_perm, uint8_t* s_owner, float* s_vx, float* s_vy,
                                           float* s_vz, uint32_t stepno, const NtcLds& ntl, CollAcc& cacc) {
@@ -1495,7 +1496,8 @@ __device__ __forceinline__ void tile_walk(const InstDesc& I, uint32_t par, uint3
     if (!S::kWide && !fits && tid == 0) over[atomicAdd(over, 1u) + 1u] = tile;
     if (fits || !S::kWide)
       tile_body<MODE, true, NT>(I, par, flags, tile, c0, fits ? nc : 0u, p0, fits ? np : 0u, start, near, tile_n,
-                                queue, qx, per_xcd, e, s_pop, start_n, near_n, pf, L.raw, L.perm, L.owner, L.vx, L.vy, vz, stepno, L.ntc, cacc);
+                                queue, qx, per_xcd, e, s_pop, start_n, near_n, pf, L.raw, L.perm, L.owner, L.vx, L.vy, vz,
+                                stepno, L.ntc, cacc);
     else
       tile_body<MODE, false, NT>(I, par, flags, tile, c0, nc, p0, np, start, near, tile_n, queue, qx,
                                  per_xcd, e, s_pop, start_n, near_n, pf, L.raw, L.perm, L.owner, L.vx,
@@ -1598,8 +1600,8 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_tile(const InstDesc* __rest
     }
     const uint32_t tile = tile_at(e);
     if (tile == kInvalidKey) return;  // no tile: this workgroup's counters stay as they are
-    tile_walk<MODE, kTileThreads>(I, par, flags, tile, e, wgs, qx, per_xcd, queue, &s_pop, stepno, lds_of(kTileCells, kLdsCap, 0u), cacc,
-                                  nullptr);
+    tile_walk<MODE, kTileThreads>(I, par, flags, tile, e, wgs, qx, per_xcd, queue, &s_pop, stepno,
+                                  lds_of(kTileCells, kLdsCap, 0u), cacc, nullptr);
   }
 
   // per-workgroup collision counters (integers: exact in any order)

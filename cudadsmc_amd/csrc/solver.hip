@@ -106,7 +106,9 @@ struct dsmc_solver {
   // tile kernel alone) 407 / 366 / 347 / 328 with limits of 200 / 300 / 400 /
   // 480, 733 with workgroups only. Never with the tile queues, which serve
   // workgroups.
-  static double narrow_limit(uint64_t tiles) { return tiles < 2048u ? 64.0 : tiles < 4096u ? 200.0 : tiles < 32768u ? 300.0 : 480.0; }
+  static double narrow_limit(uint64_t tiles) {
+    return tiles < 2048u ? 64.0 : tiles < 4096u ? 200.0 : tiles < 32768u ? 300.0 : 480.0;
+  }
   static bool is_narrow(const InstDesc& d, double per_tile, uint64_t tiles) {
     return !d.tile_dyn && d.tile_cells <= kNarrowCells && per_tile <= narrow_limit(tiles);
   }
@@ -1733,7 +1735,8 @@ int run_graph_pair(dsmc_solver* h, uint32_t f1, uint32_t f2) {
 }  // namespace
 
 // ------------------------------------------------------------------ batches
-// Several instances advanced by the same kernel launches (grid.y = instance):
+// Several instances advanced by the same kernel launches (block maps, in the
+// scan grid.y = instance):
 // the batched-ensemble step. Every instance keeps its own buffers, RNG
 // streams, dt and descriptor; the batch holds the descriptor array.
 enum BatchMap { kMapScatter = 0, kMapTile, kMapNarrow, kMapWalls, kMaps };
