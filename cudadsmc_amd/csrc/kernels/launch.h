@@ -19,7 +19,8 @@ void keys_count(const InstDesc* d, uint32_t par, uint32_t n, hipStream_t st);
 // Exclusive scan of in[0..n) into out[0..n] (out[n] = total); in is cleared,
 // total_out (device) receives the total. scratch: kScanMaxTiles uint32.
 int scan(uint32_t* in, uint32_t n, uint32_t* out, uint32_t* scratch, uint32_t* total_out, hipStream_t st);
-// Step kernels take an array of n_inst descriptors (grid.y = instance).
+// Step kernels take an array of descriptors (scan and list: n_inst of them,
+// grid.y = instance; the others by a map of blocks).
 //
 // Scan of the step: cell offsets and the inflow numbers of the freestream
 // faces. One launch for instances of up to kScanSmall cells, else two. With
