@@ -527,7 +527,7 @@ struct NoBwdWArgs {
 
 __global__ void __launch_bounds__(256) k_no_conv_bwd_w(NoBwdWArgs a) {
   // dy and the shifted x of kChunk voxels, transposed: [Cout][kLdk] then
-  // [Cin][kLdk] (dynamic LDS sized by the call's channel counts)
+  // [cin][kLdk] (dynamic LDS sized by the call's channel counts)
   extern __shared__ __align__(16) bf16 sbw[];
   bf16* const sdy = sbw;
   bf16* const sx = sbw + (long)a.Cout * kLdk;
@@ -540,14 +540,15 @@ __global__ void __launch_bounds__(256) k_no_conv_bwd_w(NoBwdWArgs a) {
   const long m0 = (long)blockIdx.x * a.chunk;
   int dz, dyo, dx;
   tap_offset(t, a.taps, a.dil, dz, dyo, dx);
-  const int tm = a.Cout >> 5, tn = a.Cin >> 5;
+  const int cin = a.Cin / gridDim.z, c0 = blockIdx.z * cin;  // this workgroup's input channels
+  const int tm = a.Cout >> 5, tn = cin >> 5;
   const int ntile = tm * tn;
   f32x16 acc[kMaxNTiles];
 #pragma unroll
   for (int j = 0; j < kMaxNTiles; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[j][i] = 0.0f;
-  const int cgy = a.Cout / 8, cgx = a.Cin / 8;
+  const int cgy = a.Cout / 8, cgx = cin / 8;
   const long m_end = m0 + a.chunk < M ? m0 + a.chunk : M;  // this workgroup's voxels: [m0, m_end)
   for (long k0 = m0; k0 < m_end; k0 += kChunk) {
     __syncthreads();
@@ -584,7 +585,7 @@ __global__ void __launch_bounds__(256) k_no_conv_bwd_w(NoBwdWArgs a) {
           if (g < cgy) {
             if (mm[h] < m_end) v[h] = *reinterpret_cast<const bf16x8*>(a.dy + mm[h] * a.Cout + g * 8);
           } else if (src[h] >= 0) {
-            v[h] = *reinterpret_cast<const bf16x8*>(a.x + src[h] * a.Cin + (g - cgy) * 8);
+            v[h] = *reinterpret_cast<const bf16x8*>(a.x + src[h] * a.Cin + c0 + (g - cgy) * 8);
           }
         }
         bf16* row = g < cgy ? sdy + (long)(g * 8) * kLdk : sx + (long)((g - cgy) * 8) * kLdk;
@@ -618,7 +619,7 @@ __global__ void __launch_bounds__(256) k_no_conv_bwd_w(NoBwdWArgs a) {
   for (int j = 0; j < kMaxNTiles; ++j) {
     const int tile = wave + j * kWaves;
     if (tile >= ntile) continue;
-    const int ci = (tile % tn) * 32 + (lane & 31);
+    const int ci = c0 + (tile % tn) * 32 + (lane & 31);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int co = (tile / tn) * 32 + 8 * (i / 4) + 4 * kg + (i % 4);
@@ -1243,8 +1244,12 @@ int dsmc_no_conv_bwd_w(const void* x, const void* dy, float* dw, float* part, lo
   if ((long)chunks * n > part_floats) return -5;
   NoBwdWArgs a{(const bf16*)x, (const bf16*)dy, part, B, Z, Y, X, Cin, Cout, taps, dil, chunk};
   if (!conv27_bwd_w(a, M, chunks, (hipStream_t)stream)) {
-    const size_t lds = (size_t)(Cout + Cin) * kLdk * sizeof(bf16);
-    hipLaunchKernelGGL(k_no_conv_bwd_w, dim3(chunks, taps), dim3(256), lds, (hipStream_t)stream, a);
+    // One tap is too few workgroups for the chip, each waiting for its own
+    // loads: up to 1024 of them, one per 32 input channels. The sums stay as
+    // they are (96 -> 32 channels, 524288 voxels: 140 -> 101 us).
+    const int parts = taps == 1 && chunks * (Cin / 32) <= 1024 ? Cin / 32 : 1;
+    const size_t lds = (size_t)(Cout + Cin / parts) * kLdk * sizeof(bf16);
+    hipLaunchKernelGGL(k_no_conv_bwd_w, dim3(chunks, taps, parts), dim3(256), lds, (hipStream_t)stream, a);
   }
   hipLaunchKernelGGL(k_no_reduce_partials, dim3(nb(n, 256)), dim3(256), 0, (hipStream_t)stream, part, n, chunks,
                      dw, accumulate);

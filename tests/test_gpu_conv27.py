@@ -110,3 +110,21 @@ def test_pointwise_convolution(M, cin, cout):
     # FP32 accumulation of at most 128 products
     assert float((y32[:M * cout].reshape(M, cout).double() - want).abs().max()) <= 2e-5 * float(want.abs().max())
     assert bool((y32[M * cout:] == 3.0).all())
+
+
+# workgroups per 32 input channels up to 1024 of them, then one for all channels
+@pytest.mark.parametrize("M,cin,cout,chunk", [(1, 128, 32, 64), (1000, 96, 128, 128), (64 * 256, 128, 32, 64),
+                                              (64 * 256 + 1, 128, 32, 64)])
+def test_one_tap_weight_gradient(M, cin, cout, chunk):
+    from cudadsmc_amd import neural
+
+    print(f"one-tap weight gradient M={M} cin={cin} cout={cout} chunk={chunk}", flush=True)
+    rng = np.random.default_rng(M + cin)
+    x = no_ref.bf16_round(rng.standard_normal((M, cin)).astype(np.float32))
+    dy = no_ref.bf16_round(rng.standard_normal((M, cout)).astype(np.float32))
+    part = torch.full(((M + chunk - 1) // chunk * cin * cout,), float("nan"), device="cuda")
+    dw = torch.full((1, cout, cin), 7.0, device="cuda")
+    want = dy.astype(np.float64).T @ x.astype(np.float64)
+    neural.conv_bwd_w(bf(x), bf(dy), dw, part, 1, (1, 1, M), cin, cout, 1, 1, chunk=chunk, accumulate=False)
+    # FP32 accumulation, as above
+    assert np.max(np.abs(dw.cpu().numpy()[0] - want)) <= 2e-5 * np.max(np.abs(want))
