@@ -1118,6 +1118,12 @@ bool conv1_n(const NoConvArgs& a, long M, hipStream_t st) {
   return true;
 }
 
+// The staged kernels are made for whole groups of channels and a grid; calls
+// without (no output channel, negative extents) stay with the general ones.
+bool conv_sizes(int B, int Z, int Y, int X, int Cin, int Cout) {
+  return B > 0 && Z > 0 && Y > 0 && X > 0 && Cin > 0 && Cout > 0;
+}
+
 // The staged kernels move 16 bytes at a time; arrays that start elsewhere
 // (views at odd offsets) go to the general ones.
 bool conv_aligned(const NoConvArgs& a) {
@@ -1125,7 +1131,8 @@ bool conv_aligned(const NoConvArgs& a) {
 }
 
 bool conv1(const NoConvArgs& a, long M, hipStream_t st) {
-  if (a.taps != 1 || M >= (1L << 31) - 64 || !conv_aligned(a)) return false;
+  if (a.taps != 1 || M >= (1L << 31) - 64 || !conv_sizes(a.B, a.Z, a.Y, a.X, a.Cin, a.Cout) || !conv_aligned(a))
+    return false;
   switch (a.Cin) {
     case 32: return conv1_n<2>(a, M, st);
     case 64: return conv1_n<4>(a, M, st);
@@ -1139,7 +1146,8 @@ bool conv1(const NoConvArgs& a, long M, hipStream_t st) {
 bool conv27(const NoConvArgs& a, long M, hipStream_t st) {
   // byte offsets into x, from a run's start before the first voxel to past the last workgroup's voxels, fit an int
   const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
-  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * a.Cin * 2 >= (1L << 31) || !conv_aligned(a))
+  if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * a.Cin * 2 >= (1L << 31) ||
+      !conv_sizes(a.B, a.Z, a.Y, a.X, a.Cin, a.Cout) || !conv_aligned(a))
     return false;
   switch (a.Cin) {
     case 32: return conv27_n<2>(a, M, st);
@@ -1177,7 +1185,7 @@ void conv27_bwd_w_n(const NoBwdWArgs& a, int chunks, hipStream_t st) {
 bool conv27_bwd_w(const NoBwdWArgs& a, long M, int chunks, hipStream_t st) {
   const long reach = M + 1024 + (long)kConvMaxDil * (a.Y + 2) * a.X;
   if (a.taps != 27 || a.dil < 0 || a.dil > kConvMaxDil || reach * std::max(a.Cin, a.Cout) * 2 >= (1L << 31) ||
-      !aligned16(a.x) || !aligned16(a.dy))
+      !conv_sizes(a.B, a.Z, a.Y, a.X, a.Cin, a.Cout) || !aligned16(a.x) || !aligned16(a.dy))
     return false;
   switch (a.Cout / 32) {
     case 1: conv27_bwd_w_n<1>(a, chunks, st); return true;
@@ -1191,7 +1199,7 @@ template <bool FUSE>
 int bias_grad(const void* dy, const void* h, void* dz, long M, int Cout, float* db, float* part, long part_floats,
               int accumulate, hipStream_t st) {
   NO_EMPTY(M);
-  if (Cout % 32 || Cout > kMaxC) return -1;
+  if (Cout % 32 || Cout <= 0 || Cout > kMaxC) return -1;
   const int chunks = (int)nb(M, kBiasChunk);
   if ((long)chunks * Cout > part_floats) return -5;
   const dim3 grid(nb(chunks, 256 / Cout));
@@ -1239,6 +1247,7 @@ int dsmc_no_conv_bwd_w(const void* x, const void* dy, float* dw, float* part, lo
   if ((Cout / 32) * (Cin / 32) > kWaves * kMaxNTiles) return -1;
   long M = (long)B * Z * Y * X;
   NO_EMPTY(M);
+  if (Cin <= 0 || Cout <= 0) return -1;
   int chunks = (int)nb(M, chunk);
   long n = (long)taps * Cout * Cin;
   if ((long)chunks * n > part_floats) return -5;
