@@ -39,12 +39,21 @@ const char* global_error() { return g_err.c_str(); }
 
 using namespace dsmc_host;
 
-// Pinned buffer of host reads, two halves filled in turn: one for the process
-// (reads wait for their data anyway), held while solvers exist.
+// Pinned buffers of host reads, two halves each filled in turn: two for the
+// process, held while solvers exist. A read takes the first if it is free and
+// may then keep it while the handle's queued steps run. Reads that come
+// meanwhile wait for their own handle's steps before they take the second, so
+// that it is held for copies alone and no handle waits for another's steps.
+// (To wait first in every read leaves the GPU idle between the last step and
+// the copy: 100 steps of 100k particles and their reads 4574 -> 4649 us.)
 struct Staging {
   static constexpr size_t kHalf = 2u << 20;
+  struct Buffer {
+    std::mutex mu;
+    char* p = nullptr;
+  };
+  Buffer first, second;
   std::mutex mu;
-  char* p = nullptr;
   int users = 0;
   void enter() {
     std::lock_guard<std::mutex> lock(mu);
@@ -52,9 +61,11 @@ struct Staging {
   }
   void leave() {
     std::lock_guard<std::mutex> lock(mu);
-    if (--users > 0 || !p) return;
-    (void)hipHostFree(p);
-    p = nullptr;
+    if (--users > 0) return;
+    for (Buffer* b : {&first, &second}) {
+      if (b->p) (void)hipHostFree(b->p);
+      b->p = nullptr;
+    }
   }
 };
 static Staging g_staging;
@@ -197,17 +208,25 @@ struct dsmc_solver {
   // at a third of the rate).
   template <class F>
   int read_back(const void* src, size_t bytes, F consume) {
-    std::lock_guard<std::mutex> lock(g_staging.mu);
-    if (!g_staging.p) {
+    Staging::Buffer* buf = &g_staging.first;
+    std::unique_lock<std::mutex> lock(buf->mu, std::try_to_lock);
+    if (!lock.owns_lock()) {
+      const hipError_t queued = hipStreamSynchronize(stream);
+      if (queued != hipSuccess) return hip(queued, "read back");
+      buf = &g_staging.second;
+      lock = std::unique_lock<std::mutex>(buf->mu);
+    }
+    if (!buf->p) {
       void* q = nullptr;
       const hipError_t e = hipHostMalloc(&q, 2 * Staging::kHalf, hipHostMallocPortable);
       if (e != hipSuccess) return hip(e, "hipHostMalloc");
-      g_staging.p = static_cast<char*>(q);
+      buf->p = static_cast<char*>(q);
     }
+    char* const staged = buf->p;
     auto issue = [&](size_t off) {
       const int half = (int)(off / Staging::kHalf % 2);
       const size_t n = std::min(Staging::kHalf, bytes - off);
-      hipError_t e = hipMemcpyAsync(g_staging.p + half * Staging::kHalf, static_cast<const char*>(src) + off, n,
+      hipError_t e = hipMemcpyAsync(staged + half * Staging::kHalf, static_cast<const char*>(src) + off, n,
                                     hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipEventRecord(read_ev[half], stream);
       return hip(e, "read back");
@@ -218,7 +237,7 @@ struct dsmc_solver {
       const int half = (int)(off / Staging::kHalf % 2);
       const int rc2 = hip(hipEventSynchronize(read_ev[half]), "read back");
       if (rc == DSMC_OK) rc = rc2;
-      if (rc == DSMC_OK) consume(g_staging.p + half * Staging::kHalf, off, std::min(Staging::kHalf, bytes - off));
+      if (rc == DSMC_OK) consume(staged + half * Staging::kHalf, off, std::min(Staging::kHalf, bytes - off));
     }
     if (rc != DSMC_OK) (void)hipStreamSynchronize(stream);  // no copy into the halves stays in flight
     return rc;
