@@ -152,8 +152,9 @@ struct dsmc_solver {
   double t_ms[6] = {0, 0, 0, 0, 0, 0};  // summed ms: scan, scatter, tile, inject, whole step, walls
   uint64_t timed_steps = 0;
   hipEvent_t read_ev[2] = {nullptr, nullptr};  // the halves of a host read
-  float* d_fields = nullptr;                   // fields on their way to the host
-  long long* d_totals = nullptr;               // totals, likewise
+  static constexpr size_t kTotals = 2 * kAccSlots;
+  float* d_fields = nullptr;                   // [5][ncells] fields on their way to the host
+  long long* d_totals = nullptr;               // [kTotals] totals, likewise
   std::vector<hipEvent_t> ev_pool;   // 5 events per timed step, resolved lazily
   size_t ev_used = 0;
   uint32_t debug_flags = 0;
@@ -510,6 +511,10 @@ int dsmc_init(dsmc_solver* h, const dsmc_settings* sp) {
   CHECK_RC(h->alloc(&I.ntc, C));
   CHECK_RC(h->alloc(&I.cstat, C));
   CHECK_RC(h->alloc(&I.samp, (size_t)5 * C));
+  // of the host reads, which allocate no device memory (nor look at which
+  // device is current)
+  CHECK_RC(h->alloc(&h->d_fields, (size_t)5 * C));
+  CHECK_RC(h->alloc(&h->d_totals, dsmc_solver::kTotals));
   CHECK_RC(h->alloc(&I.ctr, 16));
   // room for the narrow tiles' workgroups of any tile size
   const size_t acc = (size_t)std::max(I.n_vwg, dsmc_solver::narrow_wg((C + 31u) / 32u, 1u)) * kAccSlots;
@@ -1033,7 +1038,6 @@ int dsmc_get_fields(dsmc_solver* h, float* n, float* u, float* v, float* w, floa
   if (nc < I.ncells) return h->fail(DSMC_ERR_INVALID, "need %u cells", I.ncells);
   if (!h->inited) return h->fail(DSMC_ERR_STATE, "not initialised");
   const size_t C = I.ncells;
-  if (!h->d_fields) CHECK_RC(h->alloc(&h->d_fields, 5 * C));
   const double S = h->samples > 0 ? (double)h->samples : 1.0;
   const double kb = h->physics() ? kBoltz : (double)kBoltzRef;
   dsmc_launch::fields(h->d_desc, I.mode, I.ncells, S, kb, h->d_fields, h->stream);
@@ -1053,11 +1057,9 @@ int dsmc_get_fields(dsmc_solver* h, float* n, float* u, float* v, float* w, floa
 static int sum_acc(dsmc_solver* h, double out[kAccSlots]) {
   InstDesc& I = h->h;
   // the collision counters' sums, then the wall totals, in one small buffer
-  constexpr size_t kWords = 2 * kAccSlots;
-  if (!h->d_totals) CHECK_RC(h->alloc(&h->d_totals, kWords));
   dsmc_launch::totals(h->d_desc, h->n_acc_wg, h->d_totals, h->stream);
   HIPC(hipGetLastError());
-  long long acc[kWords];
+  long long acc[dsmc_solver::kTotals];
   double tacc[4] = {0.0, 0.0, 0.0, 0.0};
   CHECK_RC(h->read_to(acc, h->d_totals, sizeof(acc)));
   if (I.wall_acc) CHECK_RC(h->read_to(tacc, I.wall_acc, sizeof(tacc)));
