@@ -1765,6 +1765,7 @@ enum BatchMap { kMapScatter = 0, kMapTile, kMapNarrow, kMapWalls, kMaps };
 struct dsmc_batch {
   std::vector<dsmc_solver*> hs;
   std::string err;
+  int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
   InstDesc* d_descs = nullptr;
@@ -1774,6 +1775,7 @@ struct dsmc_batch {
   // blocks of the launches that need different numbers for each instance:
   // {instance, its block} of each, and the grids that the maps were made for
   uint2* d_map = nullptr;
+  size_t map_room = 0;  // blocks that d_map holds
   uint32_t first[kMaps] = {}, blocks[kMaps] = {};
   std::vector<uint32_t> map_of;
   bool use_graphs = true;
@@ -1863,11 +1865,21 @@ int batch_maps(dsmc_batch* b, const std::vector<InstDesc>& descs) {
   BHIP(hipStreamSynchronize(b->stream));
   for (auto& g : b->graphs) (void)hipGraphExecDestroy(g.second);
   b->graphs.clear();
-  if (b->d_map) (void)hipFree(b->d_map);
-  b->d_map = nullptr;
   b->map_of.clear();
-  BHIP(hipMalloc(&b->d_map, map.size() * sizeof(uint2)));
-  BHIP(hipMemcpy(b->d_map, map.data(), map.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  if (map.size() > b->map_room) {  // on the batch's device, whichever is current
+    if (b->d_map) (void)hipFree(b->d_map);
+    b->d_map = nullptr;
+    b->map_room = 0;
+    int current = 0;
+    BHIP(hipGetDevice(&current));
+    hipError_t e = current == b->device ? hipSuccess : hipSetDevice(b->device);
+    if (e == hipSuccess) e = hipMalloc(&b->d_map, map.size() * sizeof(uint2));
+    if (current != b->device) (void)hipSetDevice(current);
+    BHIP(e);
+    b->map_room = map.size();
+  }
+  BHIP(hipMemcpyAsync(b->d_map, map.data(), map.size() * sizeof(uint2), hipMemcpyHostToDevice, b->stream));
+  BHIP(hipStreamSynchronize(b->stream));  // map is this call's own
   b->map_of = of;
   return DSMC_OK;
 }
@@ -1898,13 +1910,20 @@ int dsmc_batch_create(dsmc_solver* const* hs, uint32_t n, dsmc_batch** out) {
     b->max_faces = std::max(b->max_faces, h->h.n_face_cells);
   }
   b->scan = dsmc_launch::step_scan_plan(b->max_cells, b->max_faces);
-  hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
+  hipError_t e = hipGetDevice(&b->device);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&b->d_descs, sizeof(InstDesc) * n);
   if (e == hipSuccess) e = hipMalloc(&b->scratch, sizeof(uint32_t) * n * b->scan.words());
   if (e != hipSuccess) {
     delete b;
     return set_global_error(DSMC_ERR_DEVICE, std::string("batch allocation: ") + hipGetErrorString(e));
+  }
+  // here, so that a run allocates nothing unless a member's grids have changed
+  if (const int rc = batch_maps(b, batch_descs(b))) {
+    const std::string what = b->err;
+    delete b;
+    return set_global_error(rc, what);
   }
   *out = b;
   return DSMC_OK;
