@@ -655,8 +655,24 @@ int dsmc_set_geometry_moved(dsmc_solver* h, const float* verts, uint32_t nv, con
       g.mx[k] += move[k];
     }
   }
-  h->free_geom();
   InstDesc& I = h->h;
+  if (h->have_geom) {
+    // the old body goes as a whole, on the device too: if the new one fails
+    // below, no descriptor names freed memory (the host reads' kernels look at
+    // fluid_frac without a load between)
+    h->have_geom = false;
+    I.has_geom = 0u;
+    I.cg_flag = I.cg_start = I.cg_end = I.cg_tri = nullptr;
+    I.tv0 = I.tv1 = I.tv2 = I.tn = nullptr;
+    I.cg_rec = nullptr;
+    I.cg_se = nullptr;
+    I.fluid_frac = nullptr;
+    I.near_cell = nullptr;
+    h->frac.clear();
+    h->nearc.clear();
+    CHECK_RC(h->upload_desc());
+  }
+  h->free_geom();
   uint32_t* flag;
   uint32_t *cs, *ce, *ct;
   float4 *t0, *t1, *t2, *tn;
@@ -687,8 +703,6 @@ int dsmc_set_geometry_moved(dsmc_solver* h, const float* verts, uint32_t nv, con
   HIPC(hipMemcpyAsync(t1, h1.data(), nt * sizeof(float4), hipMemcpyHostToDevice, st));
   HIPC(hipMemcpyAsync(t2, h2.data(), nt * sizeof(float4), hipMemcpyHostToDevice, st));
   HIPC(hipMemcpyAsync(tn, hn.data(), nt * sizeof(float4), hipMemcpyHostToDevice, st));
-  I.cg_rec = nullptr;
-  I.cg_se = nullptr;
   if (h->physics()) {
     const size_t ne = std::max<size_t>(g.tri.size(), 1);
     float4* rec;
