@@ -1,7 +1,8 @@
 """The staged 3x3x3 convolution against the float64 oracle where its tiling
 can go wrong: voxel counts at the edges of its tiles, dilations up to its
-limit and beyond the grid, every channel combination, several tiles per
-workgroup (GPU)."""
+limit and beyond the grid, combinations of channels, several tiles per
+workgroup (GPU). test_gpu_conv_forms.py has the forms of two weight buffers
+and of two workgroups per CU."""
 from __future__ import annotations
 
 import numpy as np
