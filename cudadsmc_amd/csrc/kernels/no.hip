@@ -902,23 +902,25 @@ __global__ void __launch_bounds__(256) k_no_bias_grad(const bf16* dy, const bf16
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const long m = m0 + i + 8 * k;
-        if (!whole() && m >= M) break;
+        const bool in = whole() || m < M;
         if (FUSE) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[k][e] = bf2f(act[k][e]) > 0.0f ? v[k][e] : (bf16)0.0f;
           bf16* const o = dz + m * Cout + pc * 8;
           if (VEC) {
-            *reinterpret_cast<bf16x8*>(o) = v[k];
-          } else {
+            if (in) *reinterpret_cast<bf16x8*>(o) = v[k];
+          } else if (in) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = v[k][e];
           }
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s[e] += bf2f(v[k][e]);
+        for (int e = 0; e < 8; ++e) s[e] += in ? bf2f(v[k][e]) : 0.0f;  // (adding zero leaves every sum as it is)
       }
     };
-    if (m0 + kBiasChunk <= M) {
+    // one form per wave: with 32 channels a wave has two chunks, and a ragged
+    // second one would have it run both (1000 voxels: 17 -> 11 us)
+    if (__all(m0 + kBiasChunk <= M)) {
       for (int i = vl; i < kBiasChunk; i += 64) batch(i, std::true_type{});
     } else {
       for (int i = vl; i < kBiasChunk && m0 + i < M; i += 64) batch(i, std::false_type{});

@@ -149,3 +149,28 @@ def test_infinities_and_nan_stay_where_they_are(bad, row):
         assert spread.tolist() == [5 if x_bad else 11]
         if x_bad:  # 27 voxels of the grid see it at most, and not all of them lie in the grid
             assert 0 < int((~torch.isfinite(h.reshape(M, cout))).any(1).sum()) <= 27
+
+
+# a wave has two chunks of 512 voxels at 32 channels, one else; ragged in the first and the second of them
+@pytest.mark.parametrize("M", [1, 511, 513, 1000, 1537, 4600])
+@pytest.mark.parametrize("cout", [32, 96])
+def test_bias_gradient_of_a_ragged_chunk(M, cout):
+    """The sums of a ragged last chunk are those of the chunk filled up with
+    zeros, bit for bit, and nothing is written past the end."""
+    from cudadsmc_amd import neural
+
+    rng = np.random.default_rng(M + cout)
+    chunks = (M + 511) // 512
+    dy, h = (bf(rng.standard_normal((chunks * 512, cout))) for _ in range(2))
+    dy[M:] = 0.0
+    dz = torch.full((chunks * 512, cout), 5.0, dtype=torch.bfloat16, device="cuda")
+    part = torch.full((chunks * cout,), float("nan"), device="cuda")
+    out = [torch.zeros(cout, device="cuda") for _ in range(4)]
+    neural.bias_grad(dy, M, cout, out[0], part)
+    neural.bias_grad(dy, chunks * 512, cout, out[1], part)
+    neural.relu_bias_bwd(dy, h, dz, M, cout, out[2], part)
+    assert bool((dz[M:] == 5.0).all())
+    assert torch.equal(dz[:M], torch.where(h[:M] > 0, dy[:M], torch.zeros_like(dy[:M])))
+    dz[M:] = 0.0
+    neural.bias_grad(dz, chunks * 512, cout, out[3], part)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[2], out[3])
