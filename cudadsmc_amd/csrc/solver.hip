@@ -110,24 +110,40 @@ struct dsmc_solver {
   // Tiles of at most kNarrowCells cells that expect few particles are taken
   // by single waves: the more tiles there are (also over the members of a
   // batch) for the 1024 workgroups that the GPU holds, the fuller they may be
-  // before four waves on one tile finish sooner. Measured, us per step with
-  // waves / workgroups on 64-cell tiles: 1024 tiles of 10 particles 40.2 /
-  // 40.8, of 98 45.0 / 44.4, of 195 51 / 49, of 293 58 / 53; 8192 of 128 92 /
-  // 130, of 256 108 / 148; 65536 of mixed members (the 64-instance ensemble,
-  // tile kernel alone) 407 / 366 / 347 / 328 with limits of 200 / 300 / 400 /
-  // 480, 733 with workgroups only. Never with the tile queues, which serve
-  // workgroups.
-  static double narrow_limit(uint64_t tiles) {
-    return tiles < 2048u ? 64.0 : tiles < 4096u ? 200.0 : tiles < 32768u ? 300.0 : 480.0;
+  // before four waves on one tile finish sooner. Never with the tile queues,
+  // which serve workgroups. Measured, us per step with waves / workgroups on
+  // 64-cell tiles by the particles that one expects:
+  //    tiles     64         200        300        400        480
+  //     1024  41.8/41.5  48.6/45.7  55.8/49.4  63.7/53.5  97.7/57.6
+  //     1536  49.4/54.9  59.6/62.5  70.0/71.3  79.6/77.6   117/84.6
+  //     2048  50.9/56.6  63.5/66.9  75.8/77.2  89.3/86.5   126/93.2
+  //     3072  53.2/65.2  73.9/83.5  90.2/99.7  99.0/106    140/117
+  //     4096  56.8/74.6  84.6/99.7  98.4/114    113/126    147/133
+  //     8192  75.4/111    104/135    120/156    143/168    206/183
+  //    32768      -          -       345/473    437/537    642/589
+  // The waves' lead ends between 300 and 400 particles up to 2048 tiles (at
+  // 1024, one per workgroup, they have none), and between 400 and 480 above,
+  // where tiles of more than kNarrowCap become common, which the workgroup
+  // takes afterwards: 32768 tiles of 440 489/559, of 460 550/574. The limits
+  // keep below that. A batch's waves walk over more tiles each, which hides
+  // more of it: 64 members of 1024 tiles with 480 each 1237/1378, mixed ones
+  // (the 64-instance ensemble, tile kernel alone) 407 / 366 / 347 / 328 with
+  // limits of 200 / 300 / 400 / 480, 733 with workgroups only. REFERENCE tiles
+  // gain as much (64x64x64 cells of two particles 43.6/53.6, 128x64x64 of four
+  // 104/123), but not with one particle in each of 64x32x32 cells (24.9/23.5),
+  // nor where the launch waits for one tile, the cell in which the loading
+  // parks the body's particles (32x32x32 of one: 105/97).
+  static double narrow_limit(uint64_t tiles, bool batch) {
+    return tiles < 2048u ? 64.0 : tiles < 4096u ? 200.0 : tiles < 32768u ? 300.0 : batch ? 480.0 : 460.0;
   }
-  static bool is_narrow(const InstDesc& d, double per_tile, uint64_t tiles) {
-    return !d.tile_dyn && d.tile_cells <= kNarrowCells && per_tile <= narrow_limit(tiles);
+  static bool is_narrow(const InstDesc& d, double per_tile, uint64_t tiles, bool batch) {
+    return !d.tile_dyn && d.tile_cells <= kNarrowCells && per_tile <= narrow_limit(tiles, batch);
   }
   // From 8192 tiles a wave takes two of them (the second's data load during
   // the first: 92 us per step, with one each 95).
   void set_tile_schedule() {
     h.tile_dyn = (double)h.tile_cells * ppc_exp >= 512.0 ? 1u : 0u;
-    h.tile_narrow = is_narrow(h, (double)h.tile_cells * ppc_exp, h.ntiles) ? 1u : 0u;
+    h.tile_narrow = is_narrow(h, (double)h.tile_cells * ppc_exp, h.ntiles, false) ? 1u : 0u;
     h.n_tile_wg = h.tile_narrow ? narrow_wg(h.ntiles, h.ntiles < 8192u ? 1u : 2u) : h.n_vwg;
     n_acc_wg = std::max(n_acc_wg, h.n_tile_wg);
   }
@@ -1842,7 +1858,7 @@ std::vector<InstDesc> batch_descs(dsmc_batch* b) {
   }
   for (uint32_t i = 0; i < b->n; ++i) {
     if (d[i].defer_bits && wall > kWallDirectWg) wall_grid(d[i], b->hs[i]->n_loaded, false);
-    if (!dsmc_solver::is_narrow(d[i], (double)d[i].tile_cells * b->hs[i]->ppc_exp, tiles)) continue;
+    if (!dsmc_solver::is_narrow(d[i], (double)d[i].tile_cells * b->hs[i]->ppc_exp, tiles, true)) continue;
     d[i].tile_narrow = 1u;
     d[i].n_tile_wg = dsmc_solver::narrow_wg(d[i].ntiles, tiles > kNarrowWalkTiles ? kNarrowWalk : 1u);
     b->hs[i]->n_acc_wg = std::max(b->hs[i]->n_acc_wg, d[i].n_tile_wg);
