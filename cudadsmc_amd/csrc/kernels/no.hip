@@ -1073,7 +1073,7 @@ static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t
 namespace {
 
 template <int KS, int NT, int R>
-bool conv27_launch(const NoConvArgs& a, long M, hipStream_t st) {
+void conv27_launch(const NoConvArgs& a, long M, hipStream_t st) {
   // persistent workgroups: one resident set
   static const int per_cu = [] {
     int n = 0;
@@ -1083,11 +1083,10 @@ bool conv27_launch(const NoConvArgs& a, long M, hipStream_t st) {
   const unsigned tiles = nb(M, 32 * R * kWaves);
   const unsigned grid = std::min(tiles, (unsigned)(kCus * per_cu));
   hipLaunchKernelGGL((k_no_conv27<KS, NT, R>), dim3(grid), dim3(256), 0, st, a, (int)tiles);
-  return true;
 }
 
 template <int KS, int NT>
-bool conv27_r(const NoConvArgs& a, long M, hipStream_t st) {
+void conv27_r(const NoConvArgs& a, long M, hipStream_t st) {
   // Two voxel tiles per wave; one where that leaves half the CUs without a
   // workgroup (M <= 32768: 1008 voxels of 128 -> 128 channels 35 us against
   // 56). Three or four per wave need fewer LDS reads per matrix instruction,
@@ -1098,7 +1097,7 @@ bool conv27_r(const NoConvArgs& a, long M, hipStream_t st) {
 }
 
 template <int KS>
-bool conv27_n(const NoConvArgs& a, long M, hipStream_t st) {
+void conv27_n(const NoConvArgs& a, long M, hipStream_t st) {
   switch (a.Cout / 32) {
     case 1: return conv27_r<KS, 1>(a, M, st);
     case 2: return conv27_r<KS, 2>(a, M, st);
@@ -1108,7 +1107,7 @@ bool conv27_n(const NoConvArgs& a, long M, hipStream_t st) {
 }
 
 template <int KS>
-bool conv1_n(const NoConvArgs& a, long M, hipStream_t st) {
+void conv1_n(const NoConvArgs& a, long M, hipStream_t st) {
   const unsigned tiles = nb(M, 32);
   const dim3 grid(std::min(nb(tiles, kWaves), 4u * kCus));  // four workgroups per CU
   switch (a.Cout / 32) {
@@ -1117,7 +1116,6 @@ bool conv1_n(const NoConvArgs& a, long M, hipStream_t st) {
     case 3: hipLaunchKernelGGL((k_no_conv1<KS, 3>), grid, dim3(256), 0, st, a, (int)tiles); break;
     default: hipLaunchKernelGGL((k_no_conv1<KS, 4>), grid, dim3(256), 0, st, a, (int)tiles); break;
   }
-  return true;
 }
 
 // The staged kernels are made for whole groups of channels and a grid; calls
@@ -1136,10 +1134,10 @@ bool conv1(const NoConvArgs& a, long M, hipStream_t st) {
   if (a.taps != 1 || M >= (1L << 31) - 64 || !conv_sizes(a.B, a.Z, a.Y, a.X, a.Cin, a.Cout) || !conv_aligned(a))
     return false;
   switch (a.Cin) {
-    case 32: return conv1_n<2>(a, M, st);
-    case 64: return conv1_n<4>(a, M, st);
-    case 96: return conv1_n<6>(a, M, st);
-    case 128: return conv1_n<8>(a, M, st);
+    case 32: conv1_n<2>(a, M, st); return true;
+    case 64: conv1_n<4>(a, M, st); return true;
+    case 96: conv1_n<6>(a, M, st); return true;
+    case 128: conv1_n<8>(a, M, st); return true;
     default: return false;
   }
 }
@@ -1152,10 +1150,10 @@ bool conv27(const NoConvArgs& a, long M, hipStream_t st) {
       !conv_sizes(a.B, a.Z, a.Y, a.X, a.Cin, a.Cout) || !conv_aligned(a))
     return false;
   switch (a.Cin) {
-    case 32: return conv27_n<2>(a, M, st);
-    case 64: return conv27_n<4>(a, M, st);
-    case 96: return conv27_n<6>(a, M, st);
-    case 128: return conv27_n<8>(a, M, st);
+    case 32: conv27_n<2>(a, M, st); return true;
+    case 64: conv27_n<4>(a, M, st); return true;
+    case 96: conv27_n<6>(a, M, st); return true;
+    case 128: conv27_n<8>(a, M, st); return true;
     default: return false;
   }
 }

@@ -273,7 +273,8 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(uint32_t* in, uint3
 //
 //  * k_scan_small (instances of at most kScanSmall cells): one launch. Each
 //    block of 4096 cells sums the counts before it by itself, so no block
-//    waits for another; the last one reads 15 blocks of 16 KB from L2.
+//    waits for another; the last one reads 15 blocks of 16 KB from L2 (of
+//    32 KB where the stayers are counted apart).
 //  * k_scan_reduce + k_scan_apply_step: block sums first, then each block adds
 //    up the sums before it (at most 4096 words).
 //
@@ -940,7 +941,6 @@ using dsmc_launch::kFlagHits;
 template <uint32_t NT>
 struct TileShape {
   static constexpr bool kWide = NT == kTileThreads;
-  static constexpr uint32_t kCells = kWide ? kTileCells : kNarrowCells;
   static constexpr uint32_t kCap = kWide ? kLdsCap : kNarrowCap;  // particles staged in LDS
   static constexpr uint32_t kMoveBatch = kWide ? 6 : 4;  // rounds of NT positions whose loads are issued together
   // PHYSICS: rounds of NT permutation entries of the next tile loaded into

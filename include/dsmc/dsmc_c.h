@@ -258,7 +258,9 @@ int dsmc_get_collision_grid(dsmc_solver* h, uint32_t* flags, uint32_t n);
 /* Average milliseconds per step of each kernel class {scan, scatter, cells,
  * inject, total} over the steps timed since dsmc_set_timing; out_ms[5]
  * (when n > 5) receives the number of timed steps and out_ms[6] (n > 6) the
- * wall pass of PHYSICS runs with a body. */
+ * wall pass of PHYSICS runs with a body. The inflow is generated in the wall
+ * pass's launch: with a body its time is part of out_ms[6], and out_ms[3]
+ * holds next to nothing; without one out_ms[3] is the inflow. */
 int dsmc_get_timings(dsmc_solver* h, float* out_ms, uint32_t n);
 /* Enable hipEvent timing of each kernel class (off by default). Events are
  * recorded on the solver's stream without host synchronisation and resolved
